@@ -764,6 +764,19 @@ __device__ __forceinline__ void mv_team_f32(const DMat& m, const int (&rows)[R],
     for (int i = 0; i < R; i++) acc[b][i] = row_out_f32<FMT>(team_sum<TL>(acc[b][i]), srow[i]);
 }
 
+// The balanced tree over `splits` (2, 4 or 8) partial roots `plane` floats apart, in order: the
+// butterfly of a team whose lanes were split over blocks. Every load is issued before any is used.
+__device__ __forceinline__ float split_tree(const float* __restrict__ p, size_t plane, int splits) {
+  float v[8];
+#pragma unroll
+  for (int i = 0; i < 8; i++) v[i] = p[(size_t)min(i, splits - 1) * plane];
+  const float a = v[0] + v[1];
+  if (splits == 2) return a;
+  const float b = a + (v[2] + v[3]);
+  if (splits == 4) return b;
+  return b + ((v[4] + v[5]) + (v[6] + v[7]));
+}
+
 // Team width of a matrix: 32 lanes when a row has at most 32 chunks, else 64.
 // It fixes which chunks a lane sums and the butterfly, so it is a function of
 // the shape alone and every path over a given matrix sums in one order.

@@ -143,6 +143,9 @@ __global__ void k_embed_rows(const uint16_t* __restrict__ embed, const int* __re
     rows[(size_t)t * hidden + i] = __builtin_bit_cast(float, (uint32_t)src[i] << 16);
 }
 
+// Positions from which the batched contractions run on the f32 matrix cores (launch_chain_f32).
+constexpr int kChainMinSeq = 12;
+
 int prefill_chunk(const ModelDev& m, const CacheDev& c) {
   int p = c.capacity < kPrefillChunk ? c.capacity : kPrefillChunk;
   if (m.numerics == QH_NUMERICS_EXACT && c.capacity > kPLds) {
@@ -183,6 +186,7 @@ PrefillBytes prefill_bytes(const ModelDev& m, const CacheDev& c, int matmul) {
     const LayerDev& l = m.layers_host[L];
     for (const DMat* w : {&l.qkv, &l.o, &l.gu, &l.down}) {
       if (m.numerics == QH_NUMERICS_EXACT) scratch = std::max(scratch, matvec_x64_bytes(*w, (int)P));
+      else scratch = std::max(scratch, chain_partials_bound(*w, (int)P));
       if (matmul == QH_MATMUL_MFMA && matmul_prefill_supported(*w))
         scratch = std::max(scratch, matmul_prefill_scratch_bytes(*w, (int)P));
     }
@@ -282,7 +286,11 @@ static hipError_t matmul(hipStream_t s, const ModelDev& m, int mode, const DMat&
                          const float* bias, float* y, int seq, const PrefillDev& p) {
   if (mode == QH_MATMUL_MFMA && matmul_prefill_supported(w))
     return launch_matmul_prefill(s, w, x, bias, y, seq, p.scratch, p.scratch_bytes);
-  if (m.numerics == QH_NUMERICS_FAST) return launch_matvec_f32(s, w, x, bias, y, seq);
+  if (m.numerics == QH_NUMERICS_FAST) {
+    if (seq >= kChainMinSeq)
+      return launch_chain_f32(s, w, x, bias, y, seq, static_cast<float*>(p.scratch), p.scratch_bytes);
+    return launch_matvec_f32(s, w, x, bias, y, seq);
+  }
   return launch_matvec(s, w, x, bias, y, seq, static_cast<double*>(p.scratch));
 }
 

@@ -92,6 +92,13 @@ size_t matvec_x64_bytes(const DMat& m, int seq);
 hipError_t launch_matvec_f32(hipStream_t s, const DMat& m, const float* x, const float* bias, float* y,
                              int seq);
 bool matvec_f32_supported(const DMat& m);
+// The same sums, bit for bit, on the f32 matrix cores (chain.hip). `part` holds the split roots:
+// chain_partials_bytes(m, seq) bytes, at most chain_partials_bound(m, P) for every seq up to P.
+hipError_t launch_chain_f32(hipStream_t s, const DMat& m, const float* x, const float* bias, float* y, int seq,
+                            float* part, size_t part_bytes);
+constexpr int kChainMaxSplits = 8;
+size_t chain_partials_bytes(const DMat& m, int seq);
+size_t chain_partials_bound(const DMat& m, int P);
 // The batched-prefill contraction on the int8 matrix cores over exact activation digits (int8 /
 // int4 weights): y [M, rows] = x [M, cols] . W^T
 // (+ bias). `scratch` holds `scratch_bytes` bytes; a launch that needs more returns

@@ -1,0 +1,49 @@
+"""The batched prefill's contractions on the f32 matrix cores (csrc/chain.hip) against the decode
+step: the same sums in the same order, so a prompt's logits and its f16 K/V rows are those of the
+same positions stepped one at a time, bit for bit -- at the edges of the 64-position and 64-row
+tiles, with one and several splits of the team's slots, ragged last chunks and every format."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("scheme", ["f16", "int8", "int4"])
+@pytest.mark.parametrize("hidden,ffn,heads,kv_heads", [
+    (128, 256, 2, 1),       # fewer chunks than lanes: empty slots in the tree
+    (896, 4864, 14, 2),     # the 0.5B layer: 64-lane teams, several chunks per lane (down)
+    (192, 1184, 3, 1),      # rows and chunks off the tiles
+])
+def test_batched_prefill_on_matrix_cores_equals_steps_bitwise(ctx, hip, scheme, hidden, ffn, heads, kv_heads):
+    group = 32 if hidden == 192 else 128
+    cfg = hip.ModelConfig(hidden=hidden, intermediate=ffn, layers=2, heads=heads, kv_heads=kv_heads, vocab=1000)
+    ckpt = hip.synthesize_checkpoint(cfg, seed=21)
+    model = hip.GpuModel.load(ctx, hip.device_tensors(ckpt, cfg, scheme, group, "int8"), cfg, maxPositions=512)
+    ids = hip.synth_tokens(21, "chain", cfg.vocab, 300)
+    steps = model.newCache(300)
+    model.set_matmul("matvec")
+    want = {}
+    for t in range(300):
+        if t + 1 in (12, 33, 64, 65, 129, 300):
+            want[t + 1] = model.forward_tokens(ids[t:t + 1], steps)["logits"]
+        else:
+            model.forward_tokens(ids[t:t + 1], steps, wantLogits=False)
+    kv = [steps.present(L) for L in range(cfg.layers)]
+    model.set_matmul("batched")
+    for n, logits in want.items():
+        cache = model.newCache(300)
+        got = model.forward_tokens(ids[:n], cache)["logits"]
+        np.testing.assert_array_equal(got.view(np.uint32), logits.view(np.uint32), err_msg=f"{n} positions")
+        for L in range(cfg.layers):
+            p = cache.present(L)
+            for name in ("key", "value"):
+                np.testing.assert_array_equal(p[name], kv[L][name][:, :n], err_msg=f"{n} positions, layer {L} {name}")
+        cache.destroy()
+    # after a past of odd length
+    cache = model.newCache(300)
+    model.forward_tokens(ids[:35], cache, wantLogits=False)
+    got = model.forward_tokens(ids[35:129], cache)["logits"]
+    np.testing.assert_array_equal(got.view(np.uint32), want[129].view(np.uint32))
+    cache.destroy()
+    steps.destroy()
+    model.destroy()
