@@ -24,18 +24,19 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 constexpr int kChainM = 64;                 // positions per block
 constexpr int kChainN = 64;                 // rows per block
-constexpr int kChainK = 64;                 // columns per slab
-constexpr int kChainXRow = kChainK + 4;     // staged floats per position: the pad spreads rows over the banks
 
 template <int FMT>
 struct ChainFmt {
   static constexpr int kW = Fmt<FMT>::kW;
-  static constexpr int kS = kChainK / kW;                  // slots (decode lanes) per slab
+  static constexpr int kS = FMT == QH_FMT_INT4 ? 2 : 4;    // slots (decode lanes) per slab
+  static constexpr int kK = kS * kW;                       // columns per slab
+  static constexpr int kXRow = kK + 4;                     // staged floats per position: the pad spreads rows over the banks
+  static constexpr int kXPer = kChainM * kK / 4 / kBlock;  // float4 loads per thread
   static constexpr int kWBytes = 16 * kS;                  // weight bytes of a row in a slab
   static constexpr int kWRow = kWBytes + 16;               // staged, padded against bank conflicts
   static constexpr int kPieces = kChainN * kS;             // 16-byte pieces of a weight slab
   static constexpr int kPer = (kPieces + kBlock - 1) / kBlock;
-  static constexpr int kLevels = FMT == QH_FMT_F16 ? 3 : FMT == QH_FMT_INT8 ? 4 : 5;  // log2(64 / kS)
+  static constexpr int kLevels = FMT == QH_FMT_INT4 ? 5 : 4;  // log2(64 / kS)
 };
 
 struct ChainArgs {
@@ -43,12 +44,12 @@ struct ChainArgs {
   const float* x;     // [seq][cols]
   const float* bias;  // [rows] or null
   float* y;           // [seq][rows]; with several splits [splits][seq][rows] roots without scale or bias
-  int seq, tl, slots; // decode team width; slots per split (blockIdx.z), a power of two
+  int seq, tl;        // positions; decode team width
 };
 
 template <int FMT>
 struct ChainLds {
-  float x[kChainM * kChainXRow];
+  float x[kChainM * ChainFmt<FMT>::kXRow];
   float sx[ChainFmt<FMT>::kS][kChainM];
   float sz[FMT == QH_FMT_INT4 ? kChainN * 2 * ChainFmt<FMT>::kS : 4];
   __attribute__((aligned(16))) uint8_t w[kChainN * ChainFmt<FMT>::kWRow];
@@ -57,7 +58,7 @@ struct ChainLds {
 // A slab's loads, in flight in registers while the previous slab is contracted.
 template <int FMT>
 struct ChainRegs {
-  v4f x[4];
+  v4f x[ChainFmt<FMT>::kXPer];
   v4u w[ChainFmt<FMT>::kPer];
   float s, z;
 };
@@ -69,9 +70,9 @@ __device__ __forceinline__ void chain_load(const ChainArgs& a, int row0, int pos
   using F = ChainFmt<FMT>;
   const int t = threadIdx.x;
 #pragma unroll
-  for (int j = 0; j < 4; j++) {
-    const int i = t + j * kBlock, p = min(pos0 + i / 16, a.seq - 1);
-    const int col = min(c0 * F::kW + 4 * (i & 15), a.m.cols - 4);
+  for (int j = 0; j < F::kXPer; j++) {
+    const int i = t + j * kBlock, p = min(pos0 + i / (F::kK / 4), a.seq - 1);
+    const int col = min(c0 * F::kW + 4 * (i % (F::kK / 4)), a.m.cols - 4);
     r.x[j] = *reinterpret_cast<const v4f*>(a.x + (size_t)p * a.m.cols + col);
   }
 #pragma unroll
@@ -97,10 +98,10 @@ __device__ __forceinline__ void chain_store(const ChainRegs<FMT>& r, ChainLds<FM
   using F = ChainFmt<FMT>;
   const int t = threadIdx.x;
 #pragma unroll
-  for (int j = 0; j < 4; j++) {
-    const int i = t + j * kBlock, p = i / 16, q = i & 15;
+  for (int j = 0; j < F::kXPer; j++) {
+    const int i = t + j * kBlock, p = i / (F::kK / 4), q = i % (F::kK / 4);
     const v4f v = r.x[j];
-    float* d = l.x + p * kChainXRow + 8 * (q >> 1) + 2 * (q & 1);
+    float* d = l.x + p * F::kXRow + 8 * (q >> 1) + 2 * (q & 1);
     if constexpr (FMT == QH_FMT_INT4) {
       *reinterpret_cast<float2*>(d) = float2{v.x, v.y};
       *reinterpret_cast<float2*>(d + 4) = float2{v.z, v.w};
@@ -111,14 +112,15 @@ __device__ __forceinline__ void chain_store(const ChainRegs<FMT>& r, ChainLds<FM
     if constexpr (FMT != QH_FMT_F16) {
       constexpr int G = F::kW / 4;  // consecutive lanes per chunk: the staging's own chunk sum
       const float s4 = chunk_group_sum<G>((v.x + v.y) + (v.z + v.w));
-      if ((q & (G - 1)) == 0) l.sx[q / G][p] = s4;
+      if ((q & (G - 1)) == 0) l.sx[q / G][p] = FMT == QH_FMT_INT8 ? -128.f * s4 : s4;  // exact
     }
   }
 #pragma unroll
   for (int j = 0; j < F::kPer; j++) {
     const int i = t + j * kBlock;
+    const uint32_t flip = FMT == QH_FMT_INT8 ? 0x80808080u : 0u;  // int8: q + 128 in every byte
     if (F::kPieces % kBlock == 0 || i < F::kPieces)
-      *reinterpret_cast<v4u*>(l.w + (i / F::kS) * F::kWRow + 16 * (i % F::kS)) = r.w[j];
+      *reinterpret_cast<v4u*>(l.w + (i / F::kS) * F::kWRow + 16 * (i % F::kS)) = r.w[j] ^ flip;
   }
   if constexpr (FMT == QH_FMT_INT4) {
     if (t < kChainN * F::kS) *reinterpret_cast<float2*>(l.sz + 2 * t) = float2{r.s, r.z};
@@ -129,77 +131,126 @@ __device__ __forceinline__ f32x16 chain_mfma(float x, float w, f32x16 c) {
   return __builtin_amdgcn_mfma_f32_32x32x2f32(x, w, c, 0, 0, 0);
 }
 
-// acc (+)= chunk ci of the staged slab for this wave's 32 positions x 32 rows. Accumulator
-// register r holds position 8 (r / 4) + 4 (lane / 32) + r % 4, row lane % 32.
+// One staged chunk's operands in registers for this wave's 32 positions x 32 rows.
 template <int FMT>
-__device__ __forceinline__ void chain_chunk(const ChainLds<FMT>& l, int ci, int wp, int wr, f32x16& acc) {
+struct ChainOps {
+  v4u w;
+  v4f x[ChainFmt<FMT>::kW / 8];
+  f32x16 sx;  // the chunk sums of the lane's accumulator positions (int8: times -128)
+  float2 sz;  // int4: group scale and zero point of the lane's row
+};
+template <int FMT>
+__device__ __forceinline__ void chain_ops(const ChainLds<FMT>& l, int ci, int wp, int wr, ChainOps<FMT>& o) {
   using F = ChainFmt<FMT>;
   const int n = threadIdx.x & 31, h = (threadIdx.x >> 5) & 1;
-  const float* xp = l.x + (32 * wp + n) * kChainXRow + ci * F::kW + 4 * h;
-  const v4u w = *reinterpret_cast<const v4u*>(l.w + (32 * wr + n) * F::kWRow + 16 * ci);
-  v4f xg[F::kW / 8];
+  o.w = *reinterpret_cast<const v4u*>(l.w + (32 * wr + n) * F::kWRow + 16 * ci);
+  const float* xp = l.x + (32 * wp + n) * F::kXRow + ci * F::kW + 4 * h;
 #pragma unroll
-  for (int g = 0; g < F::kW / 8; g++) xg[g] = *reinterpret_cast<const v4f*>(xp + 8 * g);
+  for (int g = 0; g < F::kW / 8; g++) o.x[g] = *reinterpret_cast<const v4f*>(xp + 8 * g);
+  if constexpr (FMT != QH_FMT_F16) {
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const v4f q = *reinterpret_cast<const v4f*>(&l.sx[ci][32 * wp + 8 * i + 4 * h]);
+#pragma unroll
+      for (int e = 0; e < 4; e++) o.sx[4 * i + e] = q[e];
+    }
+  }
+  if constexpr (FMT == QH_FMT_INT4) o.sz = *reinterpret_cast<const float2*>(l.sz + 2 * ((32 * wr + n) * F::kS + ci));
+}
+
+// acc (+)= the chunk. Accumulator register r holds position 8 (r / 4) + 4 (lane / 32) + r % 4,
+// row lane % 32. FIRST: the lane's first chunk, acc starting at 0 (an int8 chunk's sum is
+// never -0: 0 + d is d).
+template <int FMT, bool FIRST>
+__device__ __forceinline__ void chain_chunk(ChainOps<FMT>& o, f32x16& acc) {
+  const int h = (threadIdx.x >> 5) & 1;
+  if constexpr (FIRST && FMT != QH_FMT_INT8) {
+#pragma unroll
+    for (int r = 0; r < 16; r++) acc[r] = 0.f;
+  }
   if constexpr (FMT == QH_FMT_F16) {
 #pragma unroll
-    for (int k = 0; k < 4; k++) acc = chain_mfma(xg[0][k], f16_lo(w[k] >> (16 * h)), acc);
+    for (int k = 0; k < 4; k++) acc = chain_mfma(o.x[0][k], f16_lo(o.w[k] >> (16 * h)), acc);
+  } else if constexpr (FMT == QH_FMT_INT8) {
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      const uint32_t t = o.w[k] >> (8 * h);  // elements 4k + h and 4k + 2 + h in bytes 0 and 2
+      o.sx = chain_mfma(o.x[k >> 1][2 * (k & 1)], ubyte<0>(t), o.sx);
+      o.sx = chain_mfma(o.x[k >> 1][2 * (k & 1) + 1], ubyte<2>(t), o.sx);
+    }
+    if constexpr (FIRST) acc = o.sx;
+    else acc += o.sx;
   } else {
-    v4f sx[4];
+    f32x16 pe, po;
 #pragma unroll
-    for (int i = 0; i < 4; i++) sx[i] = *reinterpret_cast<const v4f*>(&l.sx[ci][32 * wp + 8 * i + 4 * h]);
-    if constexpr (FMT == QH_FMT_INT8) {
-      f32x16 d;
+    for (int r = 0; r < 16; r++) {
+      pe[r] = mul_rounded(-o.sz.y, o.sx[r]) * 0x1p-24f;
+      po[r] = 0.f;
+    }
 #pragma unroll
-      for (int r = 0; r < 16; r++) d[r] = -128.f * sx[r / 4][r % 4];  // exact
+    for (int k = 0; k < 4; k++) {
+      const uint32_t t = o.w[k] >> (8 * h);  // bytes 0 and 2: element pairs 8k + 2h and 8k + 4 + 2h
+      const uint32_t m0 = t & 0x000F000Fu, m1 = t & 0x00F000F0u;
+      pe = chain_mfma(o.x[k].x, f16_lo(m0), pe);
+      po = chain_mfma(o.x[k].y, f16_lo(m1), po);
+      pe = chain_mfma(o.x[k].z, f16_hi(m0), pe);
+      po = chain_mfma(o.x[k].w, f16_hi(m1), po);
+    }
+    const float s = o.sz.x * 0x1p24f;
 #pragma unroll
-      for (int k = 0; k < 4; k++) {
-        const uint32_t t = (w[k] ^ 0x80808080u) >> (8 * h);  // q + 128: elements 4k + h and 4k + 2 + h
-        d = chain_mfma(xg[k >> 1][2 * (k & 1)], ubyte<0>(t), d);
-        d = chain_mfma(xg[k >> 1][2 * (k & 1) + 1], ubyte<2>(t), d);
+    for (int r = 0; r < 16; r++) acc[r] = fmaf(s, fmaf(po[r], 0.0625f, pe[r]), acc[r]);
+  }
+}
+
+// The slab whose first chunk is c0 into the group's slot sums. A whole slab is straight-line
+// code with each chunk's LDS reads issued before the previous chunk's products.
+template <int FMT, bool FIRST>
+__device__ __forceinline__ void chain_slab(const ChainLds<FMT>& l, int c0, int nc, int wp, int wr,
+                                           f32x16 (&acc)[ChainFmt<FMT>::kS]) {
+  constexpr int S = ChainFmt<FMT>::kS;
+  ChainOps<FMT> o[2];
+  if (c0 + S <= nc) {
+    chain_ops<FMT>(l, 0, wp, wr, o[0]);
+#pragma unroll
+    for (int i = 0; i < S; i++) {
+      if (i + 1 < S) chain_ops<FMT>(l, i + 1, wp, wr, o[(i + 1) & 1]);
+      __builtin_amdgcn_sched_barrier(0);
+      chain_chunk<FMT, FIRST>(o[i & 1], acc[i]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < S; i++) {
+      if (c0 + i < nc) {
+        chain_ops<FMT>(l, i, wp, wr, o[0]);
+        chain_chunk<FMT, FIRST>(o[0], acc[i]);
+      } else if constexpr (FIRST) {
+#pragma unroll
+        for (int r = 0; r < 16; r++) acc[i][r] = 0.f;
       }
-#pragma unroll
-      for (int r = 0; r < 16; r++) acc[r] += d[r];
-    } else {
-      const float2 sz = *reinterpret_cast<const float2*>(l.sz + 2 * ((32 * wr + n) * F::kS + ci));
-      f32x16 pe, po;
-#pragma unroll
-      for (int r = 0; r < 16; r++) {
-        pe[r] = mul_rounded(-sz.y, sx[r / 4][r % 4]) * 0x1p-24f;
-        po[r] = 0.f;
-      }
-#pragma unroll
-      for (int k = 0; k < 4; k++) {
-        const uint32_t t = w[k] >> (8 * h);  // bytes 0 and 2: element pairs 8k + 2h and 8k + 4 + 2h
-        const uint32_t m0 = t & 0x000F000Fu, m1 = t & 0x00F000F0u;
-        pe = chain_mfma(xg[k].x, f16_lo(m0), pe);
-        po = chain_mfma(xg[k].y, f16_lo(m1), po);
-        pe = chain_mfma(xg[k].z, f16_hi(m0), pe);
-        po = chain_mfma(xg[k].w, f16_hi(m1), po);
-      }
-#pragma unroll
-      for (int r = 0; r < 16; r++) acc[r] = fmaf(sz.x * 0x1p24f, fmaf(po[r], 0.0625f, pe[r]), acc[r]);
     }
   }
 }
 
-// grid (row blocks, position blocks, splits): split z takes slots z * a.slots .. of the team.
-template <int FMT>
+// grid (row blocks, position blocks, splits): split z takes slots z * a.slots .. of the team,
+// 2^LV groups of kS. MULTI: some lane of the team sums more than one chunk.
+template <int FMT, int LV, bool MULTI>
 __global__ __launch_bounds__(kBlock, 2) void k_chain_f32(ChainArgs a) {
   using F = ChainFmt<FMT>;
   __shared__ __attribute__((aligned(16))) ChainLds<FMT> lds[2];
   const int row0 = blockIdx.x * kChainN, pos0 = blockIdx.y * kChainM;
   const int wave = threadIdx.x / kWave, wp = wave >> 1, wr = wave & 1;
   const int n = threadIdx.x & 31, h = (threadIdx.x >> 5) & 1;
-  const int first = blockIdx.z * a.slots, nc = a.m.nchunks;
-  const int groups = a.slots / F::kS;
+  constexpr int kGroups = 1 << LV;
+  const int first = blockIdx.z * (F::kS * kGroups), nc = a.m.nchunks;
   // Slabs in the order they are summed: group by group, a lane's chunks (tl apart) within it.
   auto slabs_of = [&](int g) {
     const int c = first + g * F::kS;
-    return c < nc ? (nc - 1 - c) / a.tl + 1 : 0;
+    return c < nc ? (MULTI ? (nc - 1 - c) / a.tl + 1 : 1) : 0;
   };
   const bool active = pos0 + 32 * wp < a.seq && row0 + 32 * wr < a.m.rows;  // wave-uniform
 
-  f32x16 st[F::kLevels], root;
+  f32x16 st[LV > 0 ? LV : 1], root;
   ChainRegs<FMT> regs;
   int cur = 0;
   if (slabs_of(0) > 0) {
@@ -207,37 +258,40 @@ __global__ __launch_bounds__(kBlock, 2) void k_chain_f32(ChainArgs a) {
     chain_store<FMT>(regs, lds[0]);
     __syncthreads();
   }
-  for (int g = 0; g < groups; g++) {
+#pragma unroll 1
+  for (int g = 0; g < kGroups; g++) {
     f32x16 acc[F::kS];
-#pragma unroll
-    for (int i = 0; i < F::kS; i++)
-#pragma unroll
-      for (int r = 0; r < 16; r++) acc[i][r] = 0.f;
     const int ns = slabs_of(g);
+    if (ns == 0) {
+#pragma unroll
+      for (int r = 0; r < 16; r++) root[r] = 0.f;
+    }
+#pragma unroll 1
     for (int j = 0; j < ns; j++) {
       const int c0 = first + g * F::kS + j * a.tl;
       // The next slab's chunk: the group's next, else the next group's first, if it has any.
       const int cn = j + 1 < ns ? c0 + a.tl : first + (g + 1) * F::kS;
-      const bool more = j + 1 < ns || (g + 1 < groups && slabs_of(g + 1) > 0);
+      const bool more = j + 1 < ns || (g + 1 < kGroups && slabs_of(g + 1) > 0);
       if (more) chain_load<FMT>(a, row0, pos0, cn, regs);
       if (active) {
-#pragma unroll
-        for (int i = 0; i < F::kS; i++)
-          if (c0 + i < nc) chain_chunk<FMT>(lds[cur], i, wp, wr, acc[i]);
+        if (!MULTI || j == 0) chain_slab<FMT, true>(lds[cur], c0, nc, wp, wr, acc);
+        else chain_slab<FMT, false>(lds[cur], c0, nc, wp, wr, acc);
       }
       if (more) chain_store<FMT>(regs, lds[cur ^ 1]);
       __syncthreads();
       cur ^= 1;
     }
     // The butterfly over the team's lanes: a balanced tree in lane order.
+    if (ns > 0) {
 #pragma unroll
-    for (int w = 1; w < F::kS; w *= 2)
+      for (int w = 1; w < F::kS; w *= 2)
 #pragma unroll
-      for (int i = 0; i < F::kS; i += 2 * w) acc[i] += acc[i + w];
-    root = acc[0];
+        for (int i = 0; i < F::kS; i += 2 * w) acc[i] += acc[i + w];
+      root = acc[0];
+    }
     bool open = true;
 #pragma unroll
-    for (int lv = 0; lv < F::kLevels; lv++) {
+    for (int lv = 0; lv < LV; lv++) {
       if (open) {
         if (g >> lv & 1) root = st[lv] + root;
         else {
@@ -284,7 +338,7 @@ __global__ __launch_bounds__(kBlock) void k_chain_finish(const float* __restrict
 // Splits of the team's slots over blocks: enough that the chip holds about three blocks per CU.
 // A split is a whole subtree of the butterfly, so the splits' roots meet in the same tree.
 static int chain_splits(const DMat& m, int seq) {
-  const int kS = kChainK / weights_per_chunk(m.format), tl = team_width(m.nchunks);
+  const int kS = m.format == QH_FMT_INT4 ? 2 : 4, tl = team_width(m.nchunks);
   const long blocks = (long)((m.rows + kChainN - 1) / kChainN) * ((seq + kChainM - 1) / kChainM);
   int splits = 1;
   while (splits < kChainMaxSplits && blocks * splits < 512 && tl / (2 * splits) >= 2 * kS &&
@@ -303,19 +357,29 @@ size_t chain_partials_bound(const DMat& m, int P) {
   return sizeof(float) * std::min((size_t)kChainMaxSplits * P * m.rows, (size_t)1024 * kChainM * kChainN);
 }
 
+template <int FMT, int LV>
+static void chain_lv(hipStream_t s, const ChainArgs& a, dim3 grid, int lv) {
+  if (lv == LV) {
+    if (a.m.nchunks > a.tl) hipLaunchKernelGGL((k_chain_f32<FMT, LV, true>), grid, dim3(kBlock), 0, s, a);
+    else hipLaunchKernelGGL((k_chain_f32<FMT, LV, false>), grid, dim3(kBlock), 0, s, a);
+  } else if constexpr (LV > 0) {
+    chain_lv<FMT, LV - 1>(s, a, grid, lv);
+  }
+}
+
 template <int FMT>
 static hipError_t chain_fmt(hipStream_t s, const ChainArgs& a0, float* part, int splits) {
   ChainArgs a = a0;
-  float* y = a.y;
   if (splits > 1) a.y = part;
-  a.slots = a.tl / splits;
   const dim3 grid((a.m.rows + kChainN - 1) / kChainN, (a.seq + kChainM - 1) / kChainM, splits);
-  hipLaunchKernelGGL(k_chain_f32<FMT>, grid, dim3(kBlock), 0, s, a);
+  int lv = 0;
+  while ((ChainFmt<FMT>::kS << lv) < a.tl / splits) lv++;
+  chain_lv<FMT, ChainFmt<FMT>::kLevels>(s, a, grid, lv);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || splits == 1) return e;
   const size_t plane = (size_t)a.seq * a.m.rows;
   hipLaunchKernelGGL(k_chain_finish<FMT>, dim3((unsigned)((plane + kBlock - 1) / kBlock)), dim3(kBlock), 0, s, part,
-                     splits, plane, a.m.rows, a.m.scales, a.bias, y);
+                     splits, plane, a.m.rows, a.m.scales, a.bias, a0.y);
   return hipGetLastError();
 }
 
