@@ -181,7 +181,9 @@ PrefillBytes prefill_bytes(const ModelDev& m, const CacheDev& c, int matmul) {
   if (m.numerics == QH_NUMERICS_FAST) b.floats += P * m.heads * kDecodeSlots * kPartStride;
   else if (c.capacity > kPLds) b.floats += P * m.heads * (c.score_stride + attn_spans(c.capacity));
   b.counters = m.numerics == QH_NUMERICS_EXACT ? P * m.heads : 0;
-  size_t scratch = 0;
+  // the layers' and the output head's (enqueue_head_rows)
+  size_t scratch = m.numerics == QH_NUMERICS_EXACT ? matvec_x64_bytes(m.lm_head, kHeadRows)
+                                                   : chain_partials_bound(m.lm_head, kHeadRows);
   for (int L = 0; L < m.layers; L++) {
     const LayerDev& l = m.layers_host[L];
     for (const DMat* w : {&l.qkv, &l.o, &l.gu, &l.down}) {
@@ -389,6 +391,13 @@ hipError_t enqueue_prefill_layers(hipStream_t s, const ModelDev& m, const CacheD
     if ((e = launch_add(s, p.X, p.Y, (int)n)) != hipSuccess) return e;
   }
   return hipSuccess;
+}
+
+hipError_t enqueue_head_rows(hipStream_t s, const ModelDev& m, const PrefillDev& p, int first, int n, float* logits) {
+  const hipError_t e = launch_rmsnorm(s, p.X + (size_t)first * m.hidden, m.final_norm, p.XN, n, m.hidden, m.eps,
+                                      m.numerics == QH_NUMERICS_FAST);
+  if (e != hipSuccess) return e;
+  return matmul(s, m, QH_MATMUL_BATCHED, m.lm_head, p.XN, nullptr, logits, n, p);
 }
 
 hipError_t enqueue_embed_rows(hipStream_t s, const ModelDev& m, const CacheDev& c, const PrefillDev& p, int past,

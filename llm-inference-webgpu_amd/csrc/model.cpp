@@ -142,6 +142,9 @@ struct qh_cache {
   qh::PrefillBytes pw_bytes{};
   void* pw_mem = nullptr;
   int pw_matmul = -1;  // the matmul mode the workspace was last checked for
+  // Scoring workspace, kept from the first qh_score: logits of kHeadRows rows, their partials
+  // and the scores of a whole cache.
+  void* score_mem = nullptr;
 
   int alloc(size_t n, void** p) {
     if (hipMalloc(p, n ? n : 4) != hipSuccess) return fail(QH_ERR_NOMEM, "hipMalloc of %zu bytes failed", n);
@@ -650,6 +653,7 @@ int qh_cache_free(qh_cache* c) {
   for (void* p : c->allocs) hipFree(p);
   hipFree(c->d_hidden);
   if (c->pw_mem) hipFree(c->pw_mem);
+  if (c->score_mem) hipFree(c->score_mem);
   hipHostFree(c->h_pinned);
   c->m->live_caches--;
   delete c;
@@ -781,7 +785,7 @@ int ensure_prefill(qh_cache* c) {
 // so a one-off length pays no capture), which removes the host's per-launch cost and the
 // device's gaps between the ~250 launches; the least recently used of kPrefillGraphs shapes
 // makes room for a new one. use_graph = 0 (qh_decode_use_graph) enqueues directly.
-static int prefill_chunk(qh_cache* c, bool tokens, int past, int n) {
+static int prefill_chunk(qh_cache* c, int matmul, bool tokens, int past, int n) {
   qh_model* m = c->m;
   hipStream_t s = m->ctx->stream;
   const qh::ModelDev& d = m->dev;
@@ -790,7 +794,7 @@ static int prefill_chunk(qh_cache* c, bool tokens, int past, int n) {
       const hipError_t e = qh::enqueue_embed_rows(s, d, c->dev, c->pw, past, n);
       if (e != hipSuccess) return e;
     }
-    return qh::enqueue_prefill_layers(s, d, c->dev, c->pw, m->matmul, past, n);
+    return qh::enqueue_prefill_layers(s, d, c->dev, c->pw, matmul, past, n);
   };
   if (!c->use_graph) {
     QH_HIP(enqueue());
@@ -798,7 +802,7 @@ static int prefill_chunk(qh_cache* c, bool tokens, int past, int n) {
   }
   PrefillGraph* g = nullptr;
   for (PrefillGraph& e : c->pgraphs)
-    if (e.past == past && e.n == n && e.matmul == m->matmul && e.numerics == d.numerics && e.tokens == tokens) g = &e;
+    if (e.past == past && e.n == n && e.matmul == matmul && e.numerics == d.numerics && e.tokens == tokens) g = &e;
   if (!g) {
     if ((int)c->pgraphs.size() >= kPrefillGraphs) {
       auto lru = std::min_element(c->pgraphs.begin(), c->pgraphs.end(),
@@ -808,7 +812,7 @@ static int prefill_chunk(qh_cache* c, bool tokens, int past, int n) {
       if (lru->graph) hipGraphDestroy(lru->graph);
       c->pgraphs.erase(lru);
     }
-    c->pgraphs.push_back(PrefillGraph{past, n, m->matmul, d.numerics, tokens, 0, 0, nullptr, nullptr});
+    c->pgraphs.push_back(PrefillGraph{past, n, matmul, d.numerics, tokens, 0, 0, nullptr, nullptr});
     g = &c->pgraphs.back();
   }
   g->last = ++c->pclock;
@@ -853,7 +857,7 @@ int batched_forward(qh_cache* c, const float* h_hidden, int seq, bool want, int 
       QH_HIP(hipMemcpyAsync(c->pw.X, h_hidden + (size_t)done * d.hidden, (size_t)n * d.hidden * 4,
                             hipMemcpyHostToDevice, s));
     }
-    if ((rc = prefill_chunk(c, h_hidden == nullptr, past, n))) return rc;
+    if ((rc = prefill_chunk(c, m->matmul, h_hidden == nullptr, past, n))) return rc;
   }
   QH_HIP(hipMemcpyAsync(c->dev.x, c->pw.X + (size_t)(n - 1) * d.hidden, (size_t)d.hidden * 4,
                         hipMemcpyDeviceToDevice, s));
@@ -862,6 +866,23 @@ int batched_forward(qh_cache* c, const float* h_hidden, int seq, bool want, int 
     QH_HIP(qh::enqueue_head(s, d, c->dev));
   } else if ((rc = set_state(c, c->length + seq, forced))) {
     return rc;
+  }
+  return QH_OK;
+}
+
+// The scoring workspace: kHeadRows rows of logits, their partials, and a score per position.
+size_t score_logits_bytes(const qh::ModelDev& d) {
+  return ((size_t)qh::kHeadRows * d.vocab * 4 + 255) & ~(size_t)255;
+}
+size_t score_parts_bytes() { return (qh::nll_partials_bytes(qh::kHeadRows) + 255) & ~(size_t)255; }
+int ensure_score(qh_cache* c) {
+  const int rc = ensure_prefill(c);
+  if (rc || c->score_mem) return rc;
+  const qh::ModelDev& d = c->m->dev;
+  const size_t bytes = score_logits_bytes(d) + score_parts_bytes() + (size_t)c->dev.capacity * 8;
+  if (hipMalloc(&c->score_mem, bytes) != hipSuccess) {
+    c->score_mem = nullptr;
+    return fail(QH_ERR_NOMEM, "scoring workspace of %zu bytes", bytes);
   }
   return QH_OK;
 }
@@ -950,27 +971,63 @@ int qh_score(qh_model* m, qh_cache* c, const int32_t* h_ids, int32_t n, double* 
   BusyGuard guard(c);
   QH_HIP(hipSetDevice(m->ctx->device));
   hipStream_t s = m->ctx->stream;
+  const int total = n - 1;
+  const qh::ModelDev& md = m->dev;
+  // ids[0..n-2] are fed (teacher-forced); ids[t+1] is scored under position t's logits.
+  if (total >= 2 && ensure_score(c) == QH_OK) {
+    // The positions run as the batched prefill and the head over its rows, kHeadRows at a time:
+    // the logits have the bits of one decode step after another.
+    char* mem = static_cast<char*>(c->score_mem);
+    float* logits = reinterpret_cast<float*>(mem);
+    void* parts = mem + score_logits_bytes(md);
+    double* nll = reinterpret_cast<double*>(mem + score_logits_bytes(md) + score_parts_bytes());
+    int32_t* tokens = c->dev.tokens + c->length;  // capacity + 1 entries: room for all n
+    QH_HIP(hipMemcpyAsync(tokens, h_ids, (size_t)n * 4, hipMemcpyHostToDevice, s));
+    const int P = c->pw.positions;
+    int k = 0;
+    for (int done = 0; done < total; done += k) {
+      k = std::min(P, total - done);
+      if ((rc = prefill_chunk(c, QH_MATMUL_BATCHED, true, c->length + done, k))) return rc;
+      for (int r = 0; r < k; r += qh::kHeadRows) {
+        const int rows = std::min(qh::kHeadRows, k - r);
+        QH_HIP(qh::enqueue_head_rows(s, md, c->pw, r, rows, logits));
+        QH_HIP(qh::launch_nll(s, logits, md.vocab, tokens + 1 + done + r, rows, parts, nll + done + r));
+      }
+    }
+    // The cache is left as a forward of the last position leaves it.
+    QH_HIP(hipMemcpyAsync(c->dev.x, c->pw.X + (size_t)(k - 1) * md.hidden, (size_t)md.hidden * 4,
+                          hipMemcpyDeviceToDevice, s));
+    if ((rc = set_state(c, c->length + total - 1, c->length + total))) return rc;
+    QH_HIP(qh::enqueue_head(s, md, c->dev));
+    QH_HIP(hipMemcpyAsync(h_nll, nll, (size_t)total * 8, hipMemcpyDeviceToHost, s));
+    QH_HIP(hipStreamSynchronize(s));
+    c->length += total;
+    return QH_OK;
+  }
+  // A single position, or no memory for the workspace: one decode step after another.
   struct Scratch {
     int32_t* ids = nullptr;
     double* nll = nullptr;
+    void* parts = nullptr;
     ~Scratch() {
       hipFree(ids);
       hipFree(nll);
+      hipFree(parts);
     }
   } d;
   QH_HIP(hipMalloc((void**)&d.ids, (size_t)n * 4));
-  QH_HIP(hipMalloc((void**)&d.nll, (size_t)(n - 1) * 8));
+  QH_HIP(hipMalloc((void**)&d.nll, (size_t)total * 8));
+  QH_HIP(hipMalloc(&d.parts, qh::nll_partials_bytes(1)));
   QH_HIP(hipMemcpyAsync(d.ids, h_ids, (size_t)n * 4, hipMemcpyHostToDevice, s));
-  // ids[0..n-2] are fed (teacher-forced); ids[t+1] is scored under step t's logits.
-  QH_HIP(hipMemcpyAsync(c->dev.tokens + c->length, d.ids, (size_t)(n - 1) * 4, hipMemcpyDeviceToDevice, s));
-  if ((rc = set_state(c, c->length, c->length + n - 1))) return rc;
-  for (int t = 0; t < n - 1; t++) {
-    QH_HIP(qh::enqueue_step(s, m->dev, c->dev, qh::STEP_GATHER, true));
-    QH_HIP(qh::launch_nll(s, c->dev.logits, m->dev.vocab, d.ids + t + 1, d.nll + t));
+  QH_HIP(hipMemcpyAsync(c->dev.tokens + c->length, d.ids, (size_t)total * 4, hipMemcpyDeviceToDevice, s));
+  if ((rc = set_state(c, c->length, c->length + total))) return rc;
+  for (int t = 0; t < total; t++) {
+    QH_HIP(qh::enqueue_step(s, md, c->dev, qh::STEP_GATHER, true));
+    QH_HIP(qh::launch_nll(s, c->dev.logits, md.vocab, d.ids + t + 1, 1, d.parts, d.nll + t));
   }
-  QH_HIP(hipMemcpyAsync(h_nll, d.nll, (size_t)(n - 1) * 8, hipMemcpyDeviceToHost, s));
+  QH_HIP(hipMemcpyAsync(h_nll, d.nll, (size_t)total * 8, hipMemcpyDeviceToHost, s));
   QH_HIP(hipStreamSynchronize(s));
-  c->length += n - 1;
+  c->length += total;
   return QH_OK;
 }
 

@@ -99,6 +99,11 @@ PrefillBytes prefill_bytes(const ModelDev& m, const CacheDev& c, int matmul);
 // Layers of positions past .. past+seq-1 over p.X (seq <= p.positions), writing the KV cache.
 hipError_t enqueue_prefill_layers(hipStream_t s, const ModelDev& m, const CacheDev& c, const PrefillDev& p,
                                   int matmul, int past, int seq);
+// Rows of the output head enqueue_head_rows takes at once: 39 MB of logits for 151936 tokens.
+constexpr int kHeadRows = 64;
+// logits [n][vocab] = the output head over rows first .. first+n-1 of p.X (n <= kHeadRows), each
+// the bits of a decode step's head over that row (overwrites p.XN's first rows).
+hipError_t enqueue_head_rows(hipStream_t s, const ModelDev& m, const PrefillDev& p, int first, int n, float* logits);
 // p.X = embeddings of cache tokens[past .. past+seq-1].
 hipError_t enqueue_embed_rows(hipStream_t s, const ModelDev& m, const CacheDev& c, const PrefillDev& p, int past,
                               int seq);

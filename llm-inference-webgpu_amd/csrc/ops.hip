@@ -726,18 +726,27 @@ hipError_t launch_argmax(hipStream_t s, const float* v, int n, int* counter, voi
 // The negative log-likelihood of *target under one position's logits, as the reference's
 // perplexity page computes it (web/perplexity.html:158-166): the largest logit (a NaN is
 // skipped, as `>` skips it), the f64 sum of exp(l - max) over the vocabulary, then
-// -(l[target] - max - log(sum)). One block of 1024 threads; per-thread strided f64 sums
-// combined in a fixed tree, so every run gives the same bits.
-constexpr int kNllThreads = 1024;
-__global__ __launch_bounds__(kNllThreads) void k_nll(const float* __restrict__ logits, int vocab,
-                                                     const int32_t* __restrict__ target, double* __restrict__ out) {
+// -(l[target] - max - log(sum)). grid (kNllParts, rows): a row's vocabulary in kNllParts spans of
+// their own maxima and f64 sums (per-thread strided, combined in a fixed tree, so every run gives
+// the same bits), which k_nll_finish rescales to the row's maximum. Bound: the f64 exponentials
+// and the latency of two passes; one block per row took 80 us for 151936 logits.
+constexpr int kNllThreads = 1024, kNllParts = 8;
+struct NllPart {
+  double sum;
+  float max;
+};
+__global__ __launch_bounds__(kNllThreads) void k_nll_part(const float* __restrict__ logits, int vocab,
+                                                          NllPart* __restrict__ part) {
   __shared__ float wmax[kNllThreads / kWave];
   __shared__ double wsum[kNllThreads / kWave];
   const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
+  const int span = (vocab + gridDim.x - 1) / gridDim.x;
+  const int end = min(vocab, (int)(blockIdx.x + 1) * span);
+  const float* l = logits + (size_t)blockIdx.y * vocab;
   float mx = -INFINITY;
-  for (int i = tid; i < vocab; i += kNllThreads) {
-    const float l = logits[i];
-    if (l > mx) mx = l;
+  for (int i = blockIdx.x * span + tid; i < end; i += kNllThreads) {
+    const float v = l[i];
+    if (v > mx) mx = v;
   }
   for (int off = kWave / 2; off > 0; off >>= 1) {
     const float o = __shfl_xor(mx, off);
@@ -749,9 +758,9 @@ __global__ __launch_bounds__(kNllThreads) void k_nll(const float* __restrict__ l
 #pragma unroll
   for (int w = 1; w < kNllThreads / kWave; w++)
     if (wmax[w] > mx) mx = wmax[w];
-  const double m = (double)mx;
+  const double m = mx == -INFINITY ? 0.0 : (double)mx;  // a part of -inf alone sums to 0
   double sum = 0.0;
-  for (int i = tid; i < vocab; i += kNllThreads) sum += exp((double)logits[i] - m);
+  for (int i = blockIdx.x * span + tid; i < end; i += kNllThreads) sum += exp((double)l[i] - m);
   for (int off = kWave / 2; off > 0; off >>= 1) sum += __shfl_xor(sum, off);
   if (lane == 0) wsum[wave] = sum;
   __syncthreads();
@@ -759,12 +768,33 @@ __global__ __launch_bounds__(kNllThreads) void k_nll(const float* __restrict__ l
     double total = 0.0;
 #pragma unroll
     for (int w = 0; w < kNllThreads / kWave; w++) total += wsum[w];
-    *out = -((double)logits[*target] - m - log(total));
+    part[(size_t)blockIdx.y * gridDim.x + blockIdx.x] = {total, mx};
   }
 }
 
-hipError_t launch_nll(hipStream_t s, const float* logits, int vocab, const int32_t* target, double* out) {
-  hipLaunchKernelGGL(k_nll, dim3(1), dim3(kNllThreads), 0, s, logits, vocab, target, out);
+// out[row] from the row's parts, one thread per row.
+__global__ void k_nll_finish(const float* __restrict__ logits, int vocab, const int32_t* __restrict__ target,
+                             const NllPart* __restrict__ part, int rows, double* __restrict__ out) {
+  const int r = blockIdx.x * blockDim.x + threadIdx.x;
+  if (r >= rows) return;
+  const NllPart* p = part + (size_t)r * kNllParts;
+  float mx = -INFINITY;
+  for (int k = 0; k < kNllParts; k++)
+    if (p[k].max > mx) mx = p[k].max;
+  const double m = (double)mx;
+  double total = 0.0;
+  for (int k = 0; k < kNllParts; k++) total += p[k].sum * exp((double)p[k].max - m);
+  out[r] = -((double)logits[(size_t)r * vocab + target[r]] - m - log(total));
+}
+
+size_t nll_partials_bytes(int rows) { return (size_t)rows * kNllParts * sizeof(NllPart); }
+
+hipError_t launch_nll(hipStream_t s, const float* logits, int vocab, const int32_t* target, int rows, void* partials,
+                      double* out) {
+  NllPart* part = static_cast<NllPart*>(partials);
+  hipLaunchKernelGGL(k_nll_part, dim3(kNllParts, rows), dim3(kNllThreads), 0, s, logits, vocab, part);
+  hipLaunchKernelGGL(k_nll_finish, dim3((rows + kWave - 1) / kWave), dim3(kWave), 0, s, logits, vocab, target, part,
+                     rows, out);
   return hipGetLastError();
 }
 
