@@ -401,4 +401,247 @@ hipError_t launch_chain_f32(hipStream_t s, const DMat& m, const float* x, const 
   }
 }
 
+// --------------------------------------------------------------- f64 order --
+// The exact matvec (k_matvec of ops.hip: the loader's f32 weights, f64 sums) over several
+// positions on v_mfma_f64_16x16x4f64, whose four k are ascending fused multiply-adds as above:
+// the accumulator runs through a lane's chunks, so every output has k_matvec's bits.
+//
+// Bound: the f64 matrix rate (70 TFLOP/s in a large product), which the vector unit's f64 shares
+// with everything else it does; what the VALU form lost was one LDS read of x per two products
+// and a dequantized weight per eight positions. A block takes 32 positions x 16 rows, its four
+// waves a quarter of the team's slots each (so 52 positions of a 4864-row matrix are 608 blocks),
+// joined through LDS in tree order. A wave stages its own slabs of x, so no barrier runs in the
+// loop; weights go to registers a chunk ahead. 4864 x 896 int8, 52 positions: 90 -> X us.
+typedef double f64x4 __attribute__((ext_vector_type(4)));
+
+template <int FMT>
+struct Chain64 {
+  static constexpr int kW = Fmt<FMT>::kW;
+  static constexpr int kS = FMT == QH_FMT_INT4 ? 2 : 4;  // slots per slab
+  static constexpr int kK = kS * kW;
+  static constexpr int kXRow = kK + 4;
+  static constexpr int kLevels = FMT == QH_FMT_INT4 ? 3 : 2;  // log2 of a wave's groups, 16 slots at most
+};
+constexpr int kChain64M = 32, kChain64N = 16;
+
+// One chunk of one row as the loader's f32 weights: w(s) is the lane's element 4s + g.
+template <int FMT>
+struct RowChunk {
+  v4u w;
+  float s, z;
+  int zi;
+  bool zint;
+  __device__ __forceinline__ void set(v4u w_, float s_, float z_) {
+    w = w_;
+    s = s_;
+    z = z_;
+    if constexpr (FMT == QH_FMT_INT4) {
+      zi = (int)z_;
+      zint = (float)zi == z_ && (unsigned)zi <= 15u;  // what the quantizer writes
+    }
+  }
+  template <int STEP>
+  __device__ __forceinline__ double at(int g) const {
+    if constexpr (FMT == QH_FMT_F16) {
+      const uint32_t d = g < 2 ? w[2 * STEP] : w[2 * STEP + 1];
+      return (double)f16_lo(d >> (16 * (g & 1)));
+    } else if constexpr (FMT == QH_FMT_INT8) {
+      return (double)((float)(int8_t)(uint8_t)(w[STEP] >> (8 * g)) * s);  // q*s is exact before rounding
+    } else {
+      const int lv = (int)((w[STEP / 2] >> (16 * (STEP & 1) + 4 * g)) & 0xfu);
+      if (zint) return (double)((float)(lv - zi) * s);  // exact before rounding
+      return (double)(float)(((double)lv - (double)z) * (double)s);
+    }
+  }
+};
+
+// acc[tile] += one chunk for 16 rows x two tiles of 16 positions (`two`: the second has any).
+// Accumulator register r holds position 4r + lane / 16, row lane % 16.
+template <int FMT, int STEPS, int K = 0>
+__device__ __forceinline__ void chain64_steps(const RowChunk<FMT>& rc, const float (&xv)[2][STEPS], int g, bool two,
+                                              f64x4 (&acc)[2]) {
+  if constexpr (K < STEPS) {
+    const double w = rc.template at<K>(g);
+    acc[0] = __builtin_amdgcn_mfma_f64_16x16x4f64((double)xv[0][K], w, acc[0], 0, 0, 0);
+    if (two) acc[1] = __builtin_amdgcn_mfma_f64_16x16x4f64((double)xv[1][K], w, acc[1], 0, 0, 0);
+    chain64_steps<FMT, STEPS, K + 1>(rc, xv, g, two, acc);
+  }
+}
+
+template <int FMT, bool MULTI>
+__global__ __launch_bounds__(kBlock, 2) void k_chain_f64(ChainArgs a) {
+  using F = Chain64<FMT>;
+  constexpr int S = F::kS, kLoads = kChain64M * F::kK / 4 / kWave;
+  // A wave's slab of x (its LDS operations run in order, so the next slab is stored over it after
+  // its reads), then its sums [tile][register][lane].
+  __shared__ __attribute__((aligned(16))) float xs[kBlock / kWave][kChain64M * F::kXRow];
+  static_assert(2 * 4 * kWave * 2 <= kChain64M * F::kXRow, "the sums fit the slab");
+  const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave, n = lane & 15, g4 = lane >> 4;
+  const int row0 = blockIdx.x * kChain64N, pos0 = blockIdx.y * kChain64M;
+  const int nc = a.m.nchunks, slots = a.tl / (kBlock / kWave), first = wave * slots, groups = slots / S;
+  const int row = min(row0 + n, a.m.rows - 1);
+  const bool two = pos0 + 16 < a.seq;  // uniform: the second position tile has any
+  const v4u* rp = reinterpret_cast<const v4u*>(a.m.data + (size_t)row * a.m.row_bytes);
+  const float srow = FMT == QH_FMT_INT8 ? a.m.scales[row] : 0.f;
+  auto slabs_of = [&](int g) {
+    const int c = first + g * S;
+    return c < nc ? (MULTI ? (nc - 1 - c) / a.tl + 1 : 1) : 0;
+  };
+  // x of a slab: 32 positions x kK columns, one float4 per lane and load.
+  v4f xr[kLoads];
+  v4u wr[S];
+  float sr[S], zr[S];
+  auto load = [&](int c0) {
+#pragma unroll
+    for (int j = 0; j < kLoads; j++) {
+      const int i = lane + j * kWave, p = min(pos0 + i / (F::kK / 4), a.seq - 1);
+      const int col = min(c0 * F::kW + 4 * (i % (F::kK / 4)), a.m.cols - 4);
+      xr[j] = *reinterpret_cast<const v4f*>(a.x + (size_t)p * a.m.cols + col);
+    }
+#pragma unroll
+    for (int i = 0; i < S; i++) {
+      const int c = min(c0 + i, nc - 1);
+      wr[i] = rp[c];
+      if constexpr (FMT == QH_FMT_INT4) {
+        sr[i] = a.m.scales[(size_t)row * a.m.gpr + c / a.m.cpg];
+        zr[i] = a.m.zeros[(size_t)row * a.m.gpr + c / a.m.cpg];
+      } else {
+        sr[i] = srow;
+        zr[i] = 0.f;
+      }
+    }
+  };
+  // Stored with each 16 columns as [k % 4][k / 4], so a lane's element of four instructions is
+  // one ds_read_b128 (f16's 8-column chunks: halves of it).
+  auto store = [&](float* dst) {
+#pragma unroll
+    for (int j = 0; j < kLoads; j++) {
+      const int i = lane + j * kWave, p = i / (F::kK / 4), q = i % (F::kK / 4);
+      float* d = dst + p * F::kXRow + 16 * (q >> 2) + (q & 3);
+      d[0] = xr[j].x;
+      d[4] = xr[j].y;
+      d[8] = xr[j].z;
+      d[12] = xr[j].w;
+    }
+  };
+  f64x4 st[F::kLevels][2], root[2];
+  if (slabs_of(0) > 0) {
+    load(first);
+    store(xs[wave]);
+  }
+#pragma unroll 1
+  for (int g = 0; g < groups; g++) {
+    f64x4 acc[S][2];
+#pragma unroll
+    for (int i = 0; i < S; i++)
+#pragma unroll
+      for (int t = 0; t < 2; t++) acc[i][t] = (f64x4){0.0, 0.0, 0.0, 0.0};
+    const int ns = slabs_of(g);
+#pragma unroll 1
+    for (int j = 0; j < ns; j++) {
+      const int c0 = first + g * S + j * a.tl;
+      const int cn = j + 1 < ns ? c0 + a.tl : first + (g + 1) * S;
+      const bool more = j + 1 < ns || (g + 1 < groups && slabs_of(g + 1) > 0);
+      RowChunk<FMT> rc[S];
+#pragma unroll
+      for (int i = 0; i < S; i++) rc[i].set(wr[i], sr[i], zr[i]);
+      if (more) load(cn);
+      __builtin_amdgcn_wave_barrier();  // the wave's own stores of this slab precede its reads
+      const float* xb = xs[wave];
+#pragma unroll
+      for (int i = 0; i < S; i++) {
+        if (c0 + i < nc) {
+          constexpr int kSteps = F::kW / 4;
+          float xv[2][kSteps];
+#pragma unroll
+          for (int t = 0; t < 2; t++) {
+            const float* xp = xb + (16 * t + n) * F::kXRow + 4 * g4;
+            if constexpr (FMT == QH_FMT_F16) {
+              const float2 v = *reinterpret_cast<const float2*>(xp + 16 * (i >> 1) + 2 * (i & 1));
+              xv[t][0] = v.x;
+              xv[t][1] = v.y;
+            } else {
+#pragma unroll
+              for (int q = 0; q < kSteps / 4; q++) {
+                const v4f v = *reinterpret_cast<const v4f*>(xp + i * F::kW + 16 * q);
+#pragma unroll
+                for (int e = 0; e < 4; e++) xv[t][4 * q + e] = v[e];
+              }
+            }
+          }
+          chain64_steps<FMT, kSteps>(rc[i], xv, g4, two, acc[i]);
+        }
+      }
+      __builtin_amdgcn_wave_barrier();
+      if (more) store(xs[wave]);
+    }
+#pragma unroll
+    for (int w = 1; w < S; w *= 2)
+#pragma unroll
+      for (int i = 0; i < S; i += 2 * w)
+#pragma unroll
+        for (int t = 0; t < 2; t++) acc[i][t] += acc[i + w][t];
+    bool open = true;
+#pragma unroll
+    for (int t = 0; t < 2; t++) root[t] = acc[0][t];
+#pragma unroll
+    for (int lv = 0; lv < F::kLevels; lv++) {
+      if (open) {
+        if (g >> lv & 1) {
+#pragma unroll
+          for (int t = 0; t < 2; t++) root[t] = st[lv][t] + root[t];
+        } else {
+#pragma unroll
+          for (int t = 0; t < 2; t++) st[lv][t] = root[t];
+          open = false;
+        }
+      }
+    }
+  }
+#pragma unroll
+  for (int t = 0; t < 2; t++)
+#pragma unroll
+    for (int r = 0; r < 4; r++) reinterpret_cast<double*>(xs[wave])[(t * 4 + r) * kWave + lane] = root[t][r];
+  __syncthreads();
+  // Wave w finishes register w of both tiles: position 16t + 4r + lane / 16, row lane % 16.
+  if (row0 + n >= a.m.rows) return;
+#pragma unroll
+  for (int t = 0; t < 2; t++) {
+    const int p = pos0 + 16 * t + 4 * wave + g4;
+    if (p < a.seq) {
+      double q[kBlock / kWave];
+#pragma unroll
+      for (int w = 0; w < kBlock / kWave; w++) q[w] = reinterpret_cast<const double*>(xs[w])[(t * 4 + wave) * kWave + lane];
+      const double v = (q[0] + q[1]) + (q[2] + q[3]);
+      a.y[(size_t)p * a.m.rows + row] = (float)(a.bias ? v + (double)a.bias[row] : v);
+    }
+  }
+}
+
+bool chain_f64_supported(const DMat& m, const float* x, int seq) {
+  return seq >= kChain64MinSeq && m.cols % 4 == 0 && ((uintptr_t)x & 15) == 0;
+}
+
+hipError_t launch_chain_f64(hipStream_t s, const DMat& m, const float* x, const float* bias, float* y, int seq) {
+  ChainArgs a{};
+  a.m = m;
+  a.x = x;
+  a.bias = bias;
+  a.y = y;
+  a.seq = seq;
+  a.tl = team_width(m.nchunks);
+  const dim3 grid((m.rows + kChain64N - 1) / kChain64N, (seq + kChain64M - 1) / kChain64M);
+  const bool multi = m.nchunks > a.tl;
+  auto go = [&](auto one, auto many) {
+    if (multi) hipLaunchKernelGGL(many, grid, dim3(kBlock), 0, s, a);
+    else hipLaunchKernelGGL(one, grid, dim3(kBlock), 0, s, a);
+  };
+  switch (m.format) {
+    case QH_FMT_F16: go(k_chain_f64<QH_FMT_F16, false>, k_chain_f64<QH_FMT_F16, true>); break;
+    case QH_FMT_INT8: go(k_chain_f64<QH_FMT_INT8, false>, k_chain_f64<QH_FMT_INT8, true>); break;
+    default: go(k_chain_f64<QH_FMT_INT4, false>, k_chain_f64<QH_FMT_INT4, true>); break;
+  }
+  return hipGetLastError();
+}
+
 }  // namespace qh

@@ -181,14 +181,14 @@ PrefillBytes prefill_bytes(const ModelDev& m, const CacheDev& c, int matmul) {
   if (m.numerics == QH_NUMERICS_FAST) b.floats += P * m.heads * kDecodeSlots * kPartStride;
   else if (c.capacity > kPLds) b.floats += P * m.heads * (c.score_stride + attn_spans(c.capacity));
   b.counters = m.numerics == QH_NUMERICS_EXACT ? P * m.heads : 0;
-  // the layers' and the output head's (enqueue_head_rows)
-  size_t scratch = m.numerics == QH_NUMERICS_EXACT ? matvec_x64_bytes(m.lm_head, kHeadRows)
-                                                   : chain_partials_bound(m.lm_head, kHeadRows);
+  const bool chain = m.numerics == QH_NUMERICS_FAST && !(matmul == QH_MATMUL_MFMA && all_mfma(m));
+  size_t scratch = chain ? chain_partials_bound(m.lm_head, kHeadRows) : 0;  // enqueue_head_rows
+  if (m.numerics == QH_NUMERICS_EXACT) scratch = matvec_x64_bytes(m.lm_head, kHeadRows);
   for (int L = 0; L < m.layers; L++) {
     const LayerDev& l = m.layers_host[L];
     for (const DMat* w : {&l.qkv, &l.o, &l.gu, &l.down}) {
       if (m.numerics == QH_NUMERICS_EXACT) scratch = std::max(scratch, matvec_x64_bytes(*w, (int)P));
-      else scratch = std::max(scratch, chain_partials_bound(*w, (int)P));
+      if (chain) scratch = std::max(scratch, chain_partials_bound(*w, (int)P));
       if (matmul == QH_MATMUL_MFMA && matmul_prefill_supported(*w))
         scratch = std::max(scratch, matmul_prefill_scratch_bytes(*w, (int)P));
     }

@@ -735,17 +735,20 @@ int finish_forward(qh_cache* c, int seq, float* h_logits, int32_t* h_argmax) {
 
 // The batched-prefill workspace for the model's current matmul mode: one allocation,
 // carved in the order prefill_bytes() counts it.
-int ensure_prefill(qh_cache* c) {
+int ensure_prefill(qh_cache* c, int matmul) {
   qh_model* m = c->m;
   // The sizes depend on the model, the cache and the matmul mode only: checked once per mode
   // (they walk every layer matrix on the host, in front of the forward's first launch).
-  if (c->pw_mem && c->pw_matmul == m->matmul) return QH_OK;
-  const qh::PrefillBytes b = qh::prefill_bytes(m->dev, c->dev, m->matmul);
+  if (c->pw_mem && c->pw_matmul == matmul) return QH_OK;
+  qh::PrefillBytes b = qh::prefill_bytes(m->dev, c->dev, matmul);
   if (c->pw_mem && b.floats <= c->pw_bytes.floats && b.counters <= c->pw_bytes.counters &&
       b.scratch <= c->pw_bytes.scratch) {
-    c->pw_matmul = m->matmul;
+    c->pw_matmul = matmul;
     return QH_OK;
   }
+  b.floats = std::max(b.floats, c->pw_bytes.floats);  // modes in turn keep one workspace
+  b.counters = std::max(b.counters, c->pw_bytes.counters);
+  b.scratch = std::max(b.scratch, c->pw_bytes.scratch);
   hipStream_t s = m->ctx->stream;
   QH_HIP(hipStreamSynchronize(s));
   drop_prefill_graphs(c);  // they address the workspace being replaced
@@ -758,7 +761,7 @@ int ensure_prefill(qh_cache* c) {
   }
   QH_HIP(hipMemsetAsync(static_cast<char*>(c->pw_mem) + fbytes, 0, cbytes, s));
   c->pw_bytes = b;
-  c->pw_matmul = m->matmul;
+  c->pw_matmul = matmul;
   const qh::ModelDev& d = m->dev;
   const size_t P = qh::prefill_chunk(d, c->dev);
   const size_t hd = d.hidden, kv = (size_t)d.kv_heads * d.head_dim, f = d.intermediate;
@@ -844,7 +847,7 @@ static int prefill_chunk(qh_cache* c, int matmul, bool tokens, int past, int n) 
 // cache's tokens) pass through the layers in chunks, then the last row through the head.
 int batched_forward(qh_cache* c, const float* h_hidden, int seq, bool want, int forced) {
   qh_model* m = c->m;
-  int rc = ensure_prefill(c);
+  int rc = ensure_prefill(c, m->matmul);
   if (rc) return rc;
   hipStream_t s = m->ctx->stream;
   const qh::ModelDev& d = m->dev;
@@ -876,7 +879,7 @@ size_t score_logits_bytes(const qh::ModelDev& d) {
 }
 size_t score_parts_bytes() { return (qh::nll_partials_bytes(qh::kHeadRows) + 255) & ~(size_t)255; }
 int ensure_score(qh_cache* c) {
-  const int rc = ensure_prefill(c);
+  const int rc = ensure_prefill(c, QH_MATMUL_BATCHED);
   if (rc || c->score_mem) return rc;
   const qh::ModelDev& d = c->m->dev;
   const size_t bytes = score_logits_bytes(d) + score_parts_bytes() + (size_t)c->dev.capacity * 8;

@@ -126,6 +126,7 @@ size_t matvec_x64_bytes(const DMat& m, int seq) {
 
 hipError_t launch_matvec(hipStream_t s, const DMat& m, const float* x, const float* bias, float* y,
                          int seq, double* x64_scratch) {
+  if (chain_f64_supported(m, x, seq)) return launch_chain_f64(s, m, x, bias, y, seq);
   const size_t need = matvec_x64_bytes(m, seq);
   double* x64 = nullptr;
   hipError_t e = hipSuccess;

@@ -98,6 +98,11 @@ hipError_t launch_chain_f32(hipStream_t s, const DMat& m, const float* x, const 
                             float* part, size_t part_bytes);
 constexpr int kChainMaxSplits = 8;
 size_t chain_partials_bytes(const DMat& m, int seq);
+// launch_matvec's sums, bit for bit, on the f64 matrix cores (chain.hip), from kChain64MinSeq
+// positions and for 16-byte aligned x.
+constexpr int kChain64MinSeq = 8;
+bool chain_f64_supported(const DMat& m, const float* x, int seq);
+hipError_t launch_chain_f64(hipStream_t s, const DMat& m, const float* x, const float* bias, float* y, int seq);
 size_t chain_partials_bound(const DMat& m, int P);
 // The batched-prefill contraction on the int8 matrix cores over exact activation digits (int8 /
 // int4 weights): y [M, rows] = x [M, cols] . W^T

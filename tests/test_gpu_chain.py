@@ -47,3 +47,46 @@ def test_batched_prefill_on_matrix_cores_equals_steps_bitwise(ctx, hip, scheme, 
     cache.destroy()
     steps.destroy()
     model.destroy()
+
+
+@pytest.mark.parametrize("fmt", ["f16", "int8", "int4"])
+@pytest.mark.parametrize("rows,cols,group", [
+    (1, 128, 128),          # one row: a tile of clamped rows
+    (17, 896, 128),         # one row past a tile; 56 / 28 / 112 chunks
+    (128, 4864, 128),       # several chunks per lane, a ragged last pass
+    (70, 1184, 32),         # chunks off the slabs
+])
+def test_exact_matvec_on_matrix_cores_equals_single_positions_bitwise(ctx, hip, fmt, rows, cols, group):
+    """qh_matvec from 8 positions runs on the f64 matrix cores: each position's outputs are those
+    of the one-position call, bit for bit (int4 zero points off the quantizer's integers too)."""
+    rng = np.random.default_rng(rows + cols)
+    w = (rng.standard_normal((rows, cols)) * 0.02).astype(np.float32)
+    if fmt == "f16":
+        bufs = [ctx.upload(w.astype(np.float16).view(np.uint16))]
+        W = ctx.weight(hip.FMT_F16, rows, cols, bufs[0])
+    elif fmt == "int8":
+        q, s = hip.quantize_int8(w)
+        q[0, :3] = -128
+        bufs = [ctx.upload(q), ctx.upload(s)]
+        W = ctx.weight(hip.FMT_INT8, rows, cols, *bufs)
+    else:
+        q, s, z = hip.quantize_int4(w, group)
+        z[0, 0] = 3.5
+        bufs = [ctx.upload(q), ctx.upload(s), ctx.upload(z)]
+        W = ctx.weight(hip.FMT_INT4, rows, cols, *bufs, group)
+    bias = ctx.upload(rng.standard_normal(rows).astype(np.float32))
+    x = rng.standard_normal((49, cols)).astype(np.float32)
+    dy = ctx.empty(49 * rows * 4)
+    want = np.empty((49, rows), np.float32)
+    for t in range(49):
+        dx = ctx.upload(x[t])
+        ctx.matvec(W, dx, bias, dy, 1)
+        want[t] = dy.read(count=rows)
+        dx.free()
+    dx = ctx.upload(x)
+    for seq in (8, 16, 17, 32, 33, 49):
+        ctx.matvec(W, dx, bias, dy, seq)
+        np.testing.assert_array_equal(dy.read(count=seq * rows).view(np.uint32), want[:seq].reshape(-1).view(np.uint32),
+                                      err_msg=f"{seq} positions")
+    for b in bufs + [bias, dx, dy]:
+        b.free()
