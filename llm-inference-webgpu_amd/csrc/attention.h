@@ -269,6 +269,139 @@ static __global__ __launch_bounds__(kAttnThreads) void k_attn_block(ExactArgs a)
   if (tid < kHeadDim) a.out[((size_t)t * a.heads + h) * kHeadDim + tid] = o;
 }
 
+// -------------------------------------------- exact order, a tile of queries --
+// The same evaluation for a (head, 16 queries) tile of a prompt, with both products on the matrix
+// cores: v_mfma_f64_16x16x4f64 and v_mfma_f32_16x16x4f32 evaluate their four k as ascending fused
+// multiply-adds, each rounded to nearest even, so the f64 dots over i and the f32 sums over
+// positions are the chains k_attn_block evaluates, bit for bit; the softmax keeps its thread
+// order (position p on thread p % 512 of 8 waves). Keys past the tile's first query, which some
+// queries do not see, are summed on the vector unit under each query's own bound.
+//
+// Bound: latency of its three phases (f64 products, f64 exponentials, then a chain of ctx / 4
+// products per 16 dimensions); a tile takes 16 x CTX scores of LDS, so several tiles share a CU,
+// where k_attn_block's one wave summed alone on a CU per (query, head). Tiles are launched
+// heaviest first. 512 queries, 14 heads: 182 -> X us.
+typedef double f64x4 __attribute__((ext_vector_type(4)));
+typedef float f32x4t __attribute__((ext_vector_type(4)));
+constexpr int kTileQ = 16;
+constexpr int kTileThreads = 512, kTileWaves = kTileThreads / kWave;
+static_assert(kTileThreads == kAttnThreads, "the softmax sum's thread order");
+constexpr int kTileCtx = 2048;     // the widest tile: 16 x 2052 floats of LDS
+constexpr int kTileMinSeq = 16;
+
+// Element 4s + g of 16 f16 values (s = 0..3) in two 16-byte words.
+__device__ __forceinline__ float tile_f16(const v4u (&u)[2], int s, int g) {
+  const uint64_t pair = ((uint64_t)u[s >> 1][2 * (s & 1) + 1] << 32) | u[s >> 1][2 * (s & 1)];
+  return f16_lo((uint32_t)(pair >> (16 * g)));
+}
+// Where score p of a row sits: each 16 as [p % 4][p / 4 % 4], so a lane's four k are one read.
+__device__ __forceinline__ int tile_at(int p) { return (p & ~15) | ((p & 3) << 2) | ((p >> 2) & 3); }
+
+template <int CTX>
+static __global__ __launch_bounds__(kTileThreads) void k_attn_tile(ExactArgs a, int seq) {
+  __shared__ __attribute__((aligned(16))) float sc[kTileQ][CTX + 4];
+  const int tid = threadIdx.x, lane = tid & (kWave - 1), w = tid / kWave, n = lane & 15, g = lane >> 4;
+  const int tiles = (seq + kTileQ - 1) / kTileQ;
+  const int h = blockIdx.x % a.heads, t0 = (tiles - 1 - blockIdx.x / a.heads) * kTileQ;
+  const int kvh = h / (a.heads / a.kv_heads);
+  const int kmax = a.past + min(t0 + kTileQ - 1, seq - 1);  // the tile's last key
+  if (kmax >= CTX || kmax >= a.capacity) return;            // the host keeps positions inside both
+  const uint16_t* kb = a.kc + (size_t)kvh * a.capacity * kHeadDim;
+  const uint16_t* vb = a.vt + (size_t)kvh * kHeadDim * a.vstride;
+
+  // Scores: key tiles w, w + 8, ..; accumulator register r holds query 4r + g, key n.
+  {
+    const float* q = a.q + ((size_t)min(t0 + n, seq - 1) * a.heads + h) * kHeadDim + g;
+    double qd[16];
+#pragma unroll
+    for (int s = 0; s < 16; s++) qd[s] = (double)q[4 * s];
+    auto load = [&](int kt, v4u (&k)[4][2]) {
+      const v4u* kr = reinterpret_cast<const v4u*>(kb + (size_t)min(16 * kt + n, kmax) * kHeadDim);
+#pragma unroll
+      for (int j = 0; j < 8; j++) k[j >> 1][j & 1] = kr[j];
+    };
+    v4u k[4][2], nk[4][2];
+    if (16 * w <= kmax) load(w, k);
+    for (int kt = w; 16 * kt <= kmax; kt += kTileWaves) {
+      load(kt + kTileWaves, nk);
+      f64x4 acc = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+      for (int s = 0; s < 16; s++)
+        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(qd[s], (double)tile_f16(k[s >> 2], s & 3, g), acc, 0, 0, 0);
+#pragma unroll
+      for (int r = 0; r < 4; r++) sc[4 * r + g][tile_at(16 * kt + n)] = (float)(acc[r] * 0.125);
+#pragma unroll
+      for (int j = 0; j < 8; j++) k[j >> 1][j & 1] = nk[j >> 1][j & 1];
+    }
+  }
+  __syncthreads();
+  // Softmax: wave w takes queries 2w and 2w + 1, lane l the positions of threads l, 64 + l, ..
+  for (int i = 0; i < 2; i++) {
+    const int qi = 2 * w + i;
+    if (t0 + qi >= seq) break;
+    const int ctx = a.past + t0 + qi + 1;
+    float* row = sc[qi];
+    float m = -INFINITY;
+    for (int p = lane; p < ctx; p += kWave) m = fmaxf(m, row[tile_at(p)]);
+    const double M = wave_max(m);
+    double sum = 0.0;
+    for (int v = 0; v < kTileWaves && v * kWave < ctx; v++) {
+      double part = 0.0;
+      for (int p = v * kWave + lane; p < ctx; p += kTileThreads) {
+        const double e = exp((double)row[tile_at(p)] - M);
+        row[tile_at(p)] = (float)e;
+        part += e;
+      }
+      sum += team_sum<64>(part);
+    }
+    const double inv = 1.0 / sum;
+    for (int p = lane; p < ctx; p += kWave) row[tile_at(p)] = (float)((double)row[tile_at(p)] * inv);
+  }
+  __syncthreads();
+  if (w >= 4) return;
+  // PV: wave w sums dimensions 16w .. +15 over the positions; register r holds query 4g + r.
+  const uint16_t* vr = vb + (size_t)(16 * w + n) * a.vstride;
+  const int full = (a.past + t0 + 1) >> 4;  // whole 16-position groups every query sees
+  f32x4t o = {0.f, 0.f, 0.f, 0.f};
+  constexpr int kAhead = 4;  // groups whose values are loaded together
+  v4u va[kAhead][2], vn[kAhead][2];
+  auto load = [&](int j0, v4u (&d)[kAhead][2]) {
+#pragma unroll
+    for (int j = 0; j < kAhead; j++) {
+      const v4u* src = reinterpret_cast<const v4u*>(vr + 16 * min(j0 + j, full - 1));
+      d[j][0] = src[0];
+      d[j][1] = src[1];
+    }
+  };
+  if (full > 0) load(0, va);
+  for (int j0 = 0; j0 < full; j0 += kAhead) {
+    if (j0 + kAhead < full) load(j0 + kAhead, vn);
+#pragma unroll
+    for (int j = 0; j < kAhead; j++) {
+      if (j0 + j < full) {
+        const v4f p = *reinterpret_cast<const v4f*>(&sc[n][16 * (j0 + j) + 4 * g]);
+#pragma unroll
+        for (int s = 0; s < 4; s++)
+          o = __builtin_amdgcn_mfma_f32_16x16x4f32(p[s], tile_f16(va[j], s, g), o, 0, 0, 0);
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < kAhead; j++) {
+      va[j][0] = vn[j][0];
+      va[j][1] = vn[j][1];
+    }
+  }
+  for (int p = 16 * full; p <= kmax; p++) {
+    const float v = (float)__builtin_bit_cast(_Float16, vr[p]);
+#pragma unroll
+    for (int r = 0; r < 4; r++)
+      if (p <= a.past + t0 + 4 * g + r) o[r] = fmaf(sc[4 * g + r][tile_at(p)], v, o[r]);
+  }
+#pragma unroll
+  for (int r = 0; r < 4; r++)
+    if (t0 + 4 * g + r < seq) a.out[((size_t)(t0 + 4 * g + r) * a.heads + h) * kHeadDim + 16 * w + n] = o[r];
+}
+
 // grid (spans, heads, seq). Block (span, h, t) scores positions span*256 ..
 // +255 of query t against head h and records the span's maximum; the last span
 // block of (t, h) to finish computes the probabilities and the output.
@@ -370,6 +503,25 @@ static __global__ __launch_bounds__(kBlock) void k_attn_exact(ExactArgs a) {
   }
   if (tid < kHeadDim) a.out[row * kHeadDim + tid] = o;
   if (tid == 0) a.counters[row] = 0;
+}
+
+// Exact attention of `seq` queries over past + seq positions: query tiles for prompts that fit
+// them, else a (query, head) block up to kPLds positions -- of context for the operator, of
+// capacity for the model (`limit`), whose decode step picks by capacity -- else spans. All
+// evaluate a query alike.
+static inline hipError_t launch_attn_exact(hipStream_t s, const ExactArgs& a, int seq, int limit, int spans) {
+  const int total = a.past + seq;
+  if (seq >= kTileMinSeq && total <= kTileCtx && limit <= kPLds) {
+    const dim3 grid((seq + kTileQ - 1) / kTileQ * a.heads), block(kTileThreads);
+    if (total <= 512) hipLaunchKernelGGL(k_attn_tile<512>, grid, block, 0, s, a, seq);
+    else if (total <= 1024) hipLaunchKernelGGL(k_attn_tile<1024>, grid, block, 0, s, a, seq);
+    else hipLaunchKernelGGL(k_attn_tile<kTileCtx>, grid, block, 0, s, a, seq);
+  } else if (limit <= kPLds) {
+    hipLaunchKernelGGL(k_attn_block, dim3(a.heads, seq), dim3(kAttnThreads), 0, s, a);
+  } else {
+    hipLaunchKernelGGL(k_attn_exact, dim3(spans, a.heads, seq), dim3(kBlock), 0, s, a);
+  }
+  return hipGetLastError();
 }
 
 // -------------------------------------------------------------- split-K --

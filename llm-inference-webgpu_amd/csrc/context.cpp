@@ -453,6 +453,11 @@ int qh_attention(qh_ctx* ctx, const float* d_q, const uint16_t* d_key_cache,
   // Scores and span maxima in the context scratch's partial region, counters in its counter
   // region (after the argmax counter), when they fit; else a temporary buffer.
   const size_t floats = qh::attention_exact_floats(seq, heads, past);
+  if (!floats) {
+    QH_HIP(qh::launch_attention_exact(ctx->stream, d_q, d_key_cache, d_value_cache, capacity, d_out, seq, past,
+                                      heads, kv_heads, nullptr, nullptr));
+    return QH_OK;
+  }
   const size_t room = ctx->scratch_bytes - qh_ctx::kScratchCounterBytes - 64;
   const size_t n_counters = (size_t)seq * heads;
   if ((n_counters + 16) * sizeof(int) <= qh_ctx::kScratchCounterBytes && floats * sizeof(float) <= room) {

@@ -369,12 +369,8 @@ hipError_t enqueue_prefill_layers(hipStream_t s, const ModelDev& m, const CacheD
       a.vstride = c.vstride;
       a.heads = m.heads;
       a.kv_heads = m.kv_heads;
-      // the kernel the decode step picks for this cache (the same arithmetic per query)
-      if (c.capacity <= kPLds) {
-        hipLaunchKernelGGL(k_attn_block, dim3(m.heads, seq), dim3(kAttnThreads), 0, s, a);
-      } else {
-        hipLaunchKernelGGL(k_attn_exact, dim3(attn_spans(c.capacity), m.heads, seq), dim3(kBlock), 0, s, a);
-      }
+      // the arithmetic of the kernel the decode step picks for this cache
+      if ((e = launch_attn_exact(s, a, seq, c.capacity, attn_spans(c.capacity))) != hipSuccess) return e;
     }
     if ((e = hipGetLastError()) != hipSuccess) return e;
     if ((e = matmul(s, m, mode, l.o, p.ATT, nullptr, p.Y, seq, p)) != hipSuccess) return e;

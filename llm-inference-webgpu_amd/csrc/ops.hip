@@ -449,6 +449,7 @@ static int score_stride(int total) { return (total + 3) & ~3; }
 
 size_t attention_exact_floats(int seq, int heads, int past) {
   const int total = past + seq;
+  if (total <= kPLds) return 0;  // scores stay in LDS
   return (size_t)seq * heads * (score_stride(total) + attn_spans(total));
 }
 
@@ -471,12 +472,7 @@ hipError_t launch_attention_exact(hipStream_t s, const float* q, const uint16_t*
   a.vstride = value_stride(capacity);
   a.heads = heads;
   a.kv_heads = kv_heads;
-  if (total <= kPLds) {
-    hipLaunchKernelGGL(k_attn_block, dim3(heads, seq), dim3(kAttnThreads), 0, s, a);
-  } else {
-    hipLaunchKernelGGL(k_attn_exact, dim3(a.max_stride, heads, seq), dim3(kBlock), 0, s, a);
-  }
-  return hipGetLastError();
+  return launch_attn_exact(s, a, seq, total, a.max_stride);
 }
 
 // Queries per launch of a long cache's 128 slots: their partials (476 KiB per query at 14

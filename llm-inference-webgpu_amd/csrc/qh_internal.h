@@ -156,7 +156,7 @@ hipError_t launch_kv_append(hipStream_t s, const float* k, const float* v, uint1
                             int seq);
 // Exact-order attention. `scores` holds attention_exact_floats(seq, heads, past) floats
 // (scores, then per-span maxima) and `counters` seq*heads ints, zero before the launch and
-// left zero after it.
+// left zero after it; neither is used where that is 0.
 hipError_t launch_attention_exact(hipStream_t s, const float* q, const uint16_t* kc,
                                   const uint16_t* vt, int capacity, float* out, int seq, int past,
                                   int heads, int kv_heads, float* scores, int* counters);
