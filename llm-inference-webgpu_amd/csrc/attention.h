@@ -297,9 +297,20 @@ __device__ __forceinline__ float tile_f16(const v4u (&u)[2], int s, int g) {
 // Where score p of a row sits: each 16 as [p % 4][p / 4 % 4], so a lane's four k are one read.
 __device__ __forceinline__ int tile_at(int p) { return (p & ~15) | ((p & 3) << 2) | ((p >> 2) & 3); }
 
+__device__ __forceinline__ float wave_max_dpp(float v) {
+  v = fmaxf(v, dpp32<kDppQuadXor1>(v));
+  v = fmaxf(v, dpp32<kDppQuadXor2>(v));
+  v = fmaxf(v, dpp32<kDppHalfMirror>(v));
+  v = fmaxf(v, dpp32<kDppMirror>(v));
+  v = fmaxf(v, swz_xor16(v));
+  return fmaxf(v, __shfl_xor(v, 32));
+}
+
 template <int CTX>
 static __global__ __launch_bounds__(kTileThreads) void k_attn_tile(ExactArgs a, int seq) {
   __shared__ __attribute__((aligned(16))) float sc[kTileQ][CTX + 4];
+  static_assert(CTX % kTileThreads == 0, "the softmax reads whole threads' positions");
+  __shared__ __attribute__((aligned(16))) uint16_t ks[kTileWaves][16][kHeadDim + 8];  // padded over the banks
   const int tid = threadIdx.x, lane = tid & (kWave - 1), w = tid / kWave, n = lane & 15, g = lane >> 4;
   const int tiles = (seq + kTileQ - 1) / kTileQ;
   const int h = blockIdx.x % a.heads, t0 = (tiles - 1 - blockIdx.x / a.heads) * kTileQ;
@@ -309,93 +320,197 @@ static __global__ __launch_bounds__(kTileThreads) void k_attn_tile(ExactArgs a, 
   const uint16_t* kb = a.kc + (size_t)kvh * a.capacity * kHeadDim;
   const uint16_t* vb = a.vt + (size_t)kvh * kHeadDim * a.vstride;
 
-  // Scores: key tiles w, w + 8, ..; accumulator register r holds query 4r + g, key n.
+  // Scores: key tiles w, w + 8, ..; accumulator register r holds query 4r + g, key n. A wave
+  // loads its tile's key rows once (a lane a quarter row, the next two tiles' in flight) and
+  // passes them through its own LDS to the lanes' elements 4s + g.
   {
     const float* q = a.q + ((size_t)min(t0 + n, seq - 1) * a.heads + h) * kHeadDim + g;
     double qd[16];
+    v4u k[3][2];
+    auto load = [&](int kt, v4u (&d)[2]) {
+      const v4u* kr = reinterpret_cast<const v4u*>(kb + (size_t)min(16 * kt + n, kmax) * kHeadDim) + 2 * g;
+      d[0] = kr[0];
+      d[1] = kr[1];
+    };
+    load(w, k[0]);
+    load(w + kTileWaves, k[1]);
 #pragma unroll
     for (int s = 0; s < 16; s++) qd[s] = (double)q[4 * s];
-    auto load = [&](int kt, v4u (&k)[4][2]) {
-      const v4u* kr = reinterpret_cast<const v4u*>(kb + (size_t)min(16 * kt + n, kmax) * kHeadDim);
+    auto tile = [&](int kt, const v4u (&d)[2]) {
+      v4u* dst = reinterpret_cast<v4u*>(&ks[w][n][16 * g]);
+      dst[0] = d[0];
+      dst[1] = d[1];
+      __builtin_amdgcn_wave_barrier();  // the wave's LDS operations run in order
+      _Float16 e[16];
 #pragma unroll
-      for (int j = 0; j < 8; j++) k[j >> 1][j & 1] = kr[j];
-    };
-    v4u k[4][2], nk[4][2];
-    if (16 * w <= kmax) load(w, k);
-    for (int kt = w; 16 * kt <= kmax; kt += kTileWaves) {
-      load(kt + kTileWaves, nk);
+      for (int s = 0; s < 16; s++) e[s] = __builtin_bit_cast(_Float16, ks[w][n][4 * s + g]);
+      __builtin_amdgcn_wave_barrier();
       f64x4 acc = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
       for (int s = 0; s < 16; s++)
-        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(qd[s], (double)tile_f16(k[s >> 2], s & 3, g), acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(qd[s], (double)(float)e[s], acc, 0, 0, 0);
 #pragma unroll
       for (int r = 0; r < 4; r++) sc[4 * r + g][tile_at(16 * kt + n)] = (float)(acc[r] * 0.125);
-#pragma unroll
-      for (int j = 0; j < 8; j++) k[j >> 1][j & 1] = nk[j >> 1][j & 1];
+    };
+    for (int kt = w; 16 * kt <= kmax; kt += 3 * kTileWaves) {
+      load(kt + 2 * kTileWaves, k[2]);
+      tile(kt, k[0]);
+      if (16 * (kt + kTileWaves) > kmax) break;
+      load(kt + 3 * kTileWaves, k[0]);
+      tile(kt + kTileWaves, k[1]);
+      if (16 * (kt + 2 * kTileWaves) > kmax) break;
+      load(kt + 4 * kTileWaves, k[1]);
+      tile(kt + 2 * kTileWaves, k[2]);
     }
   }
   __syncthreads();
-  // Softmax: wave w takes queries 2w and 2w + 1, lane l the positions of threads l, 64 + l, ..
-  for (int i = 0; i < 2; i++) {
-    const int qi = 2 * w + i;
-    if (t0 + qi >= seq) break;
-    const int ctx = a.past + t0 + qi + 1;
-    float* row = sc[qi];
-    float m = -INFINITY;
-    for (int p = lane; p < ctx; p += kWave) m = fmaxf(m, row[tile_at(p)]);
-    const double M = wave_max(m);
-    double sum = 0.0;
-    for (int v = 0; v < kTileWaves && v * kWave < ctx; v++) {
-      double part = 0.0;
-      for (int p = v * kWave + lane; p < ctx; p += kTileThreads) {
-        const double e = exp((double)row[tile_at(p)] - M);
-        row[tile_at(p)] = (float)e;
-        part += e;
-      }
-      sum += team_sum<64>(part);
-    }
-    const double inv = 1.0 / sum;
-    for (int p = lane; p < ctx; p += kWave) row[tile_at(p)] = (float)((double)row[tile_at(p)] * inv);
-  }
-  __syncthreads();
-  if (w >= 4) return;
-  // PV: wave w sums dimensions 16w .. +15 over the positions; register r holds query 4g + r.
-  const uint16_t* vr = vb + (size_t)(16 * w + n) * a.vstride;
+  // PV's first values load while the softmax runs (waves 0-3, 16 dimensions each).
+  const uint16_t* vr = vb + (size_t)(16 * (w & 3) + n) * a.vstride;
   const int full = (a.past + t0 + 1) >> 4;  // whole 16-position groups every query sees
-  f32x4t o = {0.f, 0.f, 0.f, 0.f};
-  constexpr int kAhead = 4;  // groups whose values are loaded together
-  v4u va[kAhead][2], vn[kAhead][2];
+  const int lastg = (a.vstride >> 4) - 1;
+  constexpr int kAhead = 4;                 // groups whose values are loaded together
+  v4u vv[3][kAhead][2];                     // three such batches: two in flight under one's products
   auto load = [&](int j0, v4u (&d)[kAhead][2]) {
 #pragma unroll
     for (int j = 0; j < kAhead; j++) {
-      const v4u* src = reinterpret_cast<const v4u*>(vr + 16 * min(j0 + j, full - 1));
+      const v4u* src = reinterpret_cast<const v4u*>(vr + 16 * min(j0 + j, lastg));
       d[j][0] = src[0];
       d[j][1] = src[1];
     }
   };
-  if (full > 0) load(0, va);
-  for (int j0 = 0; j0 < full; j0 += kAhead) {
-    if (j0 + kAhead < full) load(j0 + kAhead, vn);
+  // Softmax: wave w takes queries 2w and 2w + 1 together, lane l the positions of threads l,
+  // 64 + l, ..; two threads' worth of each query at a time, so exponentials and butterflies
+  // overlap. (A query past the end is a copy of the last.)
+  {
+    int ctx[2];
+    float* row[2];
+    double M[2], sum[2] = {0.0, 0.0}, inv[2];
 #pragma unroll
-    for (int j = 0; j < kAhead; j++) {
-      if (j0 + j < full) {
-        const v4f p = *reinterpret_cast<const v4f*>(&sc[n][16 * (j0 + j) + 4 * g]);
+    for (int i = 0; i < 2; i++) {
+      ctx[i] = a.past + min(t0 + 2 * w + i, seq - 1) + 1;
+      row[i] = sc[2 * w + i];
+    }
+    float m[2] = {-INFINITY, -INFINITY};
+    for (int p0 = 0; p0 < ctx[1]; p0 += 4 * kWave) {
+      float v[2][4];
 #pragma unroll
-        for (int s = 0; s < 4; s++)
-          o = __builtin_amdgcn_mfma_f32_16x16x4f32(p[s], tile_f16(va[j], s, g), o, 0, 0, 0);
-      }
+      for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int u = 0; u < 4; u++) v[i][u] = row[i][tile_at(p0 + u * kWave + lane)];
+#pragma unroll
+      for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+          if (p0 + u * kWave + lane < ctx[i]) m[i] = fmaxf(m[i], v[i][u]);
     }
 #pragma unroll
-    for (int j = 0; j < kAhead; j++) {
-      va[j][0] = vn[j][0];
-      va[j][1] = vn[j][1];
+    for (int i = 0; i < 2; i++) M[i] = wave_max_dpp(m[i]);
+    for (int v0 = 0; v0 < kTileWaves && v0 * kWave < ctx[1]; v0 += 2) {
+      double part[2][2] = {};
+      for (int p0 = v0 * kWave; p0 < ctx[1]; p0 += kTileThreads) {
+        double e[2][2];
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+#pragma unroll
+          for (int u = 0; u < 2; u++) e[i][u] = exp((double)row[i][tile_at(p0 + u * kWave + lane)] - M[i]);
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+#pragma unroll
+          for (int u = 0; u < 2; u++) {
+            const int p = p0 + u * kWave + lane;
+            if (p < ctx[i]) {
+              row[i][tile_at(p)] = (float)e[i][u];
+              part[i][u] += e[i][u];
+            }
+          }
+      }
+#pragma unroll
+      for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int u = 0; u < 2; u++) part[i][u] = team_sum<64>(part[i][u]);
+#pragma unroll
+      for (int i = 0; i < 2; i++) sum[i] = (sum[i] + part[i][0]) + part[i][1];
+    }
+#pragma unroll
+    for (int i = 0; i < 2; i++) inv[i] = 1.0 / sum[i];
+    for (int p0 = 0; p0 < ctx[1]; p0 += 4 * kWave) {
+      float v[2][4];
+#pragma unroll
+      for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int u = 0; u < 4; u++) v[i][u] = row[i][tile_at(p0 + u * kWave + lane)];
+#pragma unroll
+      for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+          if (p0 + u * kWave + lane < ctx[i])
+            row[i][tile_at(p0 + u * kWave + lane)] = (float)((double)v[i][u] * inv[i]);
     }
   }
-  for (int p = 16 * full; p <= kmax; p++) {
-    const float v = (float)__builtin_bit_cast(_Float16, vr[p]);
+  v4u tv[2][2];  // the tile's last groups, which not every query sees whole
+  if (w < 4) {
+    load(0, vv[0]);
+    load(kAhead, vv[1]);
 #pragma unroll
-    for (int r = 0; r < 4; r++)
-      if (p <= a.past + t0 + 4 * g + r) o[r] = fmaf(sc[4 * g + r][tile_at(p)], v, o[r]);
+    for (int j = 0; j < 2; j++) {
+      const v4u* src = reinterpret_cast<const v4u*>(vr + 16 * min(full + j, lastg));
+      tv[j][0] = src[0];
+      tv[j][1] = src[1];
+    }
+  }
+  __syncthreads();
+  if (w >= 4) return;
+  // PV: wave w sums dimensions 16w .. +15 over the positions; register r holds query 4g + r.
+  f32x4t o = {0.f, 0.f, 0.f, 0.f};
+  auto group = [&](int j, const v4u (&d)[2], const v4f p) {
+#pragma unroll
+    for (int s = 0; s < 4; s++) o = __builtin_amdgcn_mfma_f32_16x16x4f32(p[s], tile_f16(d, s, g), o, 0, 0, 0);
+  };
+  auto batch = [&](int j0, const v4u (&d)[kAhead][2]) {
+    v4f p[kAhead];
+#pragma unroll
+    for (int j = 0; j < kAhead; j++) p[j] = *reinterpret_cast<const v4f*>(&sc[n][16 * min(j0 + j, CTX / 16 - 1) + 4 * g]);
+    if (j0 + kAhead <= full) {
+#pragma unroll
+      for (int j = 0; j < kAhead; j++) group(j0 + j, d[j], p[j]);
+    } else {
+#pragma unroll
+      for (int j = 0; j < kAhead; j++)
+        if (j0 + j < full) group(j0 + j, d[j], p[j]);
+    }
+  };
+  for (int j0 = 0; j0 < full; j0 += 3 * kAhead) {
+    load(j0 + 2 * kAhead, vv[2]);
+    batch(j0, vv[0]);
+    load(j0 + 3 * kAhead, vv[0]);
+    batch(j0 + kAhead, vv[1]);
+    load(j0 + 4 * kAhead, vv[1]);
+    batch(j0 + 2 * kAhead, vv[2]);
+  }
+#pragma unroll
+  for (int j = 0; j < 2; j++) {
+    const int p0 = 16 * (full + j);
+    if (p0 <= kmax) {  // uniform
+#pragma unroll
+      for (int e4 = 0; e4 < 4; e4++) {  // positions p0 + 4 e4 .. +3
+        v4f pr[4];
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+#pragma unroll
+          for (int r = 0; r < 4; r++) pr[r][e] = sc[4 * g + r][tile_at(p0 + 4 * e4 + e)];
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          const int k = 4 * e4 + e;
+          const uint32_t d = tv[j][k >> 3][(k >> 1) & 3];
+          const float v = (k & 1) ? f16_hi(d) : f16_lo(d);
+#pragma unroll
+          for (int r = 0; r < 4; r++) {
+            const float x = fmaf(pr[r][e], v, o[r]);
+            o[r] = p0 + k <= a.past + t0 + 4 * g + r && p0 + k <= kmax ? x : o[r];
+          }
+        }
+      }
+    }
   }
 #pragma unroll
   for (int r = 0; r < 4; r++)
