@@ -352,6 +352,7 @@ static __global__ __launch_bounds__(kTileThreads) void k_attn_tile(ExactArgs a, 
 #pragma unroll
       for (int r = 0; r < 4; r++) sc[4 * r + g][tile_at(16 * kt + n)] = (float)(acc[r] * 0.125);
     };
+#pragma unroll 1
     for (int kt = w; 16 * kt <= kmax; kt += 3 * kTileWaves) {
       load(kt + 2 * kTileWaves, k[2]);
       tile(kt, k[0]);
@@ -391,6 +392,7 @@ static __global__ __launch_bounds__(kTileThreads) void k_attn_tile(ExactArgs a, 
       row[i] = sc[2 * w + i];
     }
     float m[2] = {-INFINITY, -INFINITY};
+#pragma unroll 1
     for (int p0 = 0; p0 < ctx[1]; p0 += 4 * kWave) {
       float v[2][4];
 #pragma unroll
@@ -405,8 +407,10 @@ static __global__ __launch_bounds__(kTileThreads) void k_attn_tile(ExactArgs a, 
     }
 #pragma unroll
     for (int i = 0; i < 2; i++) M[i] = wave_max_dpp(m[i]);
+#pragma unroll 1
     for (int v0 = 0; v0 < kTileWaves && v0 * kWave < ctx[1]; v0 += 2) {
       double part[2][2] = {};
+#pragma unroll 1
       for (int p0 = v0 * kWave; p0 < ctx[1]; p0 += kTileThreads) {
         double e[2][2];
 #pragma unroll
@@ -433,6 +437,7 @@ static __global__ __launch_bounds__(kTileThreads) void k_attn_tile(ExactArgs a, 
     }
 #pragma unroll
     for (int i = 0; i < 2; i++) inv[i] = 1.0 / sum[i];
+#pragma unroll 1
     for (int p0 = 0; p0 < ctx[1]; p0 += 4 * kWave) {
       float v[2][4];
 #pragma unroll
@@ -470,15 +475,11 @@ static __global__ __launch_bounds__(kTileThreads) void k_attn_tile(ExactArgs a, 
     v4f p[kAhead];
 #pragma unroll
     for (int j = 0; j < kAhead; j++) p[j] = *reinterpret_cast<const v4f*>(&sc[n][16 * min(j0 + j, CTX / 16 - 1) + 4 * g]);
-    if (j0 + kAhead <= full) {
 #pragma unroll
-      for (int j = 0; j < kAhead; j++) group(j0 + j, d[j], p[j]);
-    } else {
-#pragma unroll
-      for (int j = 0; j < kAhead; j++)
-        if (j0 + j < full) group(j0 + j, d[j], p[j]);
-    }
+    for (int j = 0; j < kAhead; j++)
+      if (j0 + j < full) group(j0 + j, d[j], p[j]);  // uniform
   };
+#pragma unroll 1
   for (int j0 = 0; j0 < full; j0 += 3 * kAhead) {
     load(j0 + 2 * kAhead, vv[2]);
     batch(j0, vv[0]);
@@ -487,26 +488,23 @@ static __global__ __launch_bounds__(kTileThreads) void k_attn_tile(ExactArgs a, 
     load(j0 + 4 * kAhead, vv[1]);
     batch(j0 + 2 * kAhead, vv[2]);
   }
+  // The last groups: positions two at a time (a dword of values), each under its query's bound.
 #pragma unroll
   for (int j = 0; j < 2; j++) {
     const int p0 = 16 * (full + j);
     if (p0 <= kmax) {  // uniform
 #pragma unroll
-      for (int e4 = 0; e4 < 4; e4++) {  // positions p0 + 4 e4 .. +3
-        v4f pr[4];
-#pragma unroll
-        for (int e = 0; e < 4; e++)
-#pragma unroll
-          for (int r = 0; r < 4; r++) pr[r][e] = sc[4 * g + r][tile_at(p0 + 4 * e4 + e)];
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-          const int k = 4 * e4 + e;
-          const uint32_t d = tv[j][k >> 3][(k >> 1) & 3];
-          const float v = (k & 1) ? f16_hi(d) : f16_lo(d);
+      for (int k = 0; k < 8; k++) {
+        const uint32_t d = tv[j][k >> 2][k & 3];
+        const int p = p0 + 2 * k;
+        if (p <= kmax) {  // uniform
 #pragma unroll
           for (int r = 0; r < 4; r++) {
-            const float x = fmaf(pr[r][e], v, o[r]);
-            o[r] = p0 + k <= a.past + t0 + 4 * g + r && p0 + k <= kmax ? x : o[r];
+            const int last = min(a.past + t0 + 4 * g + r, kmax);
+            const float x = fmaf(sc[4 * g + r][tile_at(p)], f16_lo(d), o[r]);
+            o[r] = p <= last ? x : o[r];
+            const float y = fmaf(sc[4 * g + r][tile_at(p + 1)], f16_hi(d), o[r]);
+            o[r] = p + 1 <= last ? y : o[r];
           }
         }
       }
