@@ -144,6 +144,7 @@ __device__ __forceinline__ float take_min(float best, float v) { return v < best
 // round(t), half away from zero, as an int for |t| < 2^31: the integer part and the exact
 // remainder t - trunc(t) decide it.
 __device__ __forceinline__ int round_away(double t) {
+#pragma clang fp contract(off)
   const int i = (int)t;
   const double f = t - (double)i;
   return i + (f >= 0.5 ? 1 : 0) - (f <= -0.5 ? 1 : 0);
@@ -154,12 +155,16 @@ __device__ __forceinline__ int round_away(double t) {
 // |t| <= 15 (1 + 2^-51) for int4 (an infinite x makes the scale infinite, the inverse 0 and t
 // NaN). So round(t) fits an int, the clamps are integer clamps, and NaN -- of t, or of an int4
 // zero point, which is otherwise an integer in [0, 15] -- is the typed-array store's 0.
+// The product is rounded on its own: fused into the remainder's subtraction, a product that
+// rounds to a half-integer would be judged by its unrounded value.
 __device__ __forceinline__ int code_int8(float x, double inverse) {
+#pragma clang fp contract(off)
   const double t = (double)x * inverse;
   if (t != t) return 0;
   return min(max(round_away(t), -127), 127);
 }
 __device__ __forceinline__ uint32_t code_int4(float x, double inverse, double zero) {
+#pragma clang fp contract(off)
   const double t = (double)x * inverse;
   if (t != t || zero != zero) return 0;
   return (uint32_t)min(max(round_away(t) + (int)zero, 0), 15);
@@ -169,24 +174,129 @@ __device__ __forceinline__ uint32_t code_int4(float x, double inverse, double ze
 // the f64 product t the expressions above round by at most |t| 2^-23 (the two roundings to f32,
 // 2^-24 each relative; f32(inverse) is never subnormal: |x| < 2^128 bounds the scale), and
 // |t| <= 16 (int4) or 128 (int8). So wherever t32 lies farther than kSafe from every
-// half-integer, t rounds half away from zero to the integer nearest t32; nearer a half-integer,
-// and for NaN or an infinite t32, the f64 expression decides. The codes are those of the f64
-// expressions bit for bit, at a fraction of their arithmetic.
+// half-integer, t rounds half away from zero to the integer nearest t32; where some value of a
+// chunk lies nearer a half-integer, or is NaN or infinite, the f64 expression decides the whole
+// chunk. The codes are those of the f64 expressions bit for bit, at a fraction of their arithmetic
+// and without a branch per value: a chunk costs one test (int4 of 233472 x 896 bf16 values
+// 173 -> 145 us with the packed ranges and the shared parameters
+// below, still bound by the vector unit: ~25 instructions a value before, ~13 now).
 constexpr float kSafeInt4 = 0x1p-16f;  // > 16 * 2^-23
 constexpr float kSafeInt8 = 0x1p-13f;  // > 128 * 2^-23
-__device__ __forceinline__ int code_int8_f32(float x, float inv32, double inverse) {
+// The nearest integer to x * inv32, and whether t32 is too near a half-integer (or NaN).
+__device__ __forceinline__ float nearest(float x, float inv32, float safe, bool& unsafe) {
 #pragma clang fp contract(off)
   const float t = x * inv32;
   const float r = __builtin_rintf(t);
-  if (!(fabsf(t - r) <= 0.5f - kSafeInt8)) return code_int8(x, inverse);
-  return (int)fminf(fmaxf(r, -127.f), 127.f);
+  unsafe |= !(fabsf(t - r) <= 0.5f - safe);
+  return r;
 }
-__device__ __forceinline__ uint32_t code_int4_f32(float x, float inv32, double inverse, double zero, float zf) {
-#pragma clang fp contract(off)
-  const float t = x * inv32;
-  const float r = __builtin_rintf(t);
-  if (!(fabsf(t - r) <= 0.5f - kSafeInt4)) return code_int4(x, inverse, zero);
-  return (uint32_t)fminf(fmaxf(r + zf, 0.f), 15.f);  // r and the zero point are small integers: exact
+// Codes of a chunk's four values from value j0 as bytes.
+template <bool BF16>
+__device__ __forceinline__ uint32_t codes_int8(const u32x4& c, int j0, float inv32, double inverse) {
+  uint32_t w = 0;
+  bool unsafe = false;
+#pragma unroll
+  for (int j = 0; j < 4; j++) {
+    const float r = __builtin_amdgcn_fmed3f(nearest(Chunk<BF16>::at(c, j0 + j), inv32, kSafeInt8, unsafe), -127.f, 127.f);
+    w = __builtin_amdgcn_cvt_pk_u8_f32(r + 128.f, j, w);  // an integer in [1, 255]
+  }
+  w ^= 0x80808080u;
+  if (unsafe) {
+    w = 0;
+    for (int j = 0; j < 4; j++) w |= (uint32_t)(uint8_t)(int8_t)code_int8(Chunk<BF16>::at(c, j0 + j), inverse) << (8 * j);
+  }
+  return w;
+}
+// A chunk's codes (8 or 4 nibbles, value 0 lowest) where `unsafe` stays false, for values without
+// NaN or infinity. zf: the zero point, an integer in [0, 15], added before rounding (exactly what
+// adding it after gives, farther than kSafeInt4 from a half-integer: t32 + zf is off by 2^-20 more).
+template <bool BF16>
+__device__ __forceinline__ uint32_t codes_int4(const u32x4& c, float inv32, float zf, bool& unsafe) {
+  uint32_t w = 0;
+  float far = 0.f;
+#pragma unroll
+  for (int j = 0; j < Chunk<BF16>::kVals; j += 2) {
+    const float a = fmaf(Chunk<BF16>::at(c, j), inv32, zf), b = fmaf(Chunk<BF16>::at(c, j + 1), inv32, zf);
+    const float ra = __builtin_rintf(a), rb = __builtin_rintf(b);
+    far = fmaxf(far, fmaxf(fabsf(a - ra), fabsf(b - rb)));
+    // an integer in [0, 255]
+    w = __builtin_amdgcn_cvt_pk_u8_f32(fmaf(__builtin_amdgcn_fmed3f(rb, 0.f, 15.f), 16.f,
+                                            __builtin_amdgcn_fmed3f(ra, 0.f, 15.f)), j / 2, w);
+  }
+  unsafe |= !(far <= 0.5f - kSafeInt4);
+  return w;
+}
+template <bool BF16>
+__device__ __forceinline__ uint32_t codes_int4_f64(const u32x4& c, double inverse, float zf) {
+  uint32_t w = 0;
+  for (int j = 0; j < Chunk<BF16>::kVals; j++) w |= code_int4(Chunk<BF16>::at(c, j), inverse, (double)zf) << (4 * j);
+  return w;
+}
+template <bool BF16>
+__device__ __forceinline__ void store_int4(uint8_t* out, int ci, uint32_t w) {
+  if constexpr (BF16) *reinterpret_cast<uint32_t*>(out + (size_t)ci * 4) = w;
+  else *reinterpret_cast<uint16_t*>(out + (size_t)ci * 2) = (uint16_t)w;
+}
+
+// The range of each segment of G lanes' chunks (NaN never taken, as above). bf16: the values as
+// order-preserving 16-bit keys, two to a register (a quarter of the f32 compare-selects), unless
+// some value is NaN, whose keys lie outside the infinities'.
+template <int CTRL>
+__device__ __forceinline__ uint32_t dpp_u32(uint32_t v) {
+  return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, CTRL, 0xF, 0xF, true);
+}
+typedef short s16x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ s16x2 keys_of(uint32_t u) {  // two bf16 bit patterns; its own inverse
+  const s16x2 x = __builtin_bit_cast(s16x2, u);
+  return x ^ ((x >> 15) & (s16x2){0x7fff, 0x7fff});
+}
+__device__ __forceinline__ float key_value(short k) {
+  const uint16_t u = (uint16_t)(k ^ ((k >> 15) & 0x7fff));
+  return __uint_as_float((uint32_t)u << 16);
+}
+// Returns whether the wave met a NaN.
+template <bool BF16>
+__device__ __forceinline__ bool segment_range(const u32x4& c, int G, float& lo, float& hi) {
+  if constexpr (BF16) {
+    s16x2 mx = keys_of(c.x), mn = mx;
+#pragma unroll
+    for (int j = 1; j < 4; j++) {
+      const s16x2 k = keys_of(c[j]);
+      mx = __builtin_elementwise_max(mx, k);
+      mn = __builtin_elementwise_min(mn, k);
+    }
+    auto step = [&](auto other) {
+      mx = __builtin_elementwise_max(mx, __builtin_bit_cast(s16x2, other(__builtin_bit_cast(uint32_t, mx))));
+      mn = __builtin_elementwise_min(mn, __builtin_bit_cast(s16x2, other(__builtin_bit_cast(uint32_t, mn))));
+    };
+    if (G > 1) step([](uint32_t v) { return dpp_u32<0xB1>(v); });    // quad_perm: lane ^ 1
+    if (G > 2) step([](uint32_t v) { return dpp_u32<0x4E>(v); });    // quad_perm: lane ^ 2
+    if (G > 4) step([](uint32_t v) { return dpp_u32<0x141>(v); });   // row_half_mirror
+    if (G > 8) step([](uint32_t v) { return dpp_u32<0x140>(v); });   // row_mirror
+    for (int off = 16; off < G; off <<= 1) step([&](uint32_t v) { return (uint32_t)__shfl_xor((int)v, off); });
+    const short top = mx.x > mx.y ? mx.x : mx.y, bottom = mn.x < mn.y ? mn.x : mn.y;
+    constexpr short kInf = 0x7f80, kNegInf = (short)0x807f;
+    if (!__any(top > kInf || bottom < kNegInf)) {
+      lo = key_value(bottom);
+      hi = key_value(top);
+      return false;
+    }
+  }
+  bool nan = false;
+  lo = INFINITY;
+  hi = -INFINITY;
+#pragma unroll
+  for (int j = 0; j < Chunk<BF16>::kVals; j++) {
+    const float v = Chunk<BF16>::at(c, j);
+    nan |= v != v;
+    lo = take_min(lo, v);
+    hi = take_max(hi, v);
+  }
+  for (int off = 1; off < G; off <<= 1) {
+    lo = take_min(lo, __shfl_xor(lo, off));
+    hi = take_max(hi, __shfl_xor(hi, off));
+  }
+  return __any(nan);
 }
 
 // src/core/quantize.js:36-58, one wave per row, four rows per block; MAXC chunks per lane.
@@ -220,23 +330,105 @@ __global__ __launch_bounds__(kQBlock) void k_quant_int8_rows(const void* __restr
     if (ci >= nchunks) break;
     uint32_t w[C::kVals / 4];
 #pragma unroll
-    for (int j = 0; j < C::kVals; j++) {
-      const uint32_t b = scale != 0 ? (uint32_t)(uint8_t)(int8_t)code_int8_f32(C::at(c[k], j), inv32, inverse) : 0u;
-      if (j % 4 == 0) w[j / 4] = b;
-      else w[j / 4] |= b << (8 * (j % 4));
-    }
+    for (int j = 0; j < C::kVals; j += 4) w[j / 4] = scale != 0 ? codes_int8<BF16>(c[k], j, inv32, inverse) : 0u;
     if constexpr (BF16) *reinterpret_cast<uint2*>(out + (size_t)ci * 8) = uint2{w[0], w[1]};
     else *reinterpret_cast<uint32_t*>(out + (size_t)ci * 4) = w[0];
   }
 }
 
-// src/core/quantize.js:80-132, one wave per row: a group is G = group / chunk-values
-// consecutive chunks (G a power of two up to 64), so at step k lanes [G*i, G*i + G) hold group
-// (64k + G*i) / G and its range is a segmented reduction over those lanes.
-template <bool BF16, int MAXC>
+// src/core/quantize.js:80-132, one wave per R rows of at most 64 groups together: a group is
+// G = group / chunk-values consecutive chunks (G a power of two up to 64), so at step k of a row
+// lanes [G*i, G*i + G) hold its group (64k + G*i) / G and the range is a segmented reduction over
+// those lanes. Each group's f64 parameters (the divisions and Math.min / Math.max of
+// src/core/quantize.js:95-104: ~200 instructions, over a third of a one-row wave's work at 7
+// groups a row) are worked out once, lane l for group l of the R rows, and handed back by shuffles.
+// LG: log2 of G where it is compiled in (128-column groups), else -1.
+template <bool BF16, int MAXC, int R, int LG>
 __global__ __launch_bounds__(kQBlock) void k_quant_int4_rows(const void* __restrict__ src, int rows, int cols,
-                                                             int G, uint8_t* __restrict__ q,
+                                                             int lg, uint8_t* __restrict__ q,
                                                              float* __restrict__ scales, float* __restrict__ zeros) {
+  using C = Chunk<BF16>;
+  if constexpr (LG >= 0) lg = LG;
+  const int G = 1 << lg;
+  const int row0 = (blockIdx.x * (kQBlock / 64) + (threadIdx.x >> 6)) * R;
+  if (row0 >= rows) return;
+  const int lane = threadIdx.x & 63;
+  const int nchunks = cols / C::kVals, gpr = nchunks >> lg;
+  const int steps = (nchunks + 63) / 64, lp = 6 - lg;  // 2^lp groups per step: segment s of step k is group (k << lp) + s
+  u32x4 c[R][MAXC];
+#pragma unroll
+  for (int r = 0; r < R; r++) {
+    const u32x4* in = reinterpret_cast<const u32x4*>(src) + (size_t)min(row0 + r, rows - 1) * nchunks;
+#pragma unroll
+    for (int k = 0; k < MAXC; k++) {
+      const int ci = lane + 64 * k;
+      c[r][k] = ci < nchunks ? __builtin_nontemporal_load(in + ci) : u32x4{0, 0, 0, 0};
+    }
+  }
+  // Lane l collects the range of group l % gpr of row l / gpr.
+  const int own_row = lane / gpr, own = lane - own_row * gpr;
+  const int own_step = own >> lp, from = (own & ((1 << lp) - 1)) << lg;
+  uint32_t odd = 0;  // chunks with a NaN somewhere in the wave
+  float glo = INFINITY, ghi = -INFINITY;
+#pragma unroll
+  for (int r = 0; r < R; r++)
+#pragma unroll
+    for (int k = 0; k < MAXC; k++) {
+      if (MAXC > 2 && k >= steps) continue;  // wave-uniform
+      float lo, hi, a, b;
+      if (segment_range<BF16>(c[r][k], G, lo, hi)) odd |= 1u << (r * MAXC + k);
+      if constexpr (BF16) {  // both are bf16 values: one shuffle
+        const uint32_t u = (uint32_t)__shfl((int)((__float_as_uint(lo) >> 16) | __float_as_uint(hi)), from);
+        a = __uint_as_float(u << 16);
+        b = __uint_as_float(u & 0xffff0000u);
+      } else {
+        a = __shfl(lo, from);
+        b = __shfl(hi, from);
+      }
+      if (r == own_row && k == own_step) {
+        glo = a;
+        ghi = b;
+      }
+    }
+  double ginverse = 0;
+  float ginv32 = 0.f, gzero = -1.f;  // -1: a zero scale, whose codes are 0
+  if (own_row < min(R, rows - row0)) {
+    const double dlo = js_min(glo, 0), dhi = js_max(ghi, 0);
+    const double scale = (dhi - dlo) / 15;
+    const double zero = scale == 0 ? 0.0 : js_max(0, js_min(15, round(-dlo / scale)));
+    scales[(size_t)row0 * gpr + lane] = (float)scale;
+    zeros[(size_t)row0 * gpr + lane] = (float)zero;
+    ginverse = 1 / scale;
+    ginv32 = (float)ginverse;
+    if (scale != 0) gzero = (float)zero;  // an integer in [0, 15], or NaN
+  }
+  // An infinite range, or one whose f32 inverse overflows: f32 products may be NaN.
+  const bool infinite = __any(gzero != -1.f && (ginverse == 0 || ginv32 == INFINITY));
+#pragma unroll
+  for (int r = 0; r < R; r++) {
+    uint8_t* out = q + (size_t)(row0 + r) * (cols / 2);
+#pragma unroll
+    for (int k = 0; k < MAXC; k++) {
+      if (MAXC > 2 && k >= steps) continue;
+      const int ci = lane + 64 * k, owner = r * gpr + min(ci >> lg, gpr - 1);  // the chunk's group (clamped past the row)
+      const float inv32 = __shfl(ginv32, owner), zf = __shfl(gzero, owner);
+      bool unsafe = infinite || (odd >> (r * MAXC + k) & 1);
+      uint32_t w = codes_int4<BF16>(c[r][k], inv32, zf, unsafe);
+      if (__any(unsafe)) {  // wave-uniform, for the shuffle
+        const double inverse = __shfl(ginverse, owner);
+        if (unsafe) w = codes_int4_f64<BF16>(c[r][k], inverse, zf);
+      }
+      if (ci < nchunks && row0 + r < rows) store_int4<BF16>(out, ci, zf == -1.f ? 0u : w);
+    }
+  }
+}
+
+// The same for rows of more than 64 groups, one wave per row: every lane works its group's
+// parameters out at each step.
+template <bool BF16, int MAXC>
+__global__ __launch_bounds__(kQBlock) void k_quant_int4_steps(const void* __restrict__ src, int rows, int cols,
+                                                              int G, uint8_t* __restrict__ q,
+                                                              float* __restrict__ scales, float* __restrict__ zeros) {
   using C = Chunk<BF16>;
   const int row = blockIdx.x * (kQBlock / 64) + (threadIdx.x >> 6);
   if (row >= rows) return;
@@ -251,91 +443,12 @@ __global__ __launch_bounds__(kQBlock) void k_quant_int4_rows(const void* __restr
     c[k] = ci < nchunks ? __builtin_nontemporal_load(in + ci) : u32x4{0, 0, 0, 0};
   }
   uint8_t* out = q + (size_t)row * (cols / 2);
-  if (MAXC <= 4 && gpr <= 64) {
-    // A row of at most 64 groups and 4 chunks per lane: each group's f64 parameters (the
-    // divisions and Math.min / Math.max of src/core/quantize.js:95-104) are worked out once,
-    // by lane g for group g, not by each of the group's G lanes at every step, and handed back
-    // by shuffles (with more chunks per lane, the held ranges and shuffles cost more than the
-    // divisions they save: 4864-column rows ran 29% -> 19% of HBM).
-    const int steps = (nchunks + 63) / 64, per = 64 / G;  // groups per step: segment s of step k is group k*per + s
-    float los[MAXC], his[MAXC];
-#pragma unroll
-    for (int k = 0; k < MAXC; k++) {
-      float lo = INFINITY, hi = -INFINITY;
-      if (k < steps) {  // wave-uniform: the segmented reduction needs every lane
-#pragma unroll
-        for (int j = 0; j < C::kVals; j++) {
-          const float v = C::at(c[k], j);
-          lo = take_min(lo, v);
-          hi = take_max(hi, v);
-        }
-        for (int off = 1; off < G; off <<= 1) {
-          lo = take_min(lo, __shfl_xor(lo, off));
-          hi = take_max(hi, __shfl_xor(hi, off));
-        }
-      }
-      los[k] = lo;
-      his[k] = hi;
-    }
-    // Lane g collects group g's range (segment g % per of step g / per).
-    float glo = INFINITY, ghi = -INFINITY;
-#pragma unroll
-    for (int k = 0; k < MAXC; k++) {
-      if (k >= steps) break;
-      const float a = __shfl(los[k], (lane % per) * G), b = __shfl(his[k], (lane % per) * G);
-      if (k == lane / per) {
-        glo = a;
-        ghi = b;
-      }
-    }
-    double ginverse = 0;
-    float gzero = -1.f;  // -1: a zero scale, whose codes are 0
-    if (lane < gpr) {
-      const double dlo = js_min(glo, 0), dhi = js_max(ghi, 0);
-      const double scale = (dhi - dlo) / 15;
-      const double zero = scale == 0 ? 0.0 : js_max(0, js_min(15, round(-dlo / scale)));
-      scales[(size_t)row * gpr + lane] = (float)scale;
-      zeros[(size_t)row * gpr + lane] = (float)zero;
-      ginverse = 1 / scale;
-      if (scale != 0) gzero = (float)zero;  // an integer in [0, 15], or NaN
-    }
-#pragma unroll
-    for (int k = 0; k < MAXC; k++) {
-      if (k >= steps) break;
-      const int ci = lane + 64 * k, owner = min(ci / G, gpr - 1);  // the chunk's group (clamped past the row)
-      const double inverse = __shfl(ginverse, owner);
-      const float zf = __shfl(gzero, owner);
-      if (ci >= nchunks || zf == -1.f) {
-        if (ci < nchunks) {
-          if constexpr (BF16) *reinterpret_cast<uint32_t*>(out + (size_t)ci * 4) = 0u;
-          else *reinterpret_cast<uint16_t*>(out + (size_t)ci * 2) = (uint16_t)0;
-        }
-        continue;
-      }
-      const float inv32 = (float)inverse;
-      uint32_t w = 0;
-#pragma unroll
-      for (int j = 0; j < C::kVals; j++) w |= code_int4_f32(C::at(c[k], j), inv32, inverse, (double)zf, zf) << (4 * j);
-      if constexpr (BF16) *reinterpret_cast<uint32_t*>(out + (size_t)ci * 4) = w;
-      else *reinterpret_cast<uint16_t*>(out + (size_t)ci * 2) = (uint16_t)w;
-    }
-    return;
-  }
 #pragma unroll
   for (int k = 0; k < MAXC; k++) {
     const int ci = lane + 64 * k;
     if (64 * k >= nchunks) break;   // wave-uniform: the segmented reduction needs every lane
-    float lo = INFINITY, hi = -INFINITY;
-#pragma unroll
-    for (int j = 0; j < C::kVals; j++) {
-      const float v = C::at(c[k], j);
-      lo = take_min(lo, v);
-      hi = take_max(hi, v);
-    }
-    for (int off = 1; off < G; off <<= 1) {
-      lo = take_min(lo, __shfl_xor(lo, off));
-      hi = take_max(hi, __shfl_xor(hi, off));
-    }
+    float lo, hi;
+    const bool odd = segment_range<BF16>(c[k], G, lo, hi);
     if (ci >= nchunks) continue;
     const double dlo = js_min(lo, 0), dhi = js_max(hi, 0);
     const double scale = (dhi - dlo) / 15;
@@ -346,14 +459,11 @@ __global__ __launch_bounds__(kQBlock) void k_quant_int4_rows(const void* __restr
       zeros[gi] = (float)zero;
     }
     const double inverse = 1 / scale;
-    const float inv32 = (float)inverse, zf = (float)zero;
-    uint32_t w = 0;
-    if (scale != 0) {
-#pragma unroll
-      for (int j = 0; j < C::kVals; j++) w |= code_int4_f32(C::at(c[k], j), inv32, inverse, zero, zf) << (4 * j);
-    }
-    if constexpr (BF16) *reinterpret_cast<uint32_t*>(out + (size_t)ci * 4) = w;
-    else *reinterpret_cast<uint16_t*>(out + (size_t)ci * 2) = (uint16_t)w;
+    const float inv32 = (float)inverse;
+    bool unsafe = odd || inverse == 0 || inv32 == INFINITY;  // f32 products may be NaN
+    uint32_t w = codes_int4<BF16>(c[k], inv32, (float)zero, unsafe);
+    if (unsafe) w = codes_int4_f64<BF16>(c[k], inverse, (float)zero);
+    store_int4<BF16>(out, ci, scale != 0 ? w : 0u);
   }
 }
 
@@ -429,11 +539,25 @@ void launch_int8_rows(hipStream_t s, const void* src, int rows, int cols, int8_t
   hipLaunchKernelGGL((k_quant_int8_rows<BF16, MAXC>), dim3((rows + 3) / 4), dim3(kQBlock), 0, s, src, rows, cols, q,
                      scales);
 }
-template <bool BF16, int MAXC>
+template <bool BF16, int MAXC, int R>
 void launch_int4_rows(hipStream_t s, const void* src, int rows, int cols, int G, uint8_t* q, float* scales,
                       float* zeros) {
-  hipLaunchKernelGGL((k_quant_int4_rows<BF16, MAXC>), dim3((rows + 3) / 4), dim3(kQBlock), 0, s, src, rows, cols, G,
-                     q, scales, zeros);
+  // Rows together while their groups fit the wave's lanes (R rows of MAXC chunks a lane are 8 to
+  // 16 loads in flight); more than 64 groups a row go step by step.
+  const int gpr = cols / Chunk<BF16>::kVals / G;
+  const auto blocks = [&](int r) { return dim3((rows + 4 * r - 1) / (4 * r)); };
+  int lg = 0;
+  while ((1 << lg) < G) lg++;
+  constexpr int kLg = BF16 ? 4 : 5;  // chunks of a 128-column group
+  if (R * gpr <= 64 && lg == kLg)
+    hipLaunchKernelGGL((k_quant_int4_rows<BF16, MAXC, R, kLg>), blocks(R), dim3(kQBlock), 0, s, src, rows, cols, lg,
+                       q, scales, zeros);
+  else if (gpr <= 64)
+    hipLaunchKernelGGL((k_quant_int4_rows<BF16, MAXC, 1, -1>), blocks(1), dim3(kQBlock), 0, s, src, rows, cols, lg, q,
+                       scales, zeros);
+  else
+    hipLaunchKernelGGL((k_quant_int4_steps<BF16, MAXC>), blocks(1), dim3(kQBlock), 0, s, src, rows, cols, G, q,
+                       scales, zeros);
 }
 
 template <bool BF16>
@@ -476,10 +600,10 @@ hipError_t convert_t(hipStream_t s, const void* src, int rows, int cols, int for
       uint8_t* q = static_cast<uint8_t*>(data);
       const int G = group / kVals;
       if (maxc && group % kVals == 0 && G <= 64 && (G & (G - 1)) == 0 && aligned(data, BF16 ? 4 : 2)) {
-        if (maxc == 2) launch_int4_rows<BF16, 2>(s, src, rows, cols, G, q, scales, zeros);
-        else if (maxc == 4) launch_int4_rows<BF16, 4>(s, src, rows, cols, G, q, scales, zeros);
-        else if (maxc == 8) launch_int4_rows<BF16, 8>(s, src, rows, cols, G, q, scales, zeros);
-        else launch_int4_rows<BF16, 16>(s, src, rows, cols, G, q, scales, zeros);
+        if (maxc == 2) launch_int4_rows<BF16, 2, 4>(s, src, rows, cols, G, q, scales, zeros);
+        else if (maxc == 4) launch_int4_rows<BF16, 4, 2>(s, src, rows, cols, G, q, scales, zeros);
+        else if (maxc == 8) launch_int4_rows<BF16, 8, 1>(s, src, rows, cols, G, q, scales, zeros);
+        else launch_int4_rows<BF16, 16, 1>(s, src, rows, cols, G, q, scales, zeros);
       } else {
         const size_t items = (size_t)rows * (cols / group);
         hipLaunchKernelGGL(k_quant_int4<BF16>, dim3((unsigned)((items + 3) / 4)), dim3(kQBlock), 0, s, src, rows,

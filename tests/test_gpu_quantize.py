@@ -247,3 +247,38 @@ def test_load_tensor_rejects_what_set_tensor_rejects(ctx, hip):
         hip.GpuModel.load_checkpoint(ctx, {**ckpt, name: ckpt[name].astype(np.float64)}, cfg, "int4", 128)
     with pytest.raises(hip.QwenHipError):
         hip.GpuModel.load_checkpoint(ctx, ckpt, cfg, "int4", 96)
+
+
+@pytest.mark.parametrize("src", ["bf16", "f32"])
+@pytest.mark.parametrize("rows,cols,group", [
+    (9, 896, 128),      # four rows a wave, the last wave one row
+    (5, 1792, 128),     # two rows a wave
+    (3, 4864, 128),     # one row a wave
+    (3, 4864, 32),      # more than 64 groups a row: step by step
+    (6, 64, 16),        # one group per few lanes, lanes past the row
+])
+def test_int4_shared_parameters_match_oracle(ctx, hip, src, rows, cols, group):
+    """The row forms' edges: rows past a wave's share, groups of every kind beside each other --
+    zero, one-signed, NaN, infinite, and ranges so small that their f32 inverse overflows (with
+    zeros among their values)."""
+    rng = np.random.default_rng(rows * cols)
+    w = (rng.standard_normal((rows, cols)) * 0.02).astype(np.float32)
+    g = w.reshape(rows, cols // group, group)
+    g[0, 0] = 0.0
+    g[-1, -1, ::3] = np.nan
+    g[1, 1, 5] = np.inf
+    g[2, 0] = np.where(np.arange(group) % 3 == 0, 0.0, np.sign(g[2, 0]) * np.float32(9.2e-41))
+    g[0, 2] = np.abs(g[0, 2])
+    if src == "bf16":
+        host = (w.view(np.uint32) >> 16).astype(np.uint16)
+        fmt, wide = hip.FMT_BF16, O.bf16_to_f32(host)
+    else:
+        fmt, host, wide = hip.FMT_F32, w, w
+    d = ctx.upload(host)
+    data, scales, zeros = ctx.quantize(d, fmt, rows, cols, hip.FMT_INT4, group)
+    q, s, z = O.quantize_int4(wide, group)
+    np.testing.assert_array_equal(data.read(np.uint8, rows * cols // 2), np.asarray(q).reshape(-1))
+    np.testing.assert_array_equal(bits32(scales.read(np.float32, s.size)), bits32(s).reshape(-1))
+    np.testing.assert_array_equal(bits32(zeros.read(np.float32, z.size)), bits32(z).reshape(-1))
+    for b in (d, data, scales, zeros):
+        b.free()
