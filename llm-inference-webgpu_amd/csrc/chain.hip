@@ -411,7 +411,7 @@ hipError_t launch_chain_f32(hipStream_t s, const DMat& m, const float* x, const 
 // and a dequantized weight per eight positions. A block takes 32 positions x 16 rows, its four
 // waves a quarter of the team's slots each (so 52 positions of a 4864-row matrix are 608 blocks),
 // joined through LDS in tree order. A wave stages its own slabs of x, so no barrier runs in the
-// loop; weights go to registers a chunk ahead. 4864 x 896 int8, 52 positions: 90 -> X us.
+// loop; weights go to registers a chunk ahead. 4864 x 896 int8, 52 positions: 90 -> 23 us.
 typedef double f64x4 __attribute__((ext_vector_type(4)));
 
 template <int FMT>

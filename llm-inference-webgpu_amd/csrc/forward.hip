@@ -99,24 +99,6 @@ __global__ void k_rope_kv(const float* __restrict__ qkv, int splits, const float
   }
 }
 
-// The decode step's slot merge for every query: out [seq][heads*64]. grid (seq).
-__global__ __launch_bounds__(kBlock) void k_attn_merge_rows(const float* __restrict__ part, int heads,
-                                                            float* __restrict__ out) {
-  __shared__ float wl[kBlock];
-  const int t = blockIdx.x;
-  CombineIn in;
-  in.load(part + (size_t)t * heads * kDecodeSlots * kPartStride, heads);
-  const v4f acc = attn_combine_quad(in, wl);
-  const int i = threadIdx.x;
-  if (i < heads * kCombineLanes) {
-    float* o = out + (size_t)t * heads * kHeadDim + (i / kCombineLanes) * kHeadDim + 4 * (i % kCombineLanes);
-    o[0] = acc.x;
-    o[1] = acc.y;
-    o[2] = acc.z;
-    o[3] = acc.w;
-  }
-}
-
 // h[t][j] = silu(g) * u over interleaved gate|up rows (g = gu[t][2j], u = gu[t][2j+1]), as
 // the decode step's SWIGLU epilogue evaluates it: in f64 (src/core/ops.js:81-91), or in
 // f32 for fast numerics (F32).
@@ -178,8 +160,8 @@ PrefillBytes prefill_bytes(const ModelDev& m, const CacheDev& c, int matmul) {
   const size_t d = m.hidden, kv = (size_t)m.kv_heads * m.head_dim, f = m.intermediate;
   PrefillBytes b{};
   b.floats = P * (5 * d + (d + 2 * kv) + 3 * f);
-  if (m.numerics == QH_NUMERICS_FAST) b.floats += P * m.heads * kDecodeSlots * kPartStride;
-  else if (c.capacity > kPLds) b.floats += P * m.heads * (c.score_stride + attn_spans(c.capacity));
+  if (m.numerics == QH_NUMERICS_FAST && decode_attn_long(c.capacity)) b.floats += P * m.heads * kDecodeSlots * kPartStride;
+  else if (m.numerics == QH_NUMERICS_EXACT && c.capacity > kPLds) b.floats += P * m.heads * (c.score_stride + attn_spans(c.capacity));
   b.counters = m.numerics == QH_NUMERICS_EXACT ? P * m.heads : 0;
   const bool chain = m.numerics == QH_NUMERICS_FAST && !(matmul == QH_MATMUL_MFMA && all_mfma(m));
   size_t scratch = chain ? chain_partials_bound(m.lm_head, kHeadRows) : 0;  // enqueue_head_rows
@@ -338,8 +320,8 @@ hipError_t enqueue_prefill_layers(hipStream_t s, const ModelDev& m, const CacheD
       a.heads = m.heads;
       a.kv_heads = m.kv_heads;
       if (!decode_attn_long(c.capacity)) {
-        if ((e = launch_attn_decode(s, a, seq, 1)) != hipSuccess) return e;
-        hipLaunchKernelGGL(k_attn_merge_rows, dim3(seq), dim3(kBlock), 0, s, p.part, m.heads, p.ATT);
+        a.out = p.ATT;
+        if ((e = launch_attn_prompt(s, a, seq)) != hipSuccess) return e;
       } else {
         // a long cache's kLongSlots partials per query, a share of the rows at a time so that
         // they fit the workspace sized for kDecodeSlots (each query's result is its own)

@@ -90,3 +90,28 @@ def test_exact_matvec_on_matrix_cores_equals_single_positions_bitwise(ctx, hip, 
                                       err_msg=f"{seq} positions")
     for b in bufs + [bias, dx, dy]:
         b.free()
+
+
+def test_prompt_attention_past_1024_positions_equals_steps_bitwise(ctx, hip):
+    """Slots of several chunks (four states a slot), and the step from one chunk a slot to two, in
+    the prompt's merged attention: the decode steps' logits and K/V rows bit for bit."""
+    cfg = hip.ModelConfig(hidden=256, intermediate=256, layers=2, heads=4, kv_heads=2, vocab=1000)
+    model = hip.GpuModel.load(ctx, hip.device_tensors(hip.synthesize_checkpoint(cfg, seed=22), cfg, "int8", 128, "int8"),
+                              cfg, maxPositions=2300)
+    ids = hip.synth_tokens(22, "chain.long", cfg.vocab, 2250)
+    steps, cache = model.newCache(2300), model.newCache(2300)
+    model.set_matmul("matvec")
+    want = {}
+    for a, b in ((0, 1010), (1010, 1040), (1040, 2040), (2040, 2250)):
+        want[b] = model.forward_tokens(ids[a:b], steps)["logits"]
+    model.set_matmul("batched")
+    for a, b in ((0, 1010), (1010, 1040), (1040, 2040), (2040, 2250)):
+        got = model.forward_tokens(ids[a:b], cache)["logits"]
+        np.testing.assert_array_equal(got.view(np.uint32), want[b].view(np.uint32), err_msg=f"to {b}")
+    for L in range(cfg.layers):
+        p, s = cache.present(L), steps.present(L)
+        np.testing.assert_array_equal(p["key"], s["key"])
+        np.testing.assert_array_equal(p["value"], s["value"])
+    cache.destroy()
+    steps.destroy()
+    model.destroy()
