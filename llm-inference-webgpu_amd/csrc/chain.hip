@@ -323,16 +323,9 @@ __global__ __launch_bounds__(kBlock, 2) void k_chain_f32(ChainArgs a) {
 }
 
 // y[p][r] = the balanced tree over the splits' roots, then the row scale and the bias.
-template <int FMT>
-__global__ __launch_bounds__(kBlock) void k_chain_finish(const float* __restrict__ part, int splits, size_t plane,
-                                                         int rows, const float* __restrict__ scales,
-                                                         const float* __restrict__ bias, float* __restrict__ y) {
+__global__ __launch_bounds__(kBlock) void k_chain_finish(ChainOut o, float* __restrict__ y) {
   const size_t i = (size_t)blockIdx.x * kBlock + threadIdx.x;
-  if (i >= plane) return;
-  const int r = (int)(i % rows);
-  float v = split_tree(part + i, plane, splits);
-  if constexpr (FMT == QH_FMT_INT8) v = row_out_f32<FMT>(v, scales[r]);
-  y[i] = bias ? __fadd_rn(v, bias[r]) : v;
+  if (i < (size_t)o.seq * o.rows) y[i] = chain_value(o, i, (int)(i % o.rows));
 }
 
 // Splits of the team's slots over blocks: enough that the chip holds about three blocks per CU.
@@ -367,38 +360,38 @@ static void chain_lv(hipStream_t s, const ChainArgs& a, dim3 grid, int lv) {
   }
 }
 
-template <int FMT>
-static hipError_t chain_fmt(hipStream_t s, const ChainArgs& a0, float* part, int splits) {
-  ChainArgs a = a0;
-  if (splits > 1) a.y = part;
-  const dim3 grid((a.m.rows + kChainN - 1) / kChainN, (a.seq + kChainM - 1) / kChainM, splits);
+hipError_t launch_chain_roots(hipStream_t s, const DMat& m, const float* x, const float* bias, float* y, int seq,
+                              float* part, size_t part_bytes, ChainOut* out) {
+  if (chain_partials_bytes(m, seq) > part_bytes) return hipErrorInvalidValue;
+  const int splits = chain_splits(m, seq);
+  ChainArgs a{};
+  a.m = m;
+  a.x = x;
+  a.bias = bias;
+  a.y = splits > 1 ? part : y;
+  a.seq = seq;
+  a.tl = team_width(m.nchunks);
+  const dim3 grid((m.rows + kChainN - 1) / kChainN, (seq + kChainM - 1) / kChainM, splits);
   int lv = 0;
-  while ((ChainFmt<FMT>::kS << lv) < a.tl / splits) lv++;
-  chain_lv<FMT, ChainFmt<FMT>::kLevels>(s, a, grid, lv);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess || splits == 1) return e;
-  const size_t plane = (size_t)a.seq * a.m.rows;
-  hipLaunchKernelGGL(k_chain_finish<FMT>, dim3((unsigned)((plane + kBlock - 1) / kBlock)), dim3(kBlock), 0, s, part,
-                     splits, plane, a.m.rows, a.m.scales, a.bias, a0.y);
+  while (((m.format == QH_FMT_INT4 ? 2 : 4) << lv) < a.tl / splits) lv++;
+  switch (m.format) {
+    case QH_FMT_F16: chain_lv<QH_FMT_F16, ChainFmt<QH_FMT_F16>::kLevels>(s, a, grid, lv); break;
+    case QH_FMT_INT8: chain_lv<QH_FMT_INT8, ChainFmt<QH_FMT_INT8>::kLevels>(s, a, grid, lv); break;
+    default: chain_lv<QH_FMT_INT4, ChainFmt<QH_FMT_INT4>::kLevels>(s, a, grid, lv); break;
+  }
+  *out = ChainOut{a.y, splits, m.rows, seq, splits > 1 && m.format == QH_FMT_INT8 ? m.scales : nullptr,
+                  splits > 1 ? bias : nullptr};
   return hipGetLastError();
 }
 
 hipError_t launch_chain_f32(hipStream_t s, const DMat& m, const float* x, const float* bias, float* y, int seq,
                             float* part, size_t part_bytes) {
-  if (chain_partials_bytes(m, seq) > part_bytes) return hipErrorInvalidValue;
-  ChainArgs a{};
-  a.m = m;
-  a.x = x;
-  a.bias = bias;
-  a.y = y;
-  a.seq = seq;
-  a.tl = team_width(m.nchunks);
-  const int splits = chain_splits(m, seq);
-  switch (m.format) {
-    case QH_FMT_F16: return chain_fmt<QH_FMT_F16>(s, a, part, splits);
-    case QH_FMT_INT8: return chain_fmt<QH_FMT_INT8>(s, a, part, splits);
-    default: return chain_fmt<QH_FMT_INT4>(s, a, part, splits);
-  }
+  ChainOut o;
+  const hipError_t e = launch_chain_roots(s, m, x, bias, y, seq, part, part_bytes, &o);
+  if (e != hipSuccess || o.splits == 1) return e;
+  const size_t plane = (size_t)seq * m.rows;
+  hipLaunchKernelGGL(k_chain_finish, dim3((unsigned)((plane + kBlock - 1) / kBlock)), dim3(kBlock), 0, s, o, y);
+  return hipGetLastError();
 }
 
 // --------------------------------------------------------------- f64 order --

@@ -764,17 +764,42 @@ __device__ __forceinline__ void mv_team_f32(const DMat& m, const int (&rows)[R],
     for (int i = 0; i < R; i++) acc[b][i] = row_out_f32<FMT>(team_sum<TL>(acc[b][i]), srow[i]);
 }
 
-// The balanced tree over `splits` (2, 4 or 8) partial roots `plane` floats apart, in order: the
+// The balanced tree over `splits` (1, 2, 4 or 8) partial roots `plane` elements apart, in order: the
 // butterfly of a team whose lanes were split over blocks. Every load is issued before any is used.
-__device__ __forceinline__ float split_tree(const float* __restrict__ p, size_t plane, int splits) {
-  float v[8];
+template <typename T>
+__device__ __forceinline__ T split_tree(const T* __restrict__ p, size_t plane, int splits) {
+  if (splits == 1) return p[0];
+  T v[8];
 #pragma unroll
   for (int i = 0; i < 8; i++) v[i] = p[(size_t)min(i, splits - 1) * plane];
-  const float a = v[0] + v[1];
+  const T a = v[0] + v[1];
   if (splits == 2) return a;
-  const float b = a + (v[2] + v[3]);
+  const T b = a + (v[2] + v[3]);
   if (splits == 4) return b;
   return b + ((v[4] + v[5]) + (v[6] + v[7]));
+}
+
+// Output i (of row r) of a contraction: the tree over its splits, the row scale and the bias.
+__device__ __forceinline__ float chain_value(const ChainOut& o, size_t i, int r) {
+  float v = split_tree(o.p + i, (size_t)o.seq * o.rows, o.splits);
+  if (o.scales) v = mul_rounded(o.scales[r], v);
+  return o.bias ? __fadd_rn(v, o.bias[r]) : v;
+}
+// Outputs 4 i4 .. +3 of position t (rows a multiple of 4).
+__device__ __forceinline__ v4f chain_value4(const ChainOut& o, int t, int i4) {
+  const size_t n4 = o.rows / 4;
+  v4f v = split_tree(reinterpret_cast<const v4f*>(o.p) + t * n4 + i4, o.seq * n4, o.splits);
+  if (o.scales) {
+    const v4f s = reinterpret_cast<const v4f*>(o.scales)[i4];
+#pragma unroll
+    for (int e = 0; e < 4; e++) v[e] = mul_rounded(s[e], v[e]);
+  }
+  if (o.bias) {
+    const v4f b = reinterpret_cast<const v4f*>(o.bias)[i4];
+#pragma unroll
+    for (int e = 0; e < 4; e++) v[e] = __fadd_rn(v[e], b[e]);
+  }
+  return v;
 }
 
 // Team width of a matrix: 32 lanes when a row has at most 32 chunks, else 64.

@@ -63,7 +63,9 @@ __device__ __forceinline__ void split_sum_cols(const float* row, size_t plane, i
   }
 }
 
-__global__ void k_rope_kv(const float* __restrict__ qkv, int splits, const float* __restrict__ bias,
+// CHAIN: the row comes from the f32 contraction `chain` (its splits' tree, scale and bias) instead.
+template <bool CHAIN>
+__global__ void k_rope_kv(const float* __restrict__ qkv, int splits, const float* __restrict__ bias, ChainOut chain,
                           float* __restrict__ q, uint16_t* __restrict__ kc, uint16_t* __restrict__ vt,
                           const double* __restrict__ rope_cos, const double* __restrict__ rope_sin, int past,
                           int heads, int kv_heads, int capacity, int vstride) {
@@ -80,7 +82,12 @@ __global__ void k_rope_kv(const float* __restrict__ qkv, int splits, const float
     const double cs = rope_cos[(size_t)pos * 32 + j], sn = rope_sin[(size_t)pos * 32 + j];
     const int col[2] = {base + j, base + j + 32};
     float x[2], lo, hi;
-    split_sum_cols<2>(row, plane, splits, bias, col, x);
+    if constexpr (CHAIN) {
+#pragma unroll
+      for (int k = 0; k < 2; k++) x[k] = chain_value(chain, (size_t)t * width + col[k], col[k]);
+    } else {
+      split_sum_cols<2>(row, plane, splits, bias, col, x);
+    }
     rope_pair(x[0], x[1], cs, sn, &lo, &hi);
     if (head < heads) {
       q[(size_t)t * hidden + head * kHeadDim + j] = lo;
@@ -94,7 +101,8 @@ __global__ void k_rope_kv(const float* __restrict__ qkv, int splits, const float
     const int e = i - rope_pairs;  // kv head e/64, dimension e%64
     const int col[1] = {hidden + kvd + e};
     float x[1];
-    split_sum_cols<1>(row, plane, splits, bias, col, x);
+    if constexpr (CHAIN) x[0] = chain_value(chain, (size_t)t * width + col[0], col[0]);
+    else split_sum_cols<1>(row, plane, splits, bias, col, x);
     vt[(size_t)e * vstride + pos] = __builtin_bit_cast(uint16_t, (_Float16)x[0]);
   }
 }
@@ -112,6 +120,46 @@ __global__ void k_swiglu_pairs(const float* __restrict__ gu, float* __restrict__
     const double g = gu[2 * i], u = gu[2 * i + 1];
     h[i] = (float)(g / (1.0 + exp(-g)) * u);
   }
+}
+
+// The residual add of a contraction and the rmsnorm that follows it (gain null: the add alone), a
+// row per block: x += y, xn = rmsnorm(x), as launch_add and k_rmsnorm_f32 evaluate them over a
+// finished y. n % 4 == 0, n <= kStageMax.
+__global__ __launch_bounds__(kBlock) void k_chain_add_norm(ChainOut y, float* __restrict__ x,
+                                                           const float* __restrict__ gain, float eps,
+                                                           float* __restrict__ xn) {
+  __shared__ float red[kBlock / kWave];
+  const int t = blockIdx.x, n = y.rows, n4 = n >> 2;
+  v4f* x4 = reinterpret_cast<v4f*>(x + (size_t)t * n);
+  StageIn in;
+#pragma unroll
+  for (int j = 0; j < kStageVec; j++) {
+    const int i = threadIdx.x + j * kBlock;
+    if (i < n4) {
+      const v4f r = x4[i];
+      if (gain) in.g[j] = reinterpret_cast<const v4f*>(gain)[i];
+      in.v[j] = r + chain_value4(y, t, i);
+      x4[i] = in.v[j];
+    }
+  }
+  if (!gain) return;
+  const float scale = rms_scale_f32(in, n, eps, red);
+  v4f* y4 = reinterpret_cast<v4f*>(xn + (size_t)t * n);
+#pragma unroll
+  for (int j = 0; j < kStageVec; j++) {
+    const int i = threadIdx.x + j * kBlock;
+    if (i < n4) y4[i] = rms_apply_f32(in.v[j], scale, in.g[j]);
+  }
+}
+
+// h[t][j] = silu(gate) * up over the interleaved gate|up outputs, four outputs a thread.
+// grid (ceil(rows / 4 / 256), seq).
+__global__ __launch_bounds__(kBlock) void k_chain_swiglu(ChainOut gu, float* __restrict__ h) {
+  const int t = blockIdx.y, i = blockIdx.x * kBlock + threadIdx.x;
+  if (i >= gu.rows / 4) return;
+  const v4f v = chain_value4(gu, t, i);
+  *reinterpret_cast<float2*>(h + (size_t)t * (gu.rows / 2) + 2 * i) =
+      float2{swiglu_f32(v.x, v.y), swiglu_f32(v.z, v.w)};
 }
 
 // rows [seq][hidden] = bf16 embedding rows of tokens[past .. past+seq-1], widened exactly.
@@ -236,8 +284,8 @@ static hipError_t prefill_layers_mfma(hipStream_t s, const ModelDev& m, const Ca
     Out o;
     if ((e = gemm(l.qkv, l.qkv_bias, p.QKV, &o)) != hipSuccess) return e;
     const int items = (m.heads + m.kv_heads) * 32 + m.kv_heads * m.head_dim;
-    hipLaunchKernelGGL(k_rope_kv, dim3((items + 255) / 256, seq), dim3(256), 0, s, o.p, o.splits, o.bias, p.Q, kc,
-                       vt, m.rope_cos, m.rope_sin, past, m.heads, m.kv_heads, c.capacity, c.vstride);
+    hipLaunchKernelGGL(k_rope_kv<false>, dim3((items + 255) / 256, seq), dim3(256), 0, s, o.p, o.splits, o.bias,
+                       ChainOut{}, p.Q, kc, vt, m.rope_cos, m.rope_sin, past, m.heads, m.kv_heads, c.capacity, c.vstride);
     if ((e = hipGetLastError()) != hipSuccess) return e;
     FlashArgs a{};
     a.q = p.Q;
@@ -278,9 +326,86 @@ static hipError_t matmul(hipStream_t s, const ModelDev& m, int mode, const DMat&
   return launch_matvec(s, w, x, bias, y, seq, static_cast<double*>(p.scratch));
 }
 
+// The batched fast-numerics attention of a layer: the decode step's, merged, into p.ATT.
+static hipError_t batched_attention(hipStream_t s, const ModelDev& m, const CacheDev& c, const PrefillDev& p,
+                                    const uint16_t* kc, const uint16_t* vt, int past, int seq) {
+  SlotArgs a{};
+  a.q = p.Q;
+  a.kc = kc;
+  a.vt = vt;
+  a.part = p.part;
+  a.past = past;
+  a.capacity = c.capacity;
+  a.vstride = c.vstride;
+  a.heads = m.heads;
+  a.kv_heads = m.kv_heads;
+  if (!decode_attn_long(c.capacity)) {
+    a.out = p.ATT;
+    return launch_attn_prompt(s, a, seq);
+  }
+  // a long cache's kLongSlots partials per query, a share of the rows at a time so that they fit
+  // the workspace sized for kDecodeSlots (each query's result is its own)
+  const int share = std::max(1, (int)p.positions * kDecodeSlots / kLongSlots);
+  for (int t0 = 0; t0 < seq; t0 += share) {
+    SlotArgs b = a;
+    b.q = p.Q + (size_t)t0 * m.heads * kHeadDim;
+    b.past = past + t0;
+    const hipError_t e =
+        launch_attn_decode(s, b, std::min(share, seq - t0), 1, p.ATT + (size_t)t0 * m.heads * kHeadDim);
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
+}
+
+// The batched fast-numerics layers with every contraction on the f32 matrix cores, its splits'
+// tree, scale, residual add, rmsnorm or swiglu in its consumer: eight launches a layer against
+// twelve (scoring 127 positions of int4 layers 4.1 -> 3.7 ms). The same operations in the same order, so the
+// same bits, as the launches of enqueue_prefill_layers.
+static hipError_t prefill_layers_chain(hipStream_t s, const ModelDev& m, const CacheDev& c, const PrefillDev& p,
+                                       int past, int seq) {
+  hipError_t e;
+  const int d = m.hidden, f = m.intermediate;
+  float* part = static_cast<float*>(p.scratch);
+  auto chain = [&](const DMat& w, const float* x, const float* bias, float* y, ChainOut* o) {
+    return launch_chain_roots(s, w, x, bias, y, seq, part, p.scratch_bytes, o);
+  };
+  auto add_norm = [&](const ChainOut& o, const float* gain) {
+    hipLaunchKernelGGL(k_chain_add_norm, dim3(seq), dim3(kBlock), 0, s, o, p.X, gain, (float)m.eps, p.XN);
+    return hipGetLastError();
+  };
+  if ((e = launch_rmsnorm(s, p.X, m.layers_host[0].in_norm, p.XN, seq, d, m.eps, true)) != hipSuccess) return e;
+  for (int L = 0; L < m.layers; L++) {
+    const LayerDev& l = m.layers_host[L];
+    uint16_t* kc = c.kv + (size_t)L * c.layer_elems;
+    uint16_t* vt = kc + c.key_elems;
+    ChainOut o;
+    if ((e = chain(l.qkv, p.XN, l.qkv_bias, p.QKV, &o)) != hipSuccess) return e;
+    const int items = (m.heads + m.kv_heads) * 32 + m.kv_heads * m.head_dim;
+    hipLaunchKernelGGL(k_rope_kv<true>, dim3((items + 255) / 256, seq), dim3(256), 0, s, nullptr, 1, nullptr, o, p.Q,
+                       kc, vt, m.rope_cos, m.rope_sin, past, m.heads, m.kv_heads, c.capacity, c.vstride);
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+    if ((e = batched_attention(s, m, c, p, kc, vt, past, seq)) != hipSuccess) return e;
+    if ((e = chain(l.o, p.ATT, nullptr, p.Y, &o)) != hipSuccess) return e;
+    if ((e = add_norm(o, l.post_norm)) != hipSuccess) return e;
+    if ((e = chain(l.gu, p.XN, nullptr, p.GU, &o)) != hipSuccess) return e;
+    hipLaunchKernelGGL(k_chain_swiglu, dim3((2 * f / 4 + kBlock - 1) / kBlock, seq), dim3(kBlock), 0, s, o, p.H);
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+    if ((e = chain(l.down, p.H, nullptr, p.Y, &o)) != hipSuccess) return e;
+    if ((e = add_norm(o, L + 1 < m.layers ? m.layers_host[L + 1].in_norm : nullptr)) != hipSuccess) return e;
+  }
+  return hipSuccess;
+}
+
+// Rows that prefill_layers_chain's consumers take as float4 groups.
+static bool chain_layers_supported(const ModelDev& m) {
+  return m.hidden % 4 == 0 && m.hidden <= kStageMax && m.intermediate % 2 == 0;
+}
+
 hipError_t enqueue_prefill_layers(hipStream_t s, const ModelDev& m, const CacheDev& c, const PrefillDev& p,
                                   int mode, int past, int seq) {
   if (mode == QH_MATMUL_MFMA && all_mfma(m)) return prefill_layers_mfma(s, m, c, p, past, seq);
+  if (mode != QH_MATMUL_MFMA && m.numerics == QH_NUMERICS_FAST && seq >= kChainMinSeq && chain_layers_supported(m))
+    return prefill_layers_chain(s, m, c, p, past, seq);
   hipError_t e;
   const int d = m.hidden, kvd = m.kv_heads * m.head_dim, f = m.intermediate;
   const size_t n = (size_t)seq * d;
@@ -291,7 +416,8 @@ hipError_t enqueue_prefill_layers(hipStream_t s, const ModelDev& m, const CacheD
     if ((e = launch_rmsnorm(s, p.X, l.in_norm, p.XN, seq, d, m.eps, m.numerics == QH_NUMERICS_FAST)) != hipSuccess) return e;
     if ((e = matmul(s, m, mode, l.qkv, p.XN, l.qkv_bias, p.QKV, seq, p)) != hipSuccess) return e;
     const int items = (m.heads + m.kv_heads) * 32 + kvd;
-    hipLaunchKernelGGL(k_rope_kv, dim3((items + 255) / 256, seq), dim3(256), 0, s, p.QKV, 1, nullptr, p.Q, kc, vt,
+    hipLaunchKernelGGL(k_rope_kv<false>, dim3((items + 255) / 256, seq), dim3(256), 0, s, p.QKV, 1, nullptr,
+                       ChainOut{}, p.Q, kc, vt,
                        m.rope_cos, m.rope_sin, past, m.heads, m.kv_heads, c.capacity, c.vstride);
     if ((e = hipGetLastError()) != hipSuccess) return e;
     if (mode == QH_MATMUL_MFMA) {
@@ -309,32 +435,7 @@ hipError_t enqueue_prefill_layers(hipStream_t s, const ModelDev& m, const CacheD
       a.kv_heads = m.kv_heads;
       if ((e = launch_flash_prefill(s, a)) != hipSuccess) return e;
     } else if (m.numerics == QH_NUMERICS_FAST) {
-      SlotArgs a{};
-      a.q = p.Q;
-      a.kc = kc;
-      a.vt = vt;
-      a.part = p.part;
-      a.past = past;
-      a.capacity = c.capacity;
-      a.vstride = c.vstride;
-      a.heads = m.heads;
-      a.kv_heads = m.kv_heads;
-      if (!decode_attn_long(c.capacity)) {
-        a.out = p.ATT;
-        if ((e = launch_attn_prompt(s, a, seq)) != hipSuccess) return e;
-      } else {
-        // a long cache's kLongSlots partials per query, a share of the rows at a time so that
-        // they fit the workspace sized for kDecodeSlots (each query's result is its own)
-        const int share = std::max(1, (int)p.positions * kDecodeSlots / kLongSlots);
-        for (int t0 = 0; t0 < seq; t0 += share) {
-          SlotArgs b = a;
-          b.q = p.Q + (size_t)t0 * m.heads * kHeadDim;
-          b.past = past + t0;
-          if ((e = launch_attn_decode(s, b, std::min(share, seq - t0), 1, p.ATT + (size_t)t0 * m.heads * kHeadDim)) !=
-              hipSuccess)
-            return e;
-        }
-      }
+      if ((e = batched_attention(s, m, c, p, kc, vt, past, seq)) != hipSuccess) return e;
     } else {
       ExactArgs a{};
       a.q = p.Q;

@@ -97,6 +97,17 @@ bool matvec_f32_supported(const DMat& m);
 hipError_t launch_chain_f32(hipStream_t s, const DMat& m, const float* x, const float* bias, float* y, int seq,
                             float* part, size_t part_bytes);
 constexpr int kChainMaxSplits = 8;
+// A contraction's outputs as its consumer reads them: finished rows [seq][rows], or `splits`
+// planes of roots whose tree, int8 row scale and bias are still to come.
+struct ChainOut {
+  const float* p;
+  int splits, rows, seq;
+  const float* scales;  // int8 with several splits, else null
+  const float* bias;    // with several splits, else null
+};
+// launch_chain_f32 without its finish launch: several splits stay as roots in `part`.
+hipError_t launch_chain_roots(hipStream_t s, const DMat& m, const float* x, const float* bias, float* y, int seq,
+                              float* part, size_t part_bytes, ChainOut* out);
 size_t chain_partials_bytes(const DMat& m, int seq);
 // launch_matvec's sums, bit for bit, on the f64 matrix cores (chain.hip), from kChain64MinSeq
 // positions and for 16-byte aligned x.
