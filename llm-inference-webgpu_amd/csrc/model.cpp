@@ -1008,6 +1008,7 @@ int qh_score(qh_model* m, qh_cache* c, const int32_t* h_ids, int32_t n, double* 
     return QH_OK;
   }
   // A single position, or no memory for the workspace: one decode step after another.
+  (void)hipGetLastError();  // a failed allocation is not the launches' error
   struct Scratch {
     int32_t* ids = nullptr;
     double* nll = nullptr;
