@@ -30,7 +30,7 @@ Also reported on the same JSON line:
   attention_decode  BASELINE config 3: split-K GQA attention over f16 caches at contexts
                  128 .. 32768, one list-driven launch over >= 512 MiB of distinct caches
   prefill_512    BASELINE config 5: time to first token of a 512-token prompt through each
-                 matmul path (per-position matvec, 8-position batched tiles, MFMA)
+                 matmul path (per-position matvec, batched contractions, MFMA)
   loader         the load path's conversion kernels (bf16 checkpoint -> int8 / int4 / f16
                  on the device) in GB/s, and the whole model load, host- vs device-converted
   path_comparison  the same-session comparison of the matmul paths (web/scaling.html): the
@@ -278,7 +278,7 @@ def attention_sweep(ctx, contexts=(128, 1024, 4096, 32768), heads=14, kv_heads=2
 
 def prefill_bench(ctx, cfg, ckpt, seed, prompt_len=512, modes=("matvec", "batched", "mfma")):
     """Config 5: time-to-first-token of a seeded prompt with int8 layers and head, through
-    one decode step per position, the reference's 8-position tiles, and the MFMA contraction.
+    one decode step per position, the batched contractions (the steps' bits), and the MFMA contraction.
     A token's time is wall clock around forward(): the ids' upload, the embedding gather, all
     layers, the head and the logits readback; best of 3. `ttft_ms` replays the prompt shape's
     graph (captured on the shape's second use, before the timed runs), `ttft_ms_direct` launches
@@ -765,7 +765,7 @@ def main():
     t0 = time.perf_counter()
     first = model.forward_tokens(prompt, cache)["argmax"]
     prefill_s = time.perf_counter() - t0
-    log(f"prefilled {args.context} positions in {prefill_s:.2f}s (8-position batched tiles)")
+    log(f"prefilled {args.context} positions in {prefill_s:.2f}s (batched)")
 
     if args.cold_only:
         print(json.dumps({"decode_kernels_cold": cold_decode_kernels(model, cache, cfg, args.context, None),

@@ -277,12 +277,12 @@ int qh_model_set_numerics(qh_model* m, int32_t numerics);
 
 /* How forward() processes several positions (GpuModel.load's `matmul` option, model.js:87-98,
  * 133-138, 297-317):
- *   QH_MATMUL_BATCHED (default): all positions per layer, each weight read once per 8-position
- *     tile (batchedMatvec); every output is summed as the decode step sums it, so a prefill and
+ *   QH_MATMUL_BATCHED (default): all positions per layer (batchedMatvec), on the f32 matrix
+ *     cores from 12 positions; every output is summed as the decode step sums it, so a prefill and
  *     the same positions decoded one by one give the same bits (README.md:256-272).
  *   QH_MATMUL_MATVEC: one decode step per position (the reference's 'matvec').
  *   QH_MATMUL_MFMA: all positions per layer, int8/int4 weights contracted on int8 MFMA
- *     (qh_matmul_prefill's digit planes; f16 weights use the batched tiles) and the prompt's
+ *     (qh_matmul_prefill's digit planes; f16 weights use the batched sums) and the prompt's
  *     attention on f16 MFMA (qh_attention_mfma); not bitwise equal to the others, within the
  *     reference's 1e-4 of them, as its 'tiled' path was (web/scaling.html:122-127). The
  *     reference's matmul option 'tiled' selects this mode in the bindings.
@@ -351,9 +351,9 @@ int qh_decode_collect(qh_model* m, qh_cache* c, int32_t steps, int32_t* h_tokens
  * reference, which records every step anew (src/gpu/model.js:261). */
 int qh_decode_prepare(qh_model* m, qh_cache* c);
 /* Scores a token sequence the way the reference's perplexity page does
- * (web/perplexity.html:146-170): ids[0..n-2] are fed one position at a time through the cache
- * (each step's input forced, as forward() of one token), and h_nll[t] (n - 1 doubles) receives
- * the negative log-likelihood of ids[t+1] under step t's logits, -(l[target] - max - log(sum
+ * (web/perplexity.html:146-170): ids[0..n-2] are fed through the cache with the bits
+ * of forward() of one token after another, and h_nll[t] (n - 1 doubles) receives
+ * the negative log-likelihood of ids[t+1] under position t's logits, -(l[target] - max - log(sum
  * exp(l - max))) in f64 on the device. Perplexity is exp(mean(h_nll)). The cache advances by
  * n - 1 positions; QH_ERR_RANGE for ids outside the vocabulary or a cache without room. */
 int qh_score(qh_model* m, qh_cache* c, const int32_t* h_ids, int32_t n, double* h_nll);

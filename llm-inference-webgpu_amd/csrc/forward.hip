@@ -1,6 +1,6 @@
 // The batched prefill forward: GpuModel.#forward (src/gpu/model.js:240-402) over
-// `seq` positions at once, each weight read once per 8-position tile
-// (QH_MATMUL_BATCHED, the reference's batchedMatvec, src/gpu/kernels.js:232-290,
+// `seq` positions at once, with the decode step's sums
+// (QH_MATMUL_BATCHED: chain.hip; the reference's batchedMatvec, src/gpu/kernels.js:232-290,
 // selected by src/gpu/model.js:297-306) or once per prefill on the matrix cores
 // (QH_MATMUL_MFMA, prefill.hip).
 //

@@ -694,7 +694,7 @@ class GpuModel:
         """Upload device tensors (see device_tensors) and finalize. numerics: "fast"
         (f32 sums, split-K attention on the f16 matrix cores) or "exact" (the CPU path's
         arithmetic, bit for bit). matmul: how forward() runs several positions --
-        "batched" (8-position weight tiles, bitwise equal to decoding them one by one),
+        "batched" (all positions per layer, bitwise equal to decoding them one by one),
         "matvec" (one decode step per position) or "mfma" (int8 matrix cores over exact
         activation digits, for int8/int4 weights)."""
         def upload(lib, handle):
