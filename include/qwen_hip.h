@@ -277,8 +277,8 @@ int qh_model_set_numerics(qh_model* m, int32_t numerics);
 
 /* How forward() processes several positions (GpuModel.load's `matmul` option, model.js:87-98,
  * 133-138, 297-317):
- *   QH_MATMUL_BATCHED (default): all positions per layer (batchedMatvec), on the f32 matrix
- *     cores from 12 positions; every output is summed as the decode step sums it, so a prefill and
+ *   QH_MATMUL_BATCHED (default): all positions per layer (batchedMatvec), longer prompts on
+ *     the f32 matrix cores; every output is summed as the decode step sums it, so a prefill and
  *     the same positions decoded one by one give the same bits (README.md:256-272).
  *   QH_MATMUL_MATVEC: one decode step per position (the reference's 'matvec').
  *   QH_MATMUL_MFMA: all positions per layer, int8/int4 weights contracted on int8 MFMA

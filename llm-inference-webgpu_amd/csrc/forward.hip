@@ -173,8 +173,17 @@ __global__ void k_embed_rows(const uint16_t* __restrict__ embed, const int* __re
     rows[(size_t)t * hidden + i] = __builtin_bit_cast(float, (uint32_t)src[i] << 16);
 }
 
-// Positions from which the batched contractions run on the f32 matrix cores (launch_chain_f32).
-constexpr int kChainMinSeq = 12;
+// Whether a batched contraction of `seq` positions runs on the f32 matrix cores (launch_chain_f32,
+// the same bits) or in launch_matvec_f32's tiles of 8 / 4 / 2 / 1 positions. A chain launch costs
+// the same up to 64 positions, the tiles by pass: about 4 units a tile of 8, 5 a smaller one; int4
+// chains pay more to convert their weights. Prompts of 24 layers, ms, tiles | chain: int8 10
+// positions 1.82 | 2.12, 11 2.23 | 2.14, 16 1.90 | 2.18, 20 2.36 | 2.24, 24 2.15 | 2.26, 32 2.50 |
+// 2.30, 64 3.82 | 2.42; int4 16 1.82 | 2.40, 20 2.37 | 2.43, 23 3.08 | 2.47, 28 2.63 | 2.54, 32
+// 2.35 | 2.56, 48 2.89 | 2.64; f16 16 1.95 | 2.23, 20 2.39 | 2.28, 24 2.16 | 2.29, 32 2.55 | 2.37.
+static bool chain_pays(int format, int seq) {
+  const int tiles = 4 * (seq / 8) + 5 * __builtin_popcount(seq & 7);
+  return seq > 8 && tiles > (format == QH_FMT_INT4 ? 16 : 12);
+}
 
 int prefill_chunk(const ModelDev& m, const CacheDev& c) {
   int p = c.capacity < kPrefillChunk ? c.capacity : kPrefillChunk;
@@ -319,7 +328,7 @@ static hipError_t matmul(hipStream_t s, const ModelDev& m, int mode, const DMat&
   if (mode == QH_MATMUL_MFMA && matmul_prefill_supported(w))
     return launch_matmul_prefill(s, w, x, bias, y, seq, p.scratch, p.scratch_bytes);
   if (m.numerics == QH_NUMERICS_FAST) {
-    if (seq >= kChainMinSeq)
+    if (chain_pays(w.format, seq))
       return launch_chain_f32(s, w, x, bias, y, seq, static_cast<float*>(p.scratch), p.scratch_bytes);
     return launch_matvec_f32(s, w, x, bias, y, seq);
   }
@@ -404,7 +413,8 @@ static bool chain_layers_supported(const ModelDev& m) {
 hipError_t enqueue_prefill_layers(hipStream_t s, const ModelDev& m, const CacheDev& c, const PrefillDev& p,
                                   int mode, int past, int seq) {
   if (mode == QH_MATMUL_MFMA && all_mfma(m)) return prefill_layers_mfma(s, m, c, p, past, seq);
-  if (mode != QH_MATMUL_MFMA && m.numerics == QH_NUMERICS_FAST && seq >= kChainMinSeq && chain_layers_supported(m))
+  if (mode != QH_MATMUL_MFMA && m.numerics == QH_NUMERICS_FAST && chain_pays(m.layers_host[0].gu.format, seq) &&
+      chain_layers_supported(m))
     return prefill_layers_chain(s, m, c, p, past, seq);
   hipError_t e;
   const int d = m.hidden, kvd = m.kv_heads * m.head_dim, f = m.intermediate;

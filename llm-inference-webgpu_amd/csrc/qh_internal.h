@@ -110,8 +110,10 @@ hipError_t launch_chain_roots(hipStream_t s, const DMat& m, const float* x, cons
                               float* part, size_t part_bytes, ChainOut* out);
 size_t chain_partials_bytes(const DMat& m, int seq);
 // launch_matvec's sums, bit for bit, on the f64 matrix cores (chain.hip), from kChain64MinSeq
-// positions and for 16-byte aligned x.
-constexpr int kChain64MinSeq = 8;
+// positions and for 16-byte aligned x. 896 columns, int8 | int4, 4864 rows, us, k_matvec's tiles
+// against it: 4 positions 12.4 / 12.0 | 15.8 / 12.9 (128 rows 6.3 / 8.1 | 8.4 / 9.5), 6 positions
+// 19.6 / 12.0 | 26.0 / 12.9 (128 rows 10.4 / 8.1 | 13.9 / 9.5), 8 positions 20.7 / 12.0 | 26.6 / 12.9.
+constexpr int kChain64MinSeq = 6;
 bool chain_f64_supported(const DMat& m, const float* x, int seq);
 hipError_t launch_chain_f64(hipStream_t s, const DMat& m, const float* x, const float* bias, float* y, int seq);
 size_t chain_partials_bound(const DMat& m, int P);
