@@ -174,12 +174,11 @@ __device__ __forceinline__ uint32_t code_int4(float x, double inverse, double ze
 // the f64 product t the expressions above round by at most |t| 2^-23 (the two roundings to f32,
 // 2^-24 each relative; f32(inverse) is never subnormal: |x| < 2^128 bounds the scale), and
 // |t| <= 16 (int4) or 128 (int8). So wherever t32 lies farther than kSafe from every
-// half-integer, t rounds half away from zero to the integer nearest t32; where some value of a
-// chunk lies nearer a half-integer, or is NaN or infinite, the f64 expression decides the whole
-// chunk. The codes are those of the f64 expressions bit for bit, at a fraction of their arithmetic
-// and without a branch per value: a chunk costs one test (int4 of 233472 x 896 bf16 values
-// 173 -> 145 us with the packed ranges and the shared parameters
-// below, still bound by the vector unit: ~25 instructions a value before, ~13 now).
+// half-integer, t rounds half away from zero to the integer nearest t32; nearer a half-integer,
+// and for NaN or an infinite t32, the f64 expression decides. The codes are those of the f64
+// expressions bit for bit, at a fraction of their arithmetic. int4 of bf16 tests each value, of
+// f32 each chunk of four values (65536 x 1792: bf16 76 us by value, 88 by chunk of eight; f32 112
+// by value, 105 by chunk).
 constexpr float kSafeInt4 = 0x1p-16f;  // > 16 * 2^-23
 constexpr float kSafeInt8 = 0x1p-13f;  // > 128 * 2^-23
 // The nearest integer to x * inv32, and whether t32 is too near a half-integer (or NaN).
@@ -207,16 +206,29 @@ __device__ __forceinline__ uint32_t codes_int8(const u32x4& c, int j0, float inv
   }
   return w;
 }
-// A chunk's codes (8 or 4 nibbles, value 0 lowest) where `unsafe` stays false, for values without
-// NaN or infinity. zf: the zero point, an integer in [0, 15], added before rounding (exactly what
-// adding it after gives, farther than kSafeInt4 from a half-integer: t32 + zf is off by 2^-20 more).
-template <bool BF16>
-__device__ __forceinline__ uint32_t codes_int4(const u32x4& c, float inv32, float zf, bool& unsafe) {
+// A bf16 chunk's eight codes as nibbles, value 0 lowest; zf: the zero point, an integer in
+// [0, 15], or NaN.
+__device__ __forceinline__ uint32_t codes_int4_bf16(const u32x4& c, float inv32, double inverse, float zf) {
+  uint32_t w = 0;
+#pragma unroll
+  for (int j = 0; j < 8; j++) {
+    const float x = Chunk<true>::at(c, j);
+    bool unsafe = false;
+    const float r = nearest(x, inv32, kSafeInt4, unsafe);
+    w |= (unsafe ? code_int4(x, inverse, (double)zf)
+                 : (uint32_t)fminf(fmaxf(r + zf, 0.f), 15.f)) << (4 * j);  // small integers: exact
+  }
+  return w;
+}
+// An f32 chunk's four codes where `unsafe` stays false, for values without NaN or infinity. The
+// zero point is added before rounding (exactly what adding it after gives, farther than kSafeInt4
+// from a half-integer: t32 + zf is off by 2^-20 more).
+__device__ __forceinline__ uint32_t codes_int4_f32(const u32x4& c, float inv32, float zf, bool& unsafe) {
   uint32_t w = 0;
   float far = 0.f;
 #pragma unroll
-  for (int j = 0; j < Chunk<BF16>::kVals; j += 2) {
-    const float a = fmaf(Chunk<BF16>::at(c, j), inv32, zf), b = fmaf(Chunk<BF16>::at(c, j + 1), inv32, zf);
+  for (int j = 0; j < 4; j += 2) {
+    const float a = fmaf(Chunk<false>::at(c, j), inv32, zf), b = fmaf(Chunk<false>::at(c, j + 1), inv32, zf);
     const float ra = __builtin_rintf(a), rb = __builtin_rintf(b);
     far = fmaxf(far, fmaxf(fabsf(a - ra), fabsf(b - rb)));
     // an integer in [0, 255]
@@ -226,10 +238,9 @@ __device__ __forceinline__ uint32_t codes_int4(const u32x4& c, float inv32, floa
   unsafe |= !(far <= 0.5f - kSafeInt4);
   return w;
 }
-template <bool BF16>
 __device__ __forceinline__ uint32_t codes_int4_f64(const u32x4& c, double inverse, float zf) {
   uint32_t w = 0;
-  for (int j = 0; j < Chunk<BF16>::kVals; j++) w |= code_int4(Chunk<BF16>::at(c, j), inverse, (double)zf) << (4 * j);
+  for (int j = 0; j < 4; j++) w |= code_int4(Chunk<false>::at(c, j), inverse, (double)zf) << (4 * j);
   return w;
 }
 template <bool BF16>
@@ -366,7 +377,10 @@ __global__ __launch_bounds__(kQBlock) void k_quant_int4_rows(const void* __restr
     }
   }
   // Lane l collects the range of group l % gpr of row l / gpr.
-  const int own_row = lane / gpr, own = lane - own_row * gpr;
+  int own_row = 0;
+#pragma unroll
+  for (int r = 1; r <= R; r++) own_row += lane >= r * gpr ? 1 : 0;
+  const int own = lane - own_row * gpr;
   const int own_step = own >> lp, from = (own & ((1 << lp) - 1)) << lg;
   uint32_t odd = 0;  // chunks with a NaN somewhere in the wave
   float glo = INFINITY, ghi = -INFINITY;
@@ -402,7 +416,7 @@ __global__ __launch_bounds__(kQBlock) void k_quant_int4_rows(const void* __restr
     ginv32 = (float)ginverse;
     if (scale != 0) gzero = (float)zero;  // an integer in [0, 15], or NaN
   }
-  // An infinite range, or one whose f32 inverse overflows: f32 products may be NaN.
+  // An infinite range, or one whose f32 inverse overflows: a chunk's f32 products may be NaN.
   const bool infinite = __any(gzero != -1.f && (ginverse == 0 || ginv32 == INFINITY));
 #pragma unroll
   for (int r = 0; r < R; r++) {
@@ -412,11 +426,17 @@ __global__ __launch_bounds__(kQBlock) void k_quant_int4_rows(const void* __restr
       if (MAXC > 2 && k >= steps) continue;
       const int ci = lane + 64 * k, owner = r * gpr + min(ci >> lg, gpr - 1);  // the chunk's group (clamped past the row)
       const float inv32 = __shfl(ginv32, owner), zf = __shfl(gzero, owner);
-      bool unsafe = infinite || (odd >> (r * MAXC + k) & 1);
-      uint32_t w = codes_int4<BF16>(c[r][k], inv32, zf, unsafe);
-      if (__any(unsafe)) {  // wave-uniform, for the shuffle
+      uint32_t w = 0;
+      if constexpr (BF16) {
         const double inverse = __shfl(ginverse, owner);
-        if (unsafe) w = codes_int4_f64<BF16>(c[r][k], inverse, zf);
+        if (zf != -1.f) w = codes_int4_bf16(c[r][k], inv32, inverse, zf);
+      } else {
+        bool unsafe = infinite || (odd >> (r * MAXC + k) & 1);
+        w = codes_int4_f32(c[r][k], inv32, zf, unsafe);
+        if (__any(unsafe)) {  // wave-uniform, for the shuffle
+          const double inverse = __shfl(ginverse, owner);
+          if (unsafe) w = codes_int4_f64(c[r][k], inverse, zf);
+        }
       }
       if (ci < nchunks && row0 + r < rows) store_int4<BF16>(out, ci, zf == -1.f ? 0u : w);
     }
@@ -460,9 +480,14 @@ __global__ __launch_bounds__(kQBlock) void k_quant_int4_steps(const void* __rest
     }
     const double inverse = 1 / scale;
     const float inv32 = (float)inverse;
-    bool unsafe = odd || inverse == 0 || inv32 == INFINITY;  // f32 products may be NaN
-    uint32_t w = codes_int4<BF16>(c[k], inv32, (float)zero, unsafe);
-    if (unsafe) w = codes_int4_f64<BF16>(c[k], inverse, (float)zero);
+    uint32_t w = 0;
+    if constexpr (BF16) {
+      if (scale != 0) w = codes_int4_bf16(c[k], inv32, inverse, (float)zero);
+    } else {
+      bool unsafe = odd || inverse == 0 || inv32 == INFINITY;  // f32 products may be NaN
+      w = codes_int4_f32(c[k], inv32, (float)zero, unsafe);
+      if (unsafe) w = codes_int4_f64(c[k], inverse, (float)zero);
+    }
     store_int4<BF16>(out, ci, scale != 0 ? w : 0u);
   }
 }
@@ -531,7 +556,7 @@ bool aligned(const void* p, size_t a) { return reinterpret_cast<uintptr_t>(p) % 
 // Chunks per lane of the row-per-wave kernels for `nchunks` chunks a row; 0 when too many.
 int chunks_per_lane(int nchunks) {
   const int per = (nchunks + 63) / 64;
-  return per <= 2 ? 2 : per <= 4 ? 4 : per <= 8 ? 8 : per <= 16 ? 16 : 0;
+  return per <= 1 ? 1 : per <= 2 ? 2 : per <= 4 ? 4 : per <= 8 ? 8 : per <= 16 ? 16 : 0;
 }
 
 template <bool BF16, int MAXC>
@@ -539,18 +564,25 @@ void launch_int8_rows(hipStream_t s, const void* src, int rows, int cols, int8_t
   hipLaunchKernelGGL((k_quant_int8_rows<BF16, MAXC>), dim3((rows + 3) / 4), dim3(kQBlock), 0, s, src, rows, cols, q,
                      scales);
 }
+// Rows from which a wave takes several: below, the rows after the first only wait for it. bf16 to
+// int4, us, one row a wave | four: 896 x 896 3.8 | 7.7, 8192 x 896 8.1 | 9.3, 16384 x 896 14.1 |
+// 14.5, 16384 x 512 9.0 | 8.2, 65536 x 896 45.7 | 41.0, 233472 x 896 146 | 126.
+constexpr int kSharedRows = 16384;
 template <bool BF16, int MAXC, int R>
 void launch_int4_rows(hipStream_t s, const void* src, int rows, int cols, int G, uint8_t* q, float* scales,
                       float* zeros) {
-  // Rows together while their groups fit the wave's lanes (R rows of MAXC chunks a lane are 8 to
-  // 16 loads in flight); more than 64 groups a row go step by step.
+  // R rows a wave where there are waves enough without (kSharedRows) and their groups fit the
+  // wave's lanes; more than 64 groups a row go step by step.
   const int gpr = cols / Chunk<BF16>::kVals / G;
   const auto blocks = [&](int r) { return dim3((rows + 4 * r - 1) / (4 * r)); };
   int lg = 0;
   while ((1 << lg) < G) lg++;
   constexpr int kLg = BF16 ? 4 : 5;  // chunks of a 128-column group
-  if (R * gpr <= 64 && lg == kLg)
+  if (R > 1 && R * gpr <= 64 && lg == kLg && rows >= kSharedRows)
     hipLaunchKernelGGL((k_quant_int4_rows<BF16, MAXC, R, kLg>), blocks(R), dim3(kQBlock), 0, s, src, rows, cols, lg,
+                       q, scales, zeros);
+  else if (gpr <= 64 && lg == kLg)
+    hipLaunchKernelGGL((k_quant_int4_rows<BF16, MAXC, 1, kLg>), blocks(1), dim3(kQBlock), 0, s, src, rows, cols, lg,
                        q, scales, zeros);
   else if (gpr <= 64)
     hipLaunchKernelGGL((k_quant_int4_rows<BF16, MAXC, 1, -1>), blocks(1), dim3(kQBlock), 0, s, src, rows, cols, lg, q,
@@ -587,7 +619,7 @@ hipError_t convert_t(hipStream_t s, const void* src, int rows, int cols, int for
     case QH_FMT_INT8: {
       int8_t* q = static_cast<int8_t*>(data);
       if (maxc && aligned(data, BF16 ? 8 : 4)) {
-        if (maxc == 2) launch_int8_rows<BF16, 2>(s, src, rows, cols, q, scales);
+        if (maxc <= 2) launch_int8_rows<BF16, 2>(s, src, rows, cols, q, scales);
         else if (maxc == 4) launch_int8_rows<BF16, 4>(s, src, rows, cols, q, scales);
         else if (maxc == 8) launch_int8_rows<BF16, 8>(s, src, rows, cols, q, scales);
         else launch_int8_rows<BF16, 16>(s, src, rows, cols, q, scales);
@@ -600,7 +632,8 @@ hipError_t convert_t(hipStream_t s, const void* src, int rows, int cols, int for
       uint8_t* q = static_cast<uint8_t*>(data);
       const int G = group / kVals;
       if (maxc && group % kVals == 0 && G <= 64 && (G & (G - 1)) == 0 && aligned(data, BF16 ? 4 : 2)) {
-        if (maxc == 2) launch_int4_rows<BF16, 2, 4>(s, src, rows, cols, G, q, scales, zeros);
+        if (maxc == 1) launch_int4_rows<BF16, 1, 4>(s, src, rows, cols, G, q, scales, zeros);
+        else if (maxc == 2) launch_int4_rows<BF16, 2, 4>(s, src, rows, cols, G, q, scales, zeros);
         else if (maxc == 4) launch_int4_rows<BF16, 4, 2>(s, src, rows, cols, G, q, scales, zeros);
         else if (maxc == 8) launch_int4_rows<BF16, 8, 1>(s, src, rows, cols, G, q, scales, zeros);
         else launch_int4_rows<BF16, 16, 1>(s, src, rows, cols, G, q, scales, zeros);

@@ -282,3 +282,66 @@ def test_int4_shared_parameters_match_oracle(ctx, hip, src, rows, cols, group):
     np.testing.assert_array_equal(bits32(zeros.read(np.float32, z.size)), bits32(z).reshape(-1))
     for b in (d, data, scales, zeros):
         b.free()
+
+
+@pytest.mark.parametrize("src", ["bf16", "f32"])
+@pytest.mark.parametrize("rows,cols,group", [
+    (5, 512, 128),        # one chunk a lane (f32: two), a row a wave
+    (7, 256, 32),
+    (16383, 128, 128),    # the last row count that keeps a row a wave
+    (16387, 256, 128),    # four rows a wave, the last wave three rows
+    (16385, 640, 128),    # the last wave one row
+    (16386, 1280, 128),   # bf16: two rows a wave
+])
+def test_int4_rows_a_wave_match_oracle(ctx, hip, src, rows, cols, group):
+    """A row a wave for few rows, several from 16384 on, with special groups beside plain ones at
+    both ends of the matrix."""
+    rng = np.random.default_rng(rows * cols)
+    w = (rng.standard_normal((rows, cols)) * 0.02).astype(np.float32)
+    g = w.reshape(-1, group)
+    g[0] = 0.0
+    g[1, 5] = np.inf
+    g[3] = np.where(np.arange(group) % 3 == 0, 0.0, np.sign(g[3]) * np.float32(9.2e-41))
+    g[-3] = np.abs(g[-3])
+    g[-2, 7] = -np.inf
+    g[-1, ::3] = np.nan
+    if src == "bf16":
+        host = (w.view(np.uint32) >> 16).astype(np.uint16)
+        fmt, wide = hip.FMT_BF16, O.bf16_to_f32(host)
+    else:
+        fmt, host, wide = hip.FMT_F32, w, w
+    d = ctx.upload(host)
+    data, scales, zeros = ctx.quantize(d, fmt, rows, cols, hip.FMT_INT4, group)
+    q, s, z = O.quantize_int4(wide, group)
+    np.testing.assert_array_equal(data.read(np.uint8, rows * cols // 2), np.asarray(q).reshape(-1))
+    np.testing.assert_array_equal(bits32(scales.read(np.float32, s.size)), bits32(s).reshape(-1))
+    np.testing.assert_array_equal(bits32(zeros.read(np.float32, z.size)), bits32(z).reshape(-1))
+    for b in (d, data, scales, zeros):
+        b.free()
+
+
+def test_int4_conversion_of_few_rows_costs_what_int8_costs(ctx, hip):
+    """A projection's 896 rows are far fewer than the chip's waves: several rows a wave would leave
+    each row's chain waiting for the one before it (twice int8's time where both are one launch)."""
+    rows = cols = 896
+    d = ctx.upload(np.random.default_rng(3).standard_normal((rows, cols)).astype(np.float32).view(np.uint16)[:, 1::2].copy())
+    outs = {f: ctx.quantize(d, hip.FMT_BF16, rows, cols, f, g) for f, g in ((hip.FMT_INT8, 0), (hip.FMT_INT4, 128))}
+
+    def best(fmt, group):
+        bufs = outs[fmt]
+        a, b, least = ctx.event(), ctx.event(), 1e9
+        for _ in range(10):
+            ctx.record(a)
+            for _ in range(50):
+                ctx.quantize(d, hip.FMT_BF16, rows, cols, fmt, group, *bufs)
+            ctx.record(b)
+            least = min(least, ctx.elapsed_ms(a, b))
+        ctx.destroy_event(a)
+        ctx.destroy_event(b)
+        return least
+    assert best(hip.FMT_INT4, 128) < 1.5 * best(hip.FMT_INT8, 0)
+    for bufs in outs.values():
+        for x in bufs:
+            if x is not None:
+                x.free()
+    d.free()
