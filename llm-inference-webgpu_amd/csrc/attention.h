@@ -33,6 +33,8 @@
 // products (k_flash_prefill) serves the MFMA prompt path.
 #pragma once
 
+#include <algorithm>
+
 #include "device_common.h"
 
 namespace qh {
@@ -278,16 +280,25 @@ static __global__ __launch_bounds__(kAttnThreads) void k_attn_block(ExactArgs a)
 // queries do not see, are summed on the vector unit under each query's own bound.
 //
 // Bound: latency of its three phases (f64 products, f64 exponentials, then a chain of ctx / 4
-// products per 16 dimensions); a tile takes 16 x CTX scores of LDS, so several tiles share a CU,
-// where k_attn_block's one wave summed alone on a CU per (query, head). Tiles are launched
-// heaviest first. 512 queries, 14 heads: 182 -> 36 us.
+// products per 16 dimensions), paid once for 16 queries where k_attn_block pays them per query.
+// One block of eight waves per CU (142 VGPRs; 51 to 150 KB of LDS by CTX). Tiles are launched
+// heaviest first. 512 queries, 14 heads: 182 -> 35 us.
 typedef double f64x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4t __attribute__((ext_vector_type(4)));
 constexpr int kTileQ = 16;
 constexpr int kTileThreads = 512, kTileWaves = kTileThreads / kWave;
 static_assert(kTileThreads == kAttnThreads, "the softmax sum's thread order");
 constexpr int kTileCtx = 2048;     // the widest tile: 16 x 2052 floats of LDS
+// A tile takes as long as two to three k_attn_block blocks one after another, so tiles serve the
+// prompts whose (query, head) blocks would run in more than two rounds of one per CU (up to two and
+// a half in short contexts, where many queries' blocks differ in length and fill a third round).
+// Blocks | tiles, us, queries x heads after a past: 16 x 14 after 1980 31.5 | 72.6; 32 x 14 after 0 8.3 | 11.0, after 1000 36.0 | 42.9;
+// 128 x 4 after 496 28.7 | 30.0; 320 x 2 after 0 17.5 | 20.1; 160 x 4 after 128 18.8 | 20.0; 44 x 14
+// after 128 16.1 | 15.1; 48 x 14 after 496 36.9 | 26.7; 64 x 14 after 1980 100.8 | 73.0.
 constexpr int kTileMinSeq = 16;
+inline bool attn_tile_pays(int seq, int heads, int total) {
+  return seq >= kTileMinSeq && (long)seq * heads > 512 + (total <= 512 ? std::min(seq, 128) : 0);
+}
 
 // Element 4s + g of 16 f16 values (s = 0..3) in two 16-byte words.
 __device__ __forceinline__ float tile_f16(const v4u (&u)[2], int s, int g) {
@@ -619,12 +630,12 @@ static __global__ __launch_bounds__(kBlock) void k_attn_exact(ExactArgs a) {
 }
 
 // Exact attention of `seq` queries over past + seq positions: query tiles for prompts that fit
-// them, else a (query, head) block up to kPLds positions -- of context for the operator, of
+// and fill them (attn_tile_pays), else a (query, head) block up to kPLds positions -- of context for the operator, of
 // capacity for the model (`limit`), whose decode step picks by capacity -- else spans. All
 // evaluate a query alike.
 static inline hipError_t launch_attn_exact(hipStream_t s, const ExactArgs& a, int seq, int limit, int spans) {
   const int total = a.past + seq;
-  if (seq >= kTileMinSeq && total <= kTileCtx && limit <= kPLds) {
+  if (attn_tile_pays(seq, a.heads, total) && total <= kTileCtx && limit <= kPLds) {
     const dim3 grid((seq + kTileQ - 1) / kTileQ * a.heads), block(kTileThreads);
     if (total <= 512) hipLaunchKernelGGL(k_attn_tile<512>, grid, block, 0, s, a, seq);
     else if (total <= 1024) hipLaunchKernelGGL(k_attn_tile<1024>, grid, block, 0, s, a, seq);
