@@ -15,6 +15,7 @@
 // contracted: activations as f32 with their chunk sums, weights as stored (converted in
 // registers: a conversion feeds 32 positions). The tree's pending subtrees stay in registers.
 #include <algorithm>
+#include <type_traits>
 
 #include "device_common.h"
 
@@ -401,10 +402,11 @@ hipError_t launch_chain_f32(hipStream_t s, const DMat& m, const float* x, const 
 //
 // Bound: the f64 matrix rate (70 TFLOP/s in a large product), which the vector unit's f64 shares
 // with everything else it does; what the VALU form lost was one LDS read of x per two products
-// and a dequantized weight per eight positions. A block takes 32 positions x 16 rows, its four
-// waves a quarter of the team's slots each (so 52 positions of a 4864-row matrix are 608 blocks),
-// joined through LDS in tree order. A wave stages its own slabs of x, so no barrier runs in the
-// loop; weights go to registers a chunk ahead. 4864 x 896 int8, 52 positions: 90 -> 23 us.
+// and a dequantized weight per eight positions. A block takes T tiles of 16 positions x 16 rows,
+// its four waves a quarter of the team's slots each (so 52 positions of a 4864-row matrix are 608
+// blocks of two tiles), joined through LDS in tree order. A wave stages its own slabs of x, so no
+// barrier runs in the loop; weights go to registers a chunk ahead. 4864 x 896 int8, 52 positions:
+// 90 -> 23 us.
 typedef double f64x4 __attribute__((ext_vector_type(4)));
 
 template <int FMT>
@@ -415,7 +417,7 @@ struct Chain64 {
   static constexpr int kXRow = kK + 4;
   static constexpr int kLevels = FMT == QH_FMT_INT4 ? 3 : 2;  // log2 of a wave's groups, 16 slots at most
 };
-constexpr int kChain64M = 32, kChain64N = 16;
+constexpr int kChain64M = 16, kChain64N = 16;  // a tile's positions and rows
 
 // One chunk of one row as the loader's f32 weights: w(s) is the lane's element 4s + g.
 template <int FMT>
@@ -448,39 +450,41 @@ struct RowChunk {
   }
 };
 
-// acc[tile] += one chunk for 16 rows x two tiles of 16 positions (`two`: the second has any).
+// acc[tile] += one chunk for 16 rows x T tiles of 16 positions (`two`: the second has any).
 // Accumulator register r holds position 4r + lane / 16, row lane % 16.
-template <int FMT, int STEPS, int K = 0>
-__device__ __forceinline__ void chain64_steps(const RowChunk<FMT>& rc, const float (&xv)[2][STEPS], int g, bool two,
-                                              f64x4 (&acc)[2]) {
+template <int FMT, int STEPS, int T, int K = 0>
+__device__ __forceinline__ void chain64_steps(const RowChunk<FMT>& rc, const float (&xv)[T][STEPS], int g, bool two,
+                                              f64x4 (&acc)[T]) {
   if constexpr (K < STEPS) {
     const double w = rc.template at<K>(g);
     acc[0] = __builtin_amdgcn_mfma_f64_16x16x4f64((double)xv[0][K], w, acc[0], 0, 0, 0);
-    if (two) acc[1] = __builtin_amdgcn_mfma_f64_16x16x4f64((double)xv[1][K], w, acc[1], 0, 0, 0);
-    chain64_steps<FMT, STEPS, K + 1>(rc, xv, g, two, acc);
+    if constexpr (T == 2) {
+      if (two) acc[1] = __builtin_amdgcn_mfma_f64_16x16x4f64((double)xv[1][K], w, acc[1], 0, 0, 0);
+    }
+    chain64_steps<FMT, STEPS, T, K + 1>(rc, xv, g, two, acc);
   }
 }
 
-template <int FMT, bool MULTI>
+template <int FMT, bool MULTI, int T>
 __global__ __launch_bounds__(kBlock, 2) void k_chain_f64(ChainArgs a) {
   using F = Chain64<FMT>;
-  constexpr int S = F::kS, kLoads = kChain64M * F::kK / 4 / kWave;
+  constexpr int S = F::kS, kLoads = T * kChain64M * F::kK / 4 / kWave;
   // A wave's slab of x (its LDS operations run in order, so the next slab is stored over it after
   // its reads), then its sums [tile][register][lane].
-  __shared__ __attribute__((aligned(16))) float xs[kBlock / kWave][kChain64M * F::kXRow];
-  static_assert(2 * 4 * kWave * 2 <= kChain64M * F::kXRow, "the sums fit the slab");
+  __shared__ __attribute__((aligned(16))) float xs[kBlock / kWave][T * kChain64M * F::kXRow];
+  static_assert(2 * 4 * kWave <= kChain64M * F::kXRow, "the sums fit the slab");
   const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave, n = lane & 15, g4 = lane >> 4;
-  const int row0 = blockIdx.x * kChain64N, pos0 = blockIdx.y * kChain64M;
+  const int row0 = blockIdx.x * kChain64N, pos0 = blockIdx.y * (T * kChain64M);
   const int nc = a.m.nchunks, slots = a.tl / (kBlock / kWave), first = wave * slots, groups = slots / S;
   const int row = min(row0 + n, a.m.rows - 1);
-  const bool two = pos0 + 16 < a.seq;  // uniform: the second position tile has any
+  const bool two = T == 2 && pos0 + 16 < a.seq;  // uniform: the second position tile has any
   const v4u* rp = reinterpret_cast<const v4u*>(a.m.data + (size_t)row * a.m.row_bytes);
   const float srow = FMT == QH_FMT_INT8 ? a.m.scales[row] : 0.f;
   auto slabs_of = [&](int g) {
     const int c = first + g * S;
     return c < nc ? (MULTI ? (nc - 1 - c) / a.tl + 1 : 1) : 0;
   };
-  // x of a slab: 32 positions x kK columns, one float4 per lane and load.
+  // x of a slab: 16 T positions x kK columns, one float4 per lane and load.
   v4f xr[kLoads];
   v4u wr[S];
   float sr[S], zr[S];
@@ -517,18 +521,18 @@ __global__ __launch_bounds__(kBlock, 2) void k_chain_f64(ChainArgs a) {
       d[12] = xr[j].w;
     }
   };
-  f64x4 st[F::kLevels][2], root[2];
+  f64x4 st[F::kLevels][T], root[T];
   if (slabs_of(0) > 0) {
     load(first);
     store(xs[wave]);
   }
 #pragma unroll 1
   for (int g = 0; g < groups; g++) {
-    f64x4 acc[S][2];
+    f64x4 acc[S][T];
 #pragma unroll
     for (int i = 0; i < S; i++)
 #pragma unroll
-      for (int t = 0; t < 2; t++) acc[i][t] = (f64x4){0.0, 0.0, 0.0, 0.0};
+      for (int t = 0; t < T; t++) acc[i][t] = (f64x4){0.0, 0.0, 0.0, 0.0};
     const int ns = slabs_of(g);
 #pragma unroll 1
     for (int j = 0; j < ns; j++) {
@@ -545,9 +549,9 @@ __global__ __launch_bounds__(kBlock, 2) void k_chain_f64(ChainArgs a) {
       for (int i = 0; i < S; i++) {
         if (c0 + i < nc) {
           constexpr int kSteps = F::kW / 4;
-          float xv[2][kSteps];
+          float xv[T][kSteps];
 #pragma unroll
-          for (int t = 0; t < 2; t++) {
+          for (int t = 0; t < T; t++) {
             const float* xp = xb + (16 * t + n) * F::kXRow + 4 * g4;
             if constexpr (FMT == QH_FMT_F16) {
               const float2 v = *reinterpret_cast<const float2*>(xp + 16 * (i >> 1) + 2 * (i & 1));
@@ -562,7 +566,7 @@ __global__ __launch_bounds__(kBlock, 2) void k_chain_f64(ChainArgs a) {
               }
             }
           }
-          chain64_steps<FMT, kSteps>(rc[i], xv, g4, two, acc[i]);
+          chain64_steps<FMT, kSteps, T>(rc[i], xv, g4, two, acc[i]);
         }
       }
       __builtin_amdgcn_wave_barrier();
@@ -573,33 +577,33 @@ __global__ __launch_bounds__(kBlock, 2) void k_chain_f64(ChainArgs a) {
 #pragma unroll
       for (int i = 0; i < S; i += 2 * w)
 #pragma unroll
-        for (int t = 0; t < 2; t++) acc[i][t] += acc[i + w][t];
+        for (int t = 0; t < T; t++) acc[i][t] += acc[i + w][t];
     bool open = true;
 #pragma unroll
-    for (int t = 0; t < 2; t++) root[t] = acc[0][t];
+    for (int t = 0; t < T; t++) root[t] = acc[0][t];
 #pragma unroll
     for (int lv = 0; lv < F::kLevels; lv++) {
       if (open) {
         if (g >> lv & 1) {
 #pragma unroll
-          for (int t = 0; t < 2; t++) root[t] = st[lv][t] + root[t];
+          for (int t = 0; t < T; t++) root[t] = st[lv][t] + root[t];
         } else {
 #pragma unroll
-          for (int t = 0; t < 2; t++) st[lv][t] = root[t];
+          for (int t = 0; t < T; t++) st[lv][t] = root[t];
           open = false;
         }
       }
     }
   }
 #pragma unroll
-  for (int t = 0; t < 2; t++)
+  for (int t = 0; t < T; t++)
 #pragma unroll
     for (int r = 0; r < 4; r++) reinterpret_cast<double*>(xs[wave])[(t * 4 + r) * kWave + lane] = root[t][r];
   __syncthreads();
-  // Wave w finishes register w of both tiles: position 16t + 4r + lane / 16, row lane % 16.
+  // Wave w finishes register w of each tile: position 16t + 4r + lane / 16, row lane % 16.
   if (row0 + n >= a.m.rows) return;
 #pragma unroll
-  for (int t = 0; t < 2; t++) {
+  for (int t = 0; t < T; t++) {
     const int p = pos0 + 16 * t + 4 * wave + g4;
     if (p < a.seq) {
       double q[kBlock / kWave];
@@ -623,16 +627,25 @@ hipError_t launch_chain_f64(hipStream_t s, const DMat& m, const float* x, const 
   a.y = y;
   a.seq = seq;
   a.tl = team_width(m.nchunks);
-  const dim3 grid((m.rows + kChain64N - 1) / kChain64N, (seq + kChain64M - 1) / kChain64M);
+  const int rows = (m.rows + kChain64N - 1) / kChain64N, tiles = (seq + kChain64M - 1) / kChain64M;
   const bool multi = m.nchunks > a.tl;
+  // A tile a block where each CU then has at most one: two a block would leave CUs idle and take a
+  // third longer (24 positions, us, two | one: 128 x 896 f16 12.0 | 8.5, 30 x 4864 int4 54.8 | 35.0).
+  const int t = tiles > 1 && rows * tiles > 256 ? 2 : 1;
+  const dim3 grid(rows, (tiles + t - 1) / t);
   auto go = [&](auto one, auto many) {
     if (multi) hipLaunchKernelGGL(many, grid, dim3(kBlock), 0, s, a);
     else hipLaunchKernelGGL(one, grid, dim3(kBlock), 0, s, a);
   };
+  auto fmt = [&](auto f) {
+    constexpr int F = decltype(f)::value;
+    if (t == 2) go(k_chain_f64<F, false, 2>, k_chain_f64<F, true, 2>);
+    else go(k_chain_f64<F, false, 1>, k_chain_f64<F, true, 1>);
+  };
   switch (m.format) {
-    case QH_FMT_F16: go(k_chain_f64<QH_FMT_F16, false>, k_chain_f64<QH_FMT_F16, true>); break;
-    case QH_FMT_INT8: go(k_chain_f64<QH_FMT_INT8, false>, k_chain_f64<QH_FMT_INT8, true>); break;
-    default: go(k_chain_f64<QH_FMT_INT4, false>, k_chain_f64<QH_FMT_INT4, true>); break;
+    case QH_FMT_F16: fmt(std::integral_constant<int, QH_FMT_F16>()); break;
+    case QH_FMT_INT8: fmt(std::integral_constant<int, QH_FMT_INT8>()); break;
+    default: fmt(std::integral_constant<int, QH_FMT_INT4>()); break;
   }
   return hipGetLastError();
 }

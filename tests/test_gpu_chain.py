@@ -92,6 +92,42 @@ def test_exact_matvec_on_matrix_cores_equals_single_positions_bitwise(ctx, hip, 
         b.free()
 
 
+@pytest.mark.parametrize("fmt", ["f16", "int8", "int4"])
+@pytest.mark.parametrize("rows,cols,seqs", [
+    (1361, 256, (16, 32, 33, 48)),     # 86 row blocks: 32 positions a tile of 16 per block, 33 two
+    (4097, 1184, (6, 17, 31)),         # 257: two tiles per block from 17 positions
+])
+def test_exact_matvec_tiles_per_block_equal_single_positions_bitwise(ctx, hip, fmt, rows, cols, seqs):
+    """A block takes one or two tiles of 16 positions, by how many blocks there are."""
+    rng = np.random.default_rng(rows)
+    w = (rng.standard_normal((rows, cols)) * 0.02).astype(np.float32)
+    if fmt == "f16":
+        bufs = [ctx.upload(w.astype(np.float16).view(np.uint16))]
+        W = ctx.weight(hip.FMT_F16, rows, cols, bufs[0])
+    elif fmt == "int8":
+        bufs = [ctx.upload(a) for a in hip.quantize_int8(w)]
+        W = ctx.weight(hip.FMT_INT8, rows, cols, *bufs)
+    else:
+        bufs = [ctx.upload(a) for a in hip.quantize_int4(w, 32)]
+        W = ctx.weight(hip.FMT_INT4, rows, cols, *bufs, 32)
+    n = max(seqs)
+    x = rng.standard_normal((n, cols)).astype(np.float32)
+    dy = ctx.empty(n * rows * 4)
+    want = np.empty((n, rows), np.float32)
+    for t in range(n):
+        dx = ctx.upload(x[t])
+        ctx.matvec(W, dx, None, dy, 1)
+        want[t] = dy.read(count=rows)
+        dx.free()
+    dx = ctx.upload(x)
+    for seq in seqs:
+        ctx.matvec(W, dx, None, dy, seq)
+        np.testing.assert_array_equal(dy.read(count=seq * rows).view(np.uint32), want[:seq].reshape(-1).view(np.uint32),
+                                      err_msg=f"{seq} positions")
+    for b in bufs + [dx, dy]:
+        b.free()
+
+
 def test_prompt_attention_past_1024_positions_equals_steps_bitwise(ctx, hip):
     """Slots of several chunks (four states a slot), and the step from one chunk a slot to two, in
     the prompt's merged attention: the decode steps' logits and K/V rows bit for bit."""
