@@ -17,6 +17,8 @@
 // the same bits -- the reference's prefill == incremental decode property
 // (README.md:256-272, web/model.html:169-198). QH_MATMUL_MFMA is held to a stated
 // tolerance instead.
+#include <initializer_list>
+
 #include "attention.h"
 #include "device_common.h"
 #include "model_dev.h"
@@ -173,16 +175,25 @@ __global__ void k_embed_rows(const uint16_t* __restrict__ embed, const int* __re
     rows[(size_t)t * hidden + i] = __builtin_bit_cast(float, (uint32_t)src[i] << 16);
 }
 
-// Whether a batched contraction of `seq` positions runs on the f32 matrix cores (launch_chain_f32,
-// the same bits) or in launch_matvec_f32's tiles of 8 / 4 / 2 / 1 positions. A chain launch costs
-// the same up to 64 positions, the tiles by pass: about 4 units a tile of 8, 5 a smaller one; int4
-// chains pay more to convert their weights. Prompts of 24 layers, ms, tiles | chain: int8 10
-// positions 1.82 | 2.12, 11 2.23 | 2.14, 16 1.90 | 2.18, 20 2.36 | 2.24, 24 2.15 | 2.26, 32 2.50 |
-// 2.30, 64 3.82 | 2.42; int4 16 1.82 | 2.40, 20 2.37 | 2.43, 23 3.08 | 2.47, 28 2.63 | 2.54, 32
-// 2.35 | 2.56, 48 2.89 | 2.64; f16 16 1.95 | 2.23, 20 2.39 | 2.28, 24 2.16 | 2.29, 32 2.55 | 2.37.
-static bool chain_pays(int format, int seq) {
-  const int tiles = 4 * (seq / 8) + 5 * __builtin_popcount(seq & 7);
-  return seq > 8 && tiles > (format == QH_FMT_INT4 ? 16 : 12);
+// Whether batched contractions of `seq` positions run on the f32 matrix cores (launch_chain_f32, the
+// same bits) or in launch_matvec_f32's tiles of 8 / 4 / 2 / 1 positions. A chain launch costs the
+// same up to 64 positions, the tiles by pass: about 4 units a tile of 8, 5 a smaller one; int4
+// chains pay more to convert their weights. Prompts of 24 layers of 896 columns and 4864 ffn rows,
+// ms, tiles | chain: int8 10 positions 1.82 | 2.12, 11 2.23 | 2.14, 16 1.90 | 2.18, 20 2.36 | 2.24,
+// 32 2.50 | 2.30, 64 3.82 | 2.42; int4 16 1.82 | 2.40, 23 3.08 | 2.47, 32 2.35 | 2.56, 48 2.89 | 2.64;
+// f16 20 2.39 | 2.28, 24 2.16 | 2.29, 32 2.55 | 2.37. Narrower matrices leave CUs free for more
+// tiles at once, so the chain also has to be estimated shorter over `matrices` (four layers, us: 512
+// columns and 1536 rows int4 64 positions 315 | 572, 128 and 256 int8 64 209 | 274, 512 positions
+// 334 | 372; the estimates err by a few per cent, and lean to the chain by three).
+static bool chain_pays(std::initializer_list<const DMat*> matrices, int seq) {
+  const int units = 4 * (seq / 8) + 5 * __builtin_popcount(seq & 7);
+  if (seq <= 8 || units <= ((*matrices.begin())->format == QH_FMT_INT4 ? 16 : 12)) return false;
+  float tiles = 0.f, chain = 0.f;
+  for (const DMat* m : matrices) {
+    tiles += matvec_f32_us(*m, seq);
+    chain += chain_f32_us(*m, seq);
+  }
+  return 0.97f * chain < tiles;
 }
 
 int prefill_chunk(const ModelDev& m, const CacheDev& c) {
@@ -328,7 +339,7 @@ static hipError_t matmul(hipStream_t s, const ModelDev& m, int mode, const DMat&
   if (mode == QH_MATMUL_MFMA && matmul_prefill_supported(w))
     return launch_matmul_prefill(s, w, x, bias, y, seq, p.scratch, p.scratch_bytes);
   if (m.numerics == QH_NUMERICS_FAST) {
-    if (chain_pays(w.format, seq))
+    if (chain_pays({&w}, seq))
       return launch_chain_f32(s, w, x, bias, y, seq, static_cast<float*>(p.scratch), p.scratch_bytes);
     return launch_matvec_f32(s, w, x, bias, y, seq);
   }
@@ -413,9 +424,10 @@ static bool chain_layers_supported(const ModelDev& m) {
 hipError_t enqueue_prefill_layers(hipStream_t s, const ModelDev& m, const CacheDev& c, const PrefillDev& p,
                                   int mode, int past, int seq) {
   if (mode == QH_MATMUL_MFMA && all_mfma(m)) return prefill_layers_mfma(s, m, c, p, past, seq);
-  if (mode != QH_MATMUL_MFMA && m.numerics == QH_NUMERICS_FAST && chain_pays(m.layers_host[0].gu.format, seq) &&
-      chain_layers_supported(m))
-    return prefill_layers_chain(s, m, c, p, past, seq);
+  if (mode != QH_MATMUL_MFMA && m.numerics == QH_NUMERICS_FAST && chain_layers_supported(m)) {
+    const LayerDev& l = m.layers_host[0];
+    if (chain_pays({&l.gu, &l.qkv, &l.o, &l.down}, seq)) return prefill_layers_chain(s, m, c, p, past, seq);
+  }
   hipError_t e;
   const int d = m.hidden, kvd = m.kv_heads * m.head_dim, f = m.intermediate;
   const size_t n = (size_t)seq * d;

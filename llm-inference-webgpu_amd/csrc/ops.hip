@@ -243,6 +243,25 @@ static hipError_t matvec_f32_fmt(hipStream_t s, const DMat& m, const float* x, c
   return e;
 }
 
+// A launch of k_matvec_f32: its latency, or its products (a weight's conversion shared by NB
+// positions). Fitted as chain_f32_us is.
+float matvec_f32_us(const DMat& m, int seq) {
+  const float weights = 1e-6f * m.rows * m.cols;
+  float us = 0.f;
+  int done = 0;
+  auto launch = [&](int nb, bool fits) {
+    const int tiles = fits ? (seq - done) / nb : 0;
+    if (tiles == 0) return;
+    us += std::max(3.6f, weights * tiles * (0.08f * nb + 0.07f));
+    done += tiles * nb;
+  };
+  launch(8, f32_tile_fits<8>(m));
+  launch(4, f32_tile_fits<4>(m));
+  launch(2, f32_tile_fits<2>(m));
+  launch(1, true);
+  return us;
+}
+
 bool matvec_f32_supported(const DMat& m) { return f32_tile_fits<1>(m) && m.cols % 4 == 0; }
 
 hipError_t launch_matvec_f32(hipStream_t s, const DMat& m, const float* x, const float* bias, float* y,

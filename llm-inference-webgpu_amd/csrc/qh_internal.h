@@ -109,10 +109,13 @@ struct ChainOut {
 hipError_t launch_chain_roots(hipStream_t s, const DMat& m, const float* x, const float* bias, float* y, int seq,
                               float* part, size_t part_bytes, ChainOut* out);
 size_t chain_partials_bytes(const DMat& m, int seq);
+// About how long launch_chain_f32 and launch_matvec_f32 take, us: what decides between them.
+float chain_f32_us(const DMat& m, int seq);
+float matvec_f32_us(const DMat& m, int seq);
 // launch_matvec's sums, bit for bit, on the f64 matrix cores (chain.hip), from kChain64MinSeq
-// positions and for 16-byte aligned x. 896 columns, int8 | int4, 4864 rows, us, k_matvec's tiles
-// against it: 4 positions 12.4 / 12.0 | 15.8 / 12.9 (128 rows 6.3 / 8.1 | 8.4 / 9.5), 6 positions
-// 19.6 / 12.0 | 26.0 / 12.9 (128 rows 10.4 / 8.1 | 13.9 / 9.5), 8 positions 20.7 / 12.0 | 26.6 / 12.9.
+// positions and for 16-byte aligned x. 896 columns, f16 | int8 | int4, us, k_matvec's tiles / this:
+// 6 positions of 4864 rows 14.5 / 11.7 | 19.5 / 10.2 | 25.7 / 11.2, of 128 rows 10.1 / 8.5 | 10.3 /
+// 7.1 | 13.8 / 7.7; 8 positions of 4864 rows 21.4 / 11.9 | 20.3 / 10.3 | 26.6 / 11.4.
 constexpr int kChain64MinSeq = 6;
 bool chain_f64_supported(const DMat& m, const float* x, int seq);
 hipError_t launch_chain_f64(hipStream_t s, const DMat& m, const float* x, const float* bias, float* y, int seq);

@@ -2,6 +2,8 @@
 step: the same sums in the same order, so a prompt's logits and its f16 K/V rows are those of the
 same positions stepped one at a time, bit for bit -- at the edges of the 64-position and 64-row
 tiles, with one and several splits of the team's slots, ragged last chunks and every format."""
+import time
+
 import numpy as np
 import pytest
 
@@ -150,4 +152,26 @@ def test_prompt_attention_past_1024_positions_equals_steps_bitwise(ctx, hip):
         np.testing.assert_array_equal(p["value"], s["value"])
     cache.destroy()
     steps.destroy()
+    model.destroy()
+
+
+def test_short_prompts_of_a_narrow_model_cost_what_eight_positions_cost(ctx, hip):
+    """64 positions through 512-column int4 layers are one launch of tiles per contraction, as 8 are;
+    on the matrix cores they would take twice as long."""
+    cfg = hip.ModelConfig(hidden=512, intermediate=1536, layers=4, heads=8, kv_heads=2, vocab=1000)
+    model = hip.GpuModel.load(ctx, hip.device_tensors(hip.synthesize_checkpoint(cfg, seed=23), cfg, "int4", 128, "int8"),
+                              cfg, maxPositions=64)
+    ids = hip.synth_tokens(23, "chain.narrow", cfg.vocab, 64)
+    cache = model.newCache(64)
+
+    def best(n):
+        least = 1e9
+        for _ in range(30):
+            cache.length = 0
+            start = time.perf_counter()
+            model.forward_tokens(ids[:n], cache)
+            least = min(least, time.perf_counter() - start)
+        return least
+    assert best(64) < 1.5 * best(8)
+    cache.destroy()
     model.destroy()
