@@ -355,7 +355,10 @@ int qh_decode_prepare(qh_model* m, qh_cache* c);
  * of forward() of one token after another, and h_nll[t] (n - 1 doubles) receives
  * the negative log-likelihood of ids[t+1] under position t's logits, -(l[target] - max - log(sum
  * exp(l - max))) in f64 on the device. Perplexity is exp(mean(h_nll)). The cache advances by
- * n - 1 positions; QH_ERR_RANGE for ids outside the vocabulary or a cache without room. */
+ * n - 1 positions; QH_ERR_RANGE for ids outside the vocabulary or a cache without room.
+ * The first call of several positions allocates what the cache then keeps until it is freed: the
+ * batched forward's workspace, 64 rows of logits (39 MB for 151936 tokens) and a double per
+ * position; without that memory the positions run one step at a time. */
 int qh_score(qh_model* m, qh_cache* c, const int32_t* h_ids, int32_t n, double* h_nll);
 
 /* use_graph = 0: later decodes on this cache enqueue every kernel of a step directly instead

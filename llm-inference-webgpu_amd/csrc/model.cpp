@@ -141,7 +141,7 @@ struct qh_cache {
   qh::PrefillDev pw{};
   qh::PrefillBytes pw_bytes{};
   void* pw_mem = nullptr;
-  int pw_matmul = -1;  // the matmul mode the workspace was last checked for
+  uint32_t pw_modes = 0;  // bit per matmul mode whose needs pw_bytes is known to cover
   // Scoring workspace, kept from the first qh_score: logits of kHeadRows rows, their partials
   // and the scores of a whole cache.
   void* score_mem = nullptr;
@@ -733,17 +733,17 @@ int finish_forward(qh_cache* c, int seq, float* h_logits, int32_t* h_argmax) {
   return QH_OK;
 }
 
-// The batched-prefill workspace for the model's current matmul mode: one allocation,
-// carved in the order prefill_bytes() counts it.
+// The batched-prefill workspace for a matmul mode: one allocation, carved in the order
+// prefill_bytes() counts it.
 int ensure_prefill(qh_cache* c, int matmul) {
   qh_model* m = c->m;
   // The sizes depend on the model, the cache and the matmul mode only: checked once per mode
   // (they walk every layer matrix on the host, in front of the forward's first launch).
-  if (c->pw_mem && c->pw_matmul == matmul) return QH_OK;
+  if (c->pw_mem && (c->pw_modes >> matmul & 1)) return QH_OK;
   qh::PrefillBytes b = qh::prefill_bytes(m->dev, c->dev, matmul);
   if (c->pw_mem && b.floats <= c->pw_bytes.floats && b.counters <= c->pw_bytes.counters &&
       b.scratch <= c->pw_bytes.scratch) {
-    c->pw_matmul = matmul;
+    c->pw_modes |= 1u << matmul;
     return QH_OK;
   }
   b.floats = std::max(b.floats, c->pw_bytes.floats);  // modes in turn keep one workspace
@@ -760,8 +760,8 @@ int ensure_prefill(qh_cache* c, int matmul) {
     return fail(QH_ERR_NOMEM, "prefill workspace of %zu bytes", fbytes + cbytes + b.scratch);
   }
   QH_HIP(hipMemsetAsync(static_cast<char*>(c->pw_mem) + fbytes, 0, cbytes, s));
-  c->pw_bytes = b;
-  c->pw_matmul = matmul;
+  c->pw_bytes = b;  // at least what every mode asked for before
+  c->pw_modes |= 1u << matmul;
   const qh::ModelDev& d = m->dev;
   const size_t P = qh::prefill_chunk(d, c->dev);
   const size_t hd = d.hidden, kv = (size_t)d.kv_heads * d.head_dim, f = d.intermediate;
@@ -977,7 +977,10 @@ int qh_score(qh_model* m, qh_cache* c, const int32_t* h_ids, int32_t n, double* 
   const int total = n - 1;
   const qh::ModelDev& md = m->dev;
   // ids[0..n-2] are fed (teacher-forced); ids[t+1] is scored under position t's logits.
-  if (total >= 2 && ensure_score(c) == QH_OK) {
+  // A single position takes its step, and in exact numerics up to three do, whose batched pass is
+  // no shorter (24 layers of int4, ms, batched | steps: two positions 1.79 | 1.50, three 2.58 | 2.22,
+  // four 2.45 | 2.94; f16 three 2.07 | 2.16, four 1.79 | 2.88).
+  if (total >= (md.numerics == QH_NUMERICS_EXACT ? 4 : 2) && ensure_score(c) == QH_OK) {
     // The positions run as the batched prefill and the head over its rows, kHeadRows at a time:
     // the logits have the bits of one decode step after another.
     char* mem = static_cast<char*>(c->score_mem);
@@ -1007,29 +1010,25 @@ int qh_score(qh_model* m, qh_cache* c, const int32_t* h_ids, int32_t n, double* 
     c->length += total;
     return QH_OK;
   }
-  // A single position, or no memory for the workspace: one decode step after another.
+  // One decode step after another: also where the workspace found no memory.
   (void)hipGetLastError();  // a failed allocation is not the launches' error
-  struct Scratch {
-    int32_t* ids = nullptr;
-    double* nll = nullptr;
-    void* parts = nullptr;
-    ~Scratch() {
-      hipFree(ids);
-      hipFree(nll);
-      hipFree(parts);
-    }
+  struct Scratch {  // scores, partials, ids
+    char* mem = nullptr;
+    ~Scratch() { hipFree(mem); }
   } d;
-  QH_HIP(hipMalloc((void**)&d.ids, (size_t)n * 4));
-  QH_HIP(hipMalloc((void**)&d.nll, (size_t)total * 8));
-  QH_HIP(hipMalloc(&d.parts, qh::nll_partials_bytes(1)));
-  QH_HIP(hipMemcpyAsync(d.ids, h_ids, (size_t)n * 4, hipMemcpyHostToDevice, s));
-  QH_HIP(hipMemcpyAsync(c->dev.tokens + c->length, d.ids, (size_t)total * 4, hipMemcpyDeviceToDevice, s));
+  const size_t nll_bytes = (size_t)total * 8, parts_bytes = qh::nll_partials_bytes(1);
+  QH_HIP(hipMalloc((void**)&d.mem, nll_bytes + parts_bytes + (size_t)n * 4));
+  double* nll = reinterpret_cast<double*>(d.mem);
+  void* parts = d.mem + nll_bytes;
+  int32_t* ids = reinterpret_cast<int32_t*>(d.mem + nll_bytes + parts_bytes);
+  QH_HIP(hipMemcpyAsync(ids, h_ids, (size_t)n * 4, hipMemcpyHostToDevice, s));
+  QH_HIP(hipMemcpyAsync(c->dev.tokens + c->length, ids, (size_t)total * 4, hipMemcpyDeviceToDevice, s));
   if ((rc = set_state(c, c->length, c->length + total))) return rc;
   for (int t = 0; t < total; t++) {
     QH_HIP(qh::enqueue_step(s, md, c->dev, qh::STEP_GATHER, true));
-    QH_HIP(qh::launch_nll(s, c->dev.logits, md.vocab, d.ids + t + 1, 1, d.parts, d.nll + t));
+    QH_HIP(qh::launch_nll(s, c->dev.logits, md.vocab, ids + t + 1, 1, parts, nll + t));
   }
-  QH_HIP(hipMemcpyAsync(h_nll, d.nll, (size_t)total * 8, hipMemcpyDeviceToHost, s));
+  QH_HIP(hipMemcpyAsync(h_nll, nll, nll_bytes, hipMemcpyDeviceToHost, s));
   QH_HIP(hipStreamSynchronize(s));
   c->length += total;
   return QH_OK;

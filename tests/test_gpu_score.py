@@ -93,3 +93,123 @@ def test_score_errors(ctx, hip):
     assert c.length == 0
     c.destroy()
     model.destroy()
+
+
+@pytest.fixture(scope="module", params=["fast", "exact"])
+def stepped(request, ctx, hip):
+    """A tiny model, 636 ids, and what one-token forwards of them give: logits, K/V rows."""
+    numerics = request.param
+    cfg = tiny(hip)
+    model = hip.GpuModel.load(ctx, hip.device_tensors(hip.synthesize_checkpoint(cfg, seed=34), cfg, "int8", 128, "int8"),
+                              cfg, maxPositions=700, numerics=numerics)
+    ids = hip.synth_tokens(34, "score.long", cfg.vocab, 637)
+    c = model.newCache(700)
+    logits = np.empty((636, cfg.vocab), np.float32)
+    for t in range(636):
+        logits[t] = model.forward_tokens(ids[t:t + 1], c)["logits"]
+    kv = [c.present(L) for L in range(cfg.layers)]
+    yield model, cfg, ids, logits, kv
+    c.destroy()
+    model.destroy()
+
+
+@pytest.mark.parametrize("past,total", [
+    (0, 1), (0, 2), (0, 3), (0, 4), (0, 64),
+    (0, 65),                    # a last head slice of one row
+    (0, 128), (0, 513),         # a second chunk of one position
+    (0, 600),                   # a second chunk with two head slices
+    (35, 1), (35, 2), (35, 130), (35, 601),
+])
+def test_score_of_every_slice_equals_steps(hip, stepped, past, total):
+    """Every position's score, wherever it falls among chunks of 512 positions and slices of 64 head
+    rows: the expression over the steps' own logits (the sum's spans are regrouped: 1e-12), the
+    steps' K/V rows, and a cache that goes on as after the steps."""
+    model, cfg, ids, logits, kv = stepped
+    c = model.newCache(700)
+    if past:
+        model.forward_tokens(ids[:past], c, wantLogits=False)
+    nll = model.score(ids[past:past + total + 1], c)
+    assert nll.shape == (total,) and c.length == past + total
+    for t in range(total):
+        assert nll[t] == pytest.approx(O.nll(logits[past + t], ids[past + t + 1]), rel=1e-12, abs=1e-12), t
+    for L in range(cfg.layers):
+        p = c.present(L)
+        for name in ("key", "value"):
+            np.testing.assert_array_equal(p[name].view(np.uint32), kv[L][name][:, :past + total].view(np.uint32))
+    last = logits[past + total - 1]
+    np.testing.assert_array_equal(c.vector("logits").view(np.uint32), last.view(np.uint32))
+    b = model.newCache(700)
+    for i in range(0, past + total, 300):
+        model.forward_tokens(ids[i:min(i + 300, past + total)], b, wantLogits=False)
+    first = int(np.argmax(last))
+    assert list(model.decode(c, first, 5)) == list(model.decode(b, first, 5))
+    np.testing.assert_array_equal(c.vector("logits").view(np.uint32), b.vector("logits").view(np.uint32))
+    b.destroy()
+    c.destroy()
+
+
+def test_score_between_forwards_of_every_mode(hip, stepped):
+    """Scores and forwards in turn under each matmul mode share one workspace: results stay those of
+    the mode alone."""
+    model, cfg, ids, logits, _ = stepped
+    want = {}
+    for mode in ("batched", "matvec", "mfma"):
+        model.set_matmul(mode)
+        c = model.newCache(64)
+        want[mode] = model.forward_tokens(ids[:40], c)["logits"]
+        c.destroy()
+    c = model.newCache(64)
+    for turn in range(3):
+        for mode in ("mfma", "batched", "matvec", "mfma"):
+            model.set_matmul(mode)
+            c.length = 0
+            np.testing.assert_array_equal(model.forward_tokens(ids[:40], c)["logits"].view(np.uint32),
+                                          want[mode].view(np.uint32), err_msg=f"{mode}, turn {turn}")
+            c.length = 0
+            nll = model.score(ids[:21], c)
+            for t in range(20):
+                assert nll[t] == pytest.approx(O.nll(logits[t], ids[t + 1]), rel=1e-12, abs=1e-12)
+    model.set_matmul("batched")
+    c.destroy()
+
+
+@pytest.mark.parametrize("numerics", ["fast", "exact"])
+@pytest.mark.parametrize("case", ["span of -inf", "NaN", "+inf", "all -inf"])
+def test_score_of_special_logits(ctx, hip, case, numerics):
+    """Logits with a whole span of -inf, a NaN, a +inf or nothing but -inf: what the expression gives
+    over the whole row, batched and step by step."""
+    cfg = tiny(hip)
+    ckpt = hip.synthesize_checkpoint(cfg, seed=35)
+    embed = ckpt["model.embed_tokens.weight"]
+    embed[:, 0] = 0x42C8                        # 100: dimension 0 stays positive in every row
+    t = hip.device_tensors(ckpt, cfg, "int8", 128, "f16")
+    fmt, rows, cols, group, head, s, z = t["lm_head.weight"]
+    head = head.copy()
+    only0 = np.zeros(cols, np.uint16)
+    if case == "span of -inf":
+        only0[0] = 0xFC00                       # -inf
+        head[250:375] = only0                   # one eighth of the 1000
+    elif case == "NaN":
+        head[700, 3] = 0x7E00
+    elif case == "+inf":
+        only0[0] = 0x7C00
+        head[999] = only0
+    else:
+        only0[0] = 0xFC00
+        head[:] = only0
+    t["lm_head.weight"] = (fmt, rows, cols, group, head, s, z)
+    model = hip.GpuModel.load(ctx, t, cfg, maxPositions=64, numerics=numerics)
+    ids = np.array([5, 17, 300, 800, 999, 251, 42, 374, 375, 249], np.int32)
+    c, b = model.newCache(64), model.newCache(64)
+    nll = model.score(ids, c)
+    for i in range(9):
+        row = model.forward_tokens(ids[i:i + 1], b)["logits"]
+        assert not np.isfinite(row).all()
+        want = O.nll(row, ids[i + 1])
+        b.length = i
+        one = model.score(ids[i:i + 2], b)[0]
+        for got in (nll[i], one):
+            np.testing.assert_allclose(got, want, rtol=1e-12, err_msg=f"position {i}")
+    c.destroy()
+    b.destroy()
+    model.destroy()
