@@ -233,11 +233,13 @@ PrefillBytes prefill_bytes(const ModelDev& m, const CacheDev& c, int matmul) {
   b.counters = m.numerics == QH_NUMERICS_EXACT ? P * m.heads : 0;
   const bool chain = m.numerics == QH_NUMERICS_FAST && !(matmul == QH_MATMUL_MFMA && all_mfma(m));
   size_t scratch = chain ? chain_partials_bound(m.lm_head, kHeadRows) : 0;  // enqueue_head_rows
-  if (m.numerics == QH_NUMERICS_EXACT) scratch = matvec_x64_bytes(m.lm_head, kHeadRows);
+  // exact contractions read an f64 copy of x only below the f64 matrix cores' positions
+  const int x64 = std::min((int)P, kChain64MinSeq - 1);
+  if (m.numerics == QH_NUMERICS_EXACT) scratch = matvec_x64_bytes(m.lm_head, x64);
   for (int L = 0; L < m.layers; L++) {
     const LayerDev& l = m.layers_host[L];
     for (const DMat* w : {&l.qkv, &l.o, &l.gu, &l.down}) {
-      if (m.numerics == QH_NUMERICS_EXACT) scratch = std::max(scratch, matvec_x64_bytes(*w, (int)P));
+      if (m.numerics == QH_NUMERICS_EXACT) scratch = std::max(scratch, matvec_x64_bytes(*w, x64));
       if (chain) scratch = std::max(scratch, chain_partials_bound(*w, (int)P));
       if (matmul == QH_MATMUL_MFMA && matmul_prefill_supported(*w))
         scratch = std::max(scratch, matmul_prefill_scratch_bytes(*w, (int)P));
@@ -343,6 +345,7 @@ static hipError_t matmul(hipStream_t s, const ModelDev& m, int mode, const DMat&
       return launch_chain_f32(s, w, x, bias, y, seq, static_cast<float*>(p.scratch), p.scratch_bytes);
     return launch_matvec_f32(s, w, x, bias, y, seq);
   }
+  if (!chain_f64_supported(w, x, seq) && matvec_x64_bytes(w, seq) > p.scratch_bytes) return hipErrorInvalidValue;
   return launch_matvec(s, w, x, bias, y, seq, static_cast<double*>(p.scratch));
 }
 

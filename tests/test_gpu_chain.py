@@ -2,6 +2,7 @@
 step: the same sums in the same order, so a prompt's logits and its f16 K/V rows are those of the
 same positions stepped one at a time, bit for bit -- at the edges of the 64-position and 64-row
 tiles, with one and several splits of the team's slots, ragged last chunks and every format."""
+import ctypes
 import time
 
 import numpy as np
@@ -152,6 +153,62 @@ def test_prompt_attention_past_1024_positions_equals_steps_bitwise(ctx, hip):
         np.testing.assert_array_equal(p["value"], s["value"])
     cache.destroy()
     steps.destroy()
+    model.destroy()
+
+
+@pytest.mark.parametrize("fmt", ["f16", "int8", "int4"])
+@pytest.mark.parametrize("cols", [896, 4864])     # positions in LDS; an f64 copy of all of them
+def test_matvec_of_unaligned_positions_equals_single_positions_bitwise(ctx, hip, fmt, cols):
+    """x off its 16 bytes stays in tiles of 8, 4, 2 and 1 positions."""
+    rng = np.random.default_rng(cols)
+    w = (rng.standard_normal((21, cols)) * 0.02).astype(np.float32)
+    if fmt == "f16":
+        bufs = [ctx.upload(w.astype(np.float16).view(np.uint16))]
+        W = ctx.weight(hip.FMT_F16, 21, cols, bufs[0])
+    elif fmt == "int8":
+        bufs = [ctx.upload(a) for a in hip.quantize_int8(w)]
+        W = ctx.weight(hip.FMT_INT8, 21, cols, *bufs)
+    else:
+        bufs = [ctx.upload(a) for a in hip.quantize_int4(w, 128)]
+        W = ctx.weight(hip.FMT_INT4, 21, cols, *bufs, 128)
+    x = rng.standard_normal((19, cols)).astype(np.float32)
+    dx = ctx.upload(np.concatenate([[np.float32(0)], x.reshape(-1)]))
+    off = hip.DeviceBuffer(ctx, dx.ptr + 4, dx.nbytes - 4)
+    dy = ctx.empty(19 * 21 * 4)
+    want = np.empty((19, 21), np.float32)
+    for t in range(19):
+        one = ctx.upload(x[t])
+        ctx.matvec(W, one, None, dy, 1)
+        want[t] = dy.read(count=21)
+        one.free()
+    for seq in (1, 6, 7, 8, 11, 16, 19):
+        ctx.matvec(W, off, None, dy, seq)
+        np.testing.assert_array_equal(dy.read(count=seq * 21).view(np.uint32), want[:seq].reshape(-1).view(np.uint32),
+                                      err_msg=f"{seq} positions")
+    for b in bufs + [dx, dy]:
+        b.free()
+
+
+def test_exact_workspace_holds_no_f64_copy_of_a_prompt(ctx, hip):
+    """512 positions of 4864 ffn columns would be 20 MB that no launch reads: from 6 positions the
+    exact contractions read the f32 rows."""
+    rt = ctypes.CDLL("libamdhip64.so")
+    rt.hipMemGetInfo.argtypes = [ctypes.POINTER(ctypes.c_size_t)] * 2
+
+    def free_bytes():
+        ctx.done()
+        free, total = ctypes.c_size_t(), ctypes.c_size_t()
+        assert rt.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+        return free.value
+    cfg = hip.ModelConfig(hidden=128, intermediate=4864, layers=1, heads=2, kv_heads=1, vocab=1000)
+    model = hip.GpuModel.load(ctx, hip.device_tensors(hip.synthesize_checkpoint(cfg, seed=24), cfg, "int8", 128, "int8"),
+                              cfg, maxPositions=512, numerics="exact")
+    cache = model.newCache(512)
+    ids = hip.synth_tokens(24, "chain.workspace", cfg.vocab, 5)
+    before = free_bytes()
+    model.forward_tokens(ids, cache)               # in tiles, which read the copy
+    assert before - free_bytes() < 1.25 * 512 * 4 * (7 * 128 + 3 * 4864)
+    cache.destroy()
     model.destroy()
 
 
