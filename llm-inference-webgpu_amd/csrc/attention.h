@@ -11,14 +11,14 @@
 //
 // Three algorithms:
 //
-// Exact order (k_attn_block up to kPLds positions, k_attn_exact beyond), the
+// Exact order (k_attn_block up to kPLds positions, k_attn_exact beyond; prompts by tiles, ops.hip), the
 // model's QH_NUMERICS_EXACT path. It evaluates groupedAttention (src/core/attention.js:
 // 32-66) step for step: each score is a sequential f64 dot stored to f32, the
 // softmax shifts by the global max and normalizes with an f64 sum
 // (src/core/ops.js:66-78), and the output accumulates sequentially over
 // positions in f32, as the reference's Float32Array `out += weight * value`
 // does, one lane per output dimension. k_attn_block does a (query, head) in one
-// 1024-thread block; k_attn_exact scores 256 positions per block and the last
+// 512-thread block; k_attn_exact scores 256 positions per block and the last
 // block of a (query, head) to finish does the softmax and the PV sum. The
 // result matches the CPU to the bit apart from f64-order noise, so a device f16
 // cache and the CPU's same-f16 cache stay identical.
@@ -32,8 +32,6 @@
 // the CPU's order, and checked within the kernel tolerance. A flash form of the same
 // products (k_flash_prefill) serves the MFMA prompt path.
 #pragma once
-
-#include <algorithm>
 
 #include "device_common.h"
 
@@ -169,7 +167,7 @@ __device__ __forceinline__ double block_sum_f64_n(double v, double* red) {
   return t;
 }
 
-static __global__ __launch_bounds__(kAttnThreads) void k_attn_block(ExactArgs a) {
+[[maybe_unused]] static __global__ __launch_bounds__(kAttnThreads) void k_attn_block(ExactArgs a) {
   const int h = blockIdx.x, t = blockIdx.y;
   const int past = a.d_pos ? *a.d_pos : a.past;
   const int pos = past + t;
@@ -271,265 +269,10 @@ static __global__ __launch_bounds__(kAttnThreads) void k_attn_block(ExactArgs a)
   if (tid < kHeadDim) a.out[((size_t)t * a.heads + h) * kHeadDim + tid] = o;
 }
 
-// -------------------------------------------- exact order, a tile of queries --
-// The same evaluation for a (head, 16 queries) tile of a prompt, with both products on the matrix
-// cores: v_mfma_f64_16x16x4f64 and v_mfma_f32_16x16x4f32 evaluate their four k as ascending fused
-// multiply-adds, each rounded to nearest even, so the f64 dots over i and the f32 sums over
-// positions are the chains k_attn_block evaluates, bit for bit; the softmax keeps its thread
-// order (position p on thread p % 512 of 8 waves). Keys past the tile's first query, which some
-// queries do not see, are summed on the vector unit under each query's own bound.
-//
-// Bound: latency of its three phases (f64 products, f64 exponentials, then a chain of ctx / 4
-// products per 16 dimensions), paid once for 16 queries where k_attn_block pays them per query.
-// One block of eight waves per CU (142 VGPRs; 51 to 150 KB of LDS by CTX). Tiles are launched
-// heaviest first. 512 queries, 14 heads: 182 -> 35 us.
-typedef double f64x4 __attribute__((ext_vector_type(4)));
-typedef float f32x4t __attribute__((ext_vector_type(4)));
-constexpr int kTileQ = 16;
-constexpr int kTileThreads = 512, kTileWaves = kTileThreads / kWave;
-static_assert(kTileThreads == kAttnThreads, "the softmax sum's thread order");
-constexpr int kTileCtx = 2048;     // the widest tile: 16 x 2052 floats of LDS
-// A tile takes as long as two to three k_attn_block blocks one after another, so tiles serve the
-// prompts whose (query, head) blocks would run in more than two rounds of one per CU (up to two and
-// a half in short contexts, where many queries' blocks differ in length and fill a third round).
-// Blocks | tiles, us, queries x heads after a past: 16 x 14 after 1980 31.5 | 72.6; 32 x 14 after 0 8.3 | 11.0, after 1000 36.0 | 42.9;
-// 128 x 4 after 496 28.7 | 30.0; 320 x 2 after 0 17.5 | 20.1; 160 x 4 after 128 18.8 | 20.0; 44 x 14
-// after 128 16.1 | 15.1; 48 x 14 after 496 36.9 | 26.7; 64 x 14 after 1980 100.8 | 73.0.
-constexpr int kTileMinSeq = 16;
-inline bool attn_tile_pays(int seq, int heads, int total) {
-  return seq >= kTileMinSeq && (long)seq * heads > 512 + (total <= 512 ? std::min(seq, 128) : 0);
-}
-
-// Element 4s + g of 16 f16 values (s = 0..3) in two 16-byte words.
-__device__ __forceinline__ float tile_f16(const v4u (&u)[2], int s, int g) {
-  const uint64_t pair = ((uint64_t)u[s >> 1][2 * (s & 1) + 1] << 32) | u[s >> 1][2 * (s & 1)];
-  return f16_lo((uint32_t)(pair >> (16 * g)));
-}
-// Where score p of a row sits: each 16 as [p % 4][p / 4 % 4], so a lane's four k are one read.
-__device__ __forceinline__ int tile_at(int p) { return (p & ~15) | ((p & 3) << 2) | ((p >> 2) & 3); }
-
-__device__ __forceinline__ float wave_max_dpp(float v) {
-  v = fmaxf(v, dpp32<kDppQuadXor1>(v));
-  v = fmaxf(v, dpp32<kDppQuadXor2>(v));
-  v = fmaxf(v, dpp32<kDppHalfMirror>(v));
-  v = fmaxf(v, dpp32<kDppMirror>(v));
-  v = fmaxf(v, swz_xor16(v));
-  return fmaxf(v, __shfl_xor(v, 32));
-}
-
-template <int CTX>
-static __global__ __launch_bounds__(kTileThreads) void k_attn_tile(ExactArgs a, int seq) {
-  __shared__ __attribute__((aligned(16))) float sc[kTileQ][CTX + 4];
-  static_assert(CTX % kTileThreads == 0, "the softmax reads whole threads' positions");
-  __shared__ __attribute__((aligned(16))) uint16_t ks[kTileWaves][16][kHeadDim + 8];  // padded over the banks
-  const int tid = threadIdx.x, lane = tid & (kWave - 1), w = tid / kWave, n = lane & 15, g = lane >> 4;
-  const int tiles = (seq + kTileQ - 1) / kTileQ;
-  const int h = blockIdx.x % a.heads, t0 = (tiles - 1 - blockIdx.x / a.heads) * kTileQ;
-  const int kvh = h / (a.heads / a.kv_heads);
-  const int kmax = a.past + min(t0 + kTileQ - 1, seq - 1);  // the tile's last key
-  if (kmax >= CTX || kmax >= a.capacity) return;            // the host keeps positions inside both
-  const uint16_t* kb = a.kc + (size_t)kvh * a.capacity * kHeadDim;
-  const uint16_t* vb = a.vt + (size_t)kvh * kHeadDim * a.vstride;
-
-  // Scores: key tiles w, w + 8, ..; accumulator register r holds query 4r + g, key n. A wave
-  // loads its tile's key rows once (a lane a quarter row, the next two tiles' in flight) and
-  // passes them through its own LDS to the lanes' elements 4s + g.
-  {
-    const float* q = a.q + ((size_t)min(t0 + n, seq - 1) * a.heads + h) * kHeadDim + g;
-    double qd[16];
-    v4u k[3][2];
-    auto load = [&](int kt, v4u (&d)[2]) {
-      const v4u* kr = reinterpret_cast<const v4u*>(kb + (size_t)min(16 * kt + n, kmax) * kHeadDim) + 2 * g;
-      d[0] = kr[0];
-      d[1] = kr[1];
-    };
-    load(w, k[0]);
-    load(w + kTileWaves, k[1]);
-#pragma unroll
-    for (int s = 0; s < 16; s++) qd[s] = (double)q[4 * s];
-    auto tile = [&](int kt, const v4u (&d)[2]) {
-      v4u* dst = reinterpret_cast<v4u*>(&ks[w][n][16 * g]);
-      dst[0] = d[0];
-      dst[1] = d[1];
-      __builtin_amdgcn_wave_barrier();  // the wave's LDS operations run in order
-      _Float16 e[16];
-#pragma unroll
-      for (int s = 0; s < 16; s++) e[s] = __builtin_bit_cast(_Float16, ks[w][n][4 * s + g]);
-      __builtin_amdgcn_wave_barrier();
-      f64x4 acc = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-      for (int s = 0; s < 16; s++)
-        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(qd[s], (double)(float)e[s], acc, 0, 0, 0);
-#pragma unroll
-      for (int r = 0; r < 4; r++) sc[4 * r + g][tile_at(16 * kt + n)] = (float)(acc[r] * 0.125);
-    };
-#pragma unroll 1
-    for (int kt = w; 16 * kt <= kmax; kt += 3 * kTileWaves) {
-      load(kt + 2 * kTileWaves, k[2]);
-      tile(kt, k[0]);
-      if (16 * (kt + kTileWaves) > kmax) break;
-      load(kt + 3 * kTileWaves, k[0]);
-      tile(kt + kTileWaves, k[1]);
-      if (16 * (kt + 2 * kTileWaves) > kmax) break;
-      load(kt + 4 * kTileWaves, k[1]);
-      tile(kt + 2 * kTileWaves, k[2]);
-    }
-  }
-  __syncthreads();
-  // PV's first values load while the softmax runs (waves 0-3, 16 dimensions each).
-  const uint16_t* vr = vb + (size_t)(16 * (w & 3) + n) * a.vstride;
-  const int full = (a.past + t0 + 1) >> 4;  // whole 16-position groups every query sees
-  const int lastg = (a.vstride >> 4) - 1;
-  constexpr int kAhead = 4;                 // groups whose values are loaded together
-  v4u vv[3][kAhead][2];                     // three such batches: two in flight under one's products
-  auto load = [&](int j0, v4u (&d)[kAhead][2]) {
-#pragma unroll
-    for (int j = 0; j < kAhead; j++) {
-      const v4u* src = reinterpret_cast<const v4u*>(vr + 16 * min(j0 + j, lastg));
-      d[j][0] = src[0];
-      d[j][1] = src[1];
-    }
-  };
-  // Softmax: wave w takes queries 2w and 2w + 1 together, lane l the positions of threads l,
-  // 64 + l, ..; two threads' worth of each query at a time, so exponentials and butterflies
-  // overlap. (A query past the end is a copy of the last.)
-  {
-    int ctx[2];
-    float* row[2];
-    double M[2], sum[2] = {0.0, 0.0}, inv[2];
-#pragma unroll
-    for (int i = 0; i < 2; i++) {
-      ctx[i] = a.past + min(t0 + 2 * w + i, seq - 1) + 1;
-      row[i] = sc[2 * w + i];
-    }
-    float m[2] = {-INFINITY, -INFINITY};
-#pragma unroll 1
-    for (int p0 = 0; p0 < ctx[1]; p0 += 4 * kWave) {
-      float v[2][4];
-#pragma unroll
-      for (int i = 0; i < 2; i++)
-#pragma unroll
-        for (int u = 0; u < 4; u++) v[i][u] = row[i][tile_at(p0 + u * kWave + lane)];
-#pragma unroll
-      for (int i = 0; i < 2; i++)
-#pragma unroll
-        for (int u = 0; u < 4; u++)
-          if (p0 + u * kWave + lane < ctx[i]) m[i] = fmaxf(m[i], v[i][u]);
-    }
-#pragma unroll
-    for (int i = 0; i < 2; i++) M[i] = wave_max_dpp(m[i]);
-#pragma unroll 1
-    for (int v0 = 0; v0 < kTileWaves && v0 * kWave < ctx[1]; v0 += 2) {
-      double part[2][2] = {};
-#pragma unroll 1
-      for (int p0 = v0 * kWave; p0 < ctx[1]; p0 += kTileThreads) {
-        double e[2][2];
-#pragma unroll
-        for (int i = 0; i < 2; i++)
-#pragma unroll
-          for (int u = 0; u < 2; u++) e[i][u] = exp((double)row[i][tile_at(p0 + u * kWave + lane)] - M[i]);
-#pragma unroll
-        for (int i = 0; i < 2; i++)
-#pragma unroll
-          for (int u = 0; u < 2; u++) {
-            const int p = p0 + u * kWave + lane;
-            if (p < ctx[i]) {
-              row[i][tile_at(p)] = (float)e[i][u];
-              part[i][u] += e[i][u];
-            }
-          }
-      }
-#pragma unroll
-      for (int i = 0; i < 2; i++)
-#pragma unroll
-        for (int u = 0; u < 2; u++) part[i][u] = team_sum<64>(part[i][u]);
-#pragma unroll
-      for (int i = 0; i < 2; i++) sum[i] = (sum[i] + part[i][0]) + part[i][1];
-    }
-#pragma unroll
-    for (int i = 0; i < 2; i++) inv[i] = 1.0 / sum[i];
-#pragma unroll 1
-    for (int p0 = 0; p0 < ctx[1]; p0 += 4 * kWave) {
-      float v[2][4];
-#pragma unroll
-      for (int i = 0; i < 2; i++)
-#pragma unroll
-        for (int u = 0; u < 4; u++) v[i][u] = row[i][tile_at(p0 + u * kWave + lane)];
-#pragma unroll
-      for (int i = 0; i < 2; i++)
-#pragma unroll
-        for (int u = 0; u < 4; u++)
-          if (p0 + u * kWave + lane < ctx[i])
-            row[i][tile_at(p0 + u * kWave + lane)] = (float)((double)v[i][u] * inv[i]);
-    }
-  }
-  v4u tv[2][2];  // the tile's last groups, which not every query sees whole
-  if (w < 4) {
-    load(0, vv[0]);
-    load(kAhead, vv[1]);
-#pragma unroll
-    for (int j = 0; j < 2; j++) {
-      const v4u* src = reinterpret_cast<const v4u*>(vr + 16 * min(full + j, lastg));
-      tv[j][0] = src[0];
-      tv[j][1] = src[1];
-    }
-  }
-  __syncthreads();
-  if (w >= 4) return;
-  // PV: wave w sums dimensions 16w .. +15 over the positions; register r holds query 4g + r.
-  f32x4t o = {0.f, 0.f, 0.f, 0.f};
-  auto group = [&](int j, const v4u (&d)[2], const v4f p) {
-#pragma unroll
-    for (int s = 0; s < 4; s++) o = __builtin_amdgcn_mfma_f32_16x16x4f32(p[s], tile_f16(d, s, g), o, 0, 0, 0);
-  };
-  auto batch = [&](int j0, const v4u (&d)[kAhead][2]) {
-    v4f p[kAhead];
-#pragma unroll
-    for (int j = 0; j < kAhead; j++) p[j] = *reinterpret_cast<const v4f*>(&sc[n][16 * min(j0 + j, CTX / 16 - 1) + 4 * g]);
-#pragma unroll
-    for (int j = 0; j < kAhead; j++)
-      if (j0 + j < full) group(j0 + j, d[j], p[j]);  // uniform
-  };
-#pragma unroll 1
-  for (int j0 = 0; j0 < full; j0 += 3 * kAhead) {
-    load(j0 + 2 * kAhead, vv[2]);
-    batch(j0, vv[0]);
-    load(j0 + 3 * kAhead, vv[0]);
-    batch(j0 + kAhead, vv[1]);
-    load(j0 + 4 * kAhead, vv[1]);
-    batch(j0 + 2 * kAhead, vv[2]);
-  }
-  // The last groups: positions two at a time (a dword of values), each under its query's bound.
-#pragma unroll
-  for (int j = 0; j < 2; j++) {
-    const int p0 = 16 * (full + j);
-    if (p0 <= kmax) {  // uniform
-#pragma unroll
-      for (int k = 0; k < 8; k++) {
-        const uint32_t d = tv[j][k >> 2][k & 3];
-        const int p = p0 + 2 * k;
-        if (p <= kmax) {  // uniform
-#pragma unroll
-          for (int r = 0; r < 4; r++) {
-            const int last = min(a.past + t0 + 4 * g + r, kmax);
-            const float x = fmaf(sc[4 * g + r][tile_at(p)], f16_lo(d), o[r]);
-            o[r] = p <= last ? x : o[r];
-            const float y = fmaf(sc[4 * g + r][tile_at(p + 1)], f16_hi(d), o[r]);
-            o[r] = p + 1 <= last ? y : o[r];
-          }
-        }
-      }
-    }
-  }
-#pragma unroll
-  for (int r = 0; r < 4; r++)
-    if (t0 + 4 * g + r < seq) a.out[((size_t)(t0 + 4 * g + r) * a.heads + h) * kHeadDim + 16 * w + n] = o[r];
-}
-
 // grid (spans, heads, seq). Block (span, h, t) scores positions span*256 ..
 // +255 of query t against head h and records the span's maximum; the last span
 // block of (t, h) to finish computes the probabilities and the output.
-static __global__ __launch_bounds__(kBlock) void k_attn_exact(ExactArgs a) {
+[[maybe_unused]] static __global__ __launch_bounds__(kBlock) void k_attn_exact(ExactArgs a) {
   const int sp = blockIdx.x, h = blockIdx.y, t = blockIdx.z;
   const int past = a.d_pos ? *a.d_pos : a.past;
   const int pos = past + t;
@@ -629,24 +372,10 @@ static __global__ __launch_bounds__(kBlock) void k_attn_exact(ExactArgs a) {
   if (tid == 0) a.counters[row] = 0;
 }
 
-// Exact attention of `seq` queries over past + seq positions: query tiles for prompts that fit
-// and fill them (attn_tile_pays), else a (query, head) block up to kPLds positions -- of context for the operator, of
-// capacity for the model (`limit`), whose decode step picks by capacity -- else spans. All
-// evaluate a query alike.
-static inline hipError_t launch_attn_exact(hipStream_t s, const ExactArgs& a, int seq, int limit, int spans) {
-  const int total = a.past + seq;
-  if (attn_tile_pays(seq, a.heads, total) && total <= kTileCtx && limit <= kPLds) {
-    const dim3 grid((seq + kTileQ - 1) / kTileQ * a.heads), block(kTileThreads);
-    if (total <= 512) hipLaunchKernelGGL(k_attn_tile<512>, grid, block, 0, s, a, seq);
-    else if (total <= 1024) hipLaunchKernelGGL(k_attn_tile<1024>, grid, block, 0, s, a, seq);
-    else hipLaunchKernelGGL(k_attn_tile<kTileCtx>, grid, block, 0, s, a, seq);
-  } else if (limit <= kPLds) {
-    hipLaunchKernelGGL(k_attn_block, dim3(a.heads, seq), dim3(kAttnThreads), 0, s, a);
-  } else {
-    hipLaunchKernelGGL(k_attn_exact, dim3(spans, a.heads, seq), dim3(kBlock), 0, s, a);
-  }
-  return hipGetLastError();
-}
+// Exact attention of `seq` queries over past + seq positions (ops.hip). `limit` picks between a
+// (query, head) block, up to kPLds positions, and `spans` spans: the context for the operator, the
+// capacity for the model, whose decode step picks by capacity.
+hipError_t launch_attn_exact(hipStream_t s, const ExactArgs& a, int seq, int limit, int spans);
 
 // -------------------------------------------------------------- split-K --
 // Split-K online softmax. The context is cut into 64-position chunks; a "slot"
@@ -1299,106 +1028,6 @@ __device__ __forceinline__ void stage_attn_combine_f32(const CombineIn& in, int 
   const int i = threadIdx.x;
   stage_group_f32<FMT>(acc, i, i < heads * kCombineLanes, xs, xs + heads * kHeadDim, lay);
   __syncthreads();
-}
-
-// ------------------------------------------- a prompt's queries, merged in place --
-// The decode step's attention for each query of a prompt (caches of up to kLongCapacity
-// positions), slots and merge in one block per (kv head, query): the step's launch gives a query
-// 32 blocks, most of them empty at prompt lengths, and passes 16 slots of partials through memory
-// to a merge launch. A wave takes slots w and w + 8; a slot's steps go to four states (two where
-// no slot has more than one chunk), the step's four waves, merged in wave order, and the slots
-// merge by the step's own combine: every output has the decode step's bits. An empty slot is the
-// neutral partial and is never read. Bound: latency, a query's K/V from L2. 512 queries, 14 heads:
-// 83 us (plus a 6 us merge) -> 20 us.
-constexpr int kPromptWaves = 8;
-template <int NS>
-static __global__ __launch_bounds__(kPromptWaves * kWave) void k_attn_prompt(SlotArgs a) {
-  __shared__ __attribute__((aligned(16))) float part[kDecodeSlots][8][kPartStride];
-  __shared__ float wl[8 * kCombineLanes];
-  const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave, n = lane & 15, g = lane >> 4;
-  const int group = a.heads / a.kv_heads, kvh = blockIdx.x;
-  const int t = gridDim.y - 1 - blockIdx.y;  // the longest contexts first
-  const int ctx = a.past + t + 1, nch = attn_chunks(ctx);
-  const float* q = a.q + ((size_t)t * a.heads + kvh * group) * kHeadDim;
-  f16x8 qh[2], ql[2];
-  load_query_split(q + (n < group ? n : 0) * kHeadDim, g, qh, ql);
-  const uint16_t* kb = a.kc + (size_t)kvh * a.capacity * kHeadDim;
-  const uint16_t* vb = a.vt + (size_t)kvh * kHeadDim * a.vstride;
-  for (int sl = w; sl < kDecodeSlots && sl < nch; sl += kPromptWaves) {
-    const int chunks = (nch - 1 - sl) / kDecodeSlots + 1;
-    const int last = sl + (chunks - 1) * kDecodeSlots;
-    const int steps = 2 * chunks - (last * kChunk + 32 >= ctx ? 1 : 0);
-    float m[NS], l[NS];
-    f32x4 o[NS][4];
-    KvStep d[2];
-    kv_load(kb, vb, gqa_p0<kDecodeSlots>(sl, 0), a.capacity, a.vstride, n, g, d[0]);
-#pragma unroll
-    for (int v = 0; v < NS; v++) {
-      m[v] = -INFINITY;
-      l[v] = 0.f;
-#pragma unroll
-      for (int dt = 0; dt < 4; dt++) o[v][dt] = (f32x4){0.f, 0.f, 0.f, 0.f};
-    }
-    // Step i belongs to state i % 4, the next step's loads in flight.
-#pragma unroll 1
-    for (int i0 = 0; i0 < steps; i0 += NS) {
-#pragma unroll
-      for (int v = 0; v < NS; v++) {
-        if (i0 + v < steps) {
-          if (i0 + v + 1 < steps)
-            kv_load(kb, vb, gqa_p0<kDecodeSlots>(sl, i0 + v + 1), a.capacity, a.vstride, n, g, d[(v + 1) & 1]);
-          kv_step(qh, ql, d[v & 1], gqa_p0<kDecodeSlots>(sl, i0 + v), ctx, ctx, g, m[v], l[v], o[v]);
-        }
-      }
-    }
-    float mx = -INFINITY;
-#pragma unroll
-    for (int v = 0; v < NS; v++) mx = fmaxf(mx, m[v]);
-    float wt[NS], lt = 0.f;
-#pragma unroll
-    for (int v = 0; v < NS; v++) {
-      wt[v] = m[v] == -INFINITY ? 0.f : exp2_reduced(m[v] - mx);
-      lt = fmaf(l[v], wt[v], lt);
-    }
-    if (n < group) {
-#pragma unroll
-      for (int dt = 0; dt < 4; dt++) {
-        v4f ot = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int v = 0; v < NS; v++)
-#pragma unroll
-          for (int r = 0; r < 4; r++) ot[r] = fmaf(o[v][dt][r], wt[v], ot[r]);
-        if (NS < kDecodeWaves) ot += (v4f){0.f, 0.f, 0.f, 0.f};  // the empty waves' + 0 (it turns a -0 around)
-        *reinterpret_cast<v4f*>(&part[sl][n][4 + 16 * dt + 4 * g]) = ot;
-      }
-      if (g == 0) {
-        part[sl][n][0] = mx;
-        part[sl][n][1] = lt;
-      }
-    }
-  }
-  __syncthreads();
-  const int i = threadIdx.x;
-  if (i >= 8 * kCombineLanes) return;  // whole waves
-  const int h = min(i / kCombineLanes, group - 1), k = i % kCombineLanes;
-  CombineIn in;
-#pragma unroll
-  for (int s = 0; s < kDecodeSlots; s++)
-    in.ov[s] = s < nch ? *reinterpret_cast<const v4f*>(&part[s][h][4 + 4 * k]) : (v4f){0.f, 0.f, 0.f, 0.f};
-  in.mv = k < nch ? part[k][h][0] : -INFINITY;
-  in.lv = k < nch ? part[k][h][1] : 0.f;
-  const v4f acc = attn_combine_quad(in, wl);
-  if (i < group * kCombineLanes)
-    *reinterpret_cast<v4f*>(a.out + ((size_t)t * a.heads + kvh * group) * kHeadDim + 4 * i) = acc;
-}
-
-// The decode step's attention of `seq` prompt queries, merged into a.out [seq][heads*64]; for
-// caches that decode_attn_long does not claim.
-static inline hipError_t launch_attn_prompt(hipStream_t s, const SlotArgs& a, int seq) {
-  const dim3 grid(a.kv_heads, seq), block(kPromptWaves * kWave);
-  if (attn_chunks(a.past + seq) <= kDecodeSlots) hipLaunchKernelGGL(k_attn_prompt<2>, grid, block, 0, s, a);
-  else hipLaunchKernelGGL(k_attn_prompt<kDecodeWaves>, grid, block, 0, s, a);
-  return hipGetLastError();
 }
 
 }  // namespace qh

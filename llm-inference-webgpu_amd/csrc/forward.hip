@@ -349,6 +349,106 @@ static hipError_t matmul(hipStream_t s, const ModelDev& m, int mode, const DMat&
   return launch_matvec(s, w, x, bias, y, seq, static_cast<double*>(p.scratch));
 }
 
+// ------------------------------------------- a prompt's queries, merged in place --
+// The decode step's attention for each query of a prompt (caches of up to kLongCapacity
+// positions), slots and merge in one block per (kv head, query): the step's launch gives a query
+// 32 blocks, most of them empty at prompt lengths, and passes 16 slots of partials through memory
+// to a merge launch. A wave takes slots w and w + 8; a slot's steps go to four states (two where
+// no slot has more than one chunk), the step's four waves, merged in wave order, and the slots
+// merge by the step's own combine: every output has the decode step's bits. An empty slot is the
+// neutral partial and is never read. Bound: latency, a query's K/V from L2. 512 queries, 14 heads:
+// 83 us (plus a 6 us merge) -> 20 us.
+constexpr int kPromptWaves = 8;
+template <int NS>
+static __global__ __launch_bounds__(kPromptWaves * kWave) void k_attn_prompt(SlotArgs a) {
+  __shared__ __attribute__((aligned(16))) float part[kDecodeSlots][8][kPartStride];
+  __shared__ float wl[8 * kCombineLanes];
+  const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave, n = lane & 15, g = lane >> 4;
+  const int group = a.heads / a.kv_heads, kvh = blockIdx.x;
+  const int t = gridDim.y - 1 - blockIdx.y;  // the longest contexts first
+  const int ctx = a.past + t + 1, nch = attn_chunks(ctx);
+  const float* q = a.q + ((size_t)t * a.heads + kvh * group) * kHeadDim;
+  f16x8 qh[2], ql[2];
+  load_query_split(q + (n < group ? n : 0) * kHeadDim, g, qh, ql);
+  const uint16_t* kb = a.kc + (size_t)kvh * a.capacity * kHeadDim;
+  const uint16_t* vb = a.vt + (size_t)kvh * kHeadDim * a.vstride;
+  for (int sl = w; sl < kDecodeSlots && sl < nch; sl += kPromptWaves) {
+    const int chunks = (nch - 1 - sl) / kDecodeSlots + 1;
+    const int last = sl + (chunks - 1) * kDecodeSlots;
+    const int steps = 2 * chunks - (last * kChunk + 32 >= ctx ? 1 : 0);
+    float m[NS], l[NS];
+    f32x4 o[NS][4];
+    KvStep d[2];
+    kv_load(kb, vb, gqa_p0<kDecodeSlots>(sl, 0), a.capacity, a.vstride, n, g, d[0]);
+#pragma unroll
+    for (int v = 0; v < NS; v++) {
+      m[v] = -INFINITY;
+      l[v] = 0.f;
+#pragma unroll
+      for (int dt = 0; dt < 4; dt++) o[v][dt] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    }
+    // Step i belongs to state i % 4, the next step's loads in flight.
+#pragma unroll 1
+    for (int i0 = 0; i0 < steps; i0 += NS) {
+#pragma unroll
+      for (int v = 0; v < NS; v++) {
+        if (i0 + v < steps) {
+          if (i0 + v + 1 < steps)
+            kv_load(kb, vb, gqa_p0<kDecodeSlots>(sl, i0 + v + 1), a.capacity, a.vstride, n, g, d[(v + 1) & 1]);
+          kv_step(qh, ql, d[v & 1], gqa_p0<kDecodeSlots>(sl, i0 + v), ctx, ctx, g, m[v], l[v], o[v]);
+        }
+      }
+    }
+    float mx = -INFINITY;
+#pragma unroll
+    for (int v = 0; v < NS; v++) mx = fmaxf(mx, m[v]);
+    float wt[NS], lt = 0.f;
+#pragma unroll
+    for (int v = 0; v < NS; v++) {
+      wt[v] = m[v] == -INFINITY ? 0.f : exp2_reduced(m[v] - mx);
+      lt = fmaf(l[v], wt[v], lt);
+    }
+    if (n < group) {
+#pragma unroll
+      for (int dt = 0; dt < 4; dt++) {
+        v4f ot = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int v = 0; v < NS; v++)
+#pragma unroll
+          for (int r = 0; r < 4; r++) ot[r] = fmaf(o[v][dt][r], wt[v], ot[r]);
+        if (NS < kDecodeWaves) ot += (v4f){0.f, 0.f, 0.f, 0.f};  // the empty waves' + 0 (it turns a -0 around)
+        *reinterpret_cast<v4f*>(&part[sl][n][4 + 16 * dt + 4 * g]) = ot;
+      }
+      if (g == 0) {
+        part[sl][n][0] = mx;
+        part[sl][n][1] = lt;
+      }
+    }
+  }
+  __syncthreads();
+  const int i = threadIdx.x;
+  if (i >= 8 * kCombineLanes) return;  // whole waves
+  const int h = min(i / kCombineLanes, group - 1), k = i % kCombineLanes;
+  CombineIn in;
+#pragma unroll
+  for (int s = 0; s < kDecodeSlots; s++)
+    in.ov[s] = s < nch ? *reinterpret_cast<const v4f*>(&part[s][h][4 + 4 * k]) : (v4f){0.f, 0.f, 0.f, 0.f};
+  in.mv = k < nch ? part[k][h][0] : -INFINITY;
+  in.lv = k < nch ? part[k][h][1] : 0.f;
+  const v4f acc = attn_combine_quad(in, wl);
+  if (i < group * kCombineLanes)
+    *reinterpret_cast<v4f*>(a.out + ((size_t)t * a.heads + kvh * group) * kHeadDim + 4 * i) = acc;
+}
+
+// The decode step's attention of `seq` prompt queries, merged into a.out [seq][heads*64]; for
+// caches that decode_attn_long does not claim.
+static hipError_t launch_attn_prompt(hipStream_t s, const SlotArgs& a, int seq) {
+  const dim3 grid(a.kv_heads, seq), block(kPromptWaves * kWave);
+  if (attn_chunks(a.past + seq) <= kDecodeSlots) hipLaunchKernelGGL(k_attn_prompt<2>, grid, block, 0, s, a);
+  else hipLaunchKernelGGL(k_attn_prompt<kDecodeWaves>, grid, block, 0, s, a);
+  return hipGetLastError();
+}
+
 // The batched fast-numerics attention of a layer: the decode step's, merged, into p.ATT.
 static hipError_t batched_attention(hipStream_t s, const ModelDev& m, const CacheDev& c, const PrefillDev& p,
                                     const uint16_t* kc, const uint16_t* vt, int past, int seq) {

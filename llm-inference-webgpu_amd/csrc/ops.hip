@@ -463,6 +463,280 @@ hipError_t launch_kv_append(hipStream_t s, const float* k, const float* v, uint1
   return hipGetLastError();
 }
 
+// -------------------------------------------- exact order, a tile of queries --
+// The same evaluation for a (head, 16 queries) tile of a prompt, with both products on the matrix
+// cores: v_mfma_f64_16x16x4f64 and v_mfma_f32_16x16x4f32 evaluate their four k as ascending fused
+// multiply-adds, each rounded to nearest even, so the f64 dots over i and the f32 sums over
+// positions are the chains k_attn_block evaluates, bit for bit; the softmax keeps its thread
+// order (position p on thread p % 512 of 8 waves). Keys past the tile's first query, which some
+// queries do not see, are summed on the vector unit under each query's own bound.
+//
+// Bound: latency of its three phases (f64 products, f64 exponentials, then a chain of ctx / 4
+// products per 16 dimensions), paid once for 16 queries where k_attn_block pays them per query.
+// One block of eight waves per CU (142 VGPRs; 51 to 150 KB of LDS by CTX). Tiles are launched
+// heaviest first. 512 queries, 14 heads: 182 -> 35 us.
+typedef double f64x4 __attribute__((ext_vector_type(4)));
+typedef float f32x4t __attribute__((ext_vector_type(4)));
+constexpr int kTileQ = 16;
+constexpr int kTileThreads = 512, kTileWaves = kTileThreads / kWave;
+static_assert(kTileThreads == kAttnThreads, "the softmax sum's thread order");
+constexpr int kTileCtx = 2048;     // the widest tile: 16 x 2052 floats of LDS
+// A tile takes as long as two to three k_attn_block blocks one after another, so tiles serve the
+// prompts whose (query, head) blocks would run in more than two rounds of one per CU (up to two and
+// a half in short contexts, where many queries' blocks differ in length and fill a third round).
+// Blocks | tiles, us, queries x heads after a past: 16 x 14 after 1980 31.5 | 72.6; 32 x 14 after 0 8.3 | 11.0, after 1000 36.0 | 42.9;
+// 128 x 4 after 496 28.7 | 30.0; 320 x 2 after 0 17.5 | 20.1; 160 x 4 after 128 18.8 | 20.0; 44 x 14
+// after 128 16.1 | 15.1; 48 x 14 after 496 36.9 | 26.7; 64 x 14 after 1980 100.8 | 73.0.
+constexpr int kTileMinSeq = 16;
+static bool attn_tile_pays(int seq, int heads, int total) {
+  return seq >= kTileMinSeq && (long)seq * heads > 512 + (total <= 512 ? std::min(seq, 128) : 0);
+}
+
+// Element 4s + g of 16 f16 values (s = 0..3) in two 16-byte words.
+__device__ __forceinline__ float tile_f16(const v4u (&u)[2], int s, int g) {
+  const uint64_t pair = ((uint64_t)u[s >> 1][2 * (s & 1) + 1] << 32) | u[s >> 1][2 * (s & 1)];
+  return f16_lo((uint32_t)(pair >> (16 * g)));
+}
+// Where score p of a row sits: each 16 as [p % 4][p / 4 % 4], so a lane's four k are one read.
+__device__ __forceinline__ int tile_at(int p) { return (p & ~15) | ((p & 3) << 2) | ((p >> 2) & 3); }
+
+__device__ __forceinline__ float wave_max_dpp(float v) {
+  v = fmaxf(v, dpp32<kDppQuadXor1>(v));
+  v = fmaxf(v, dpp32<kDppQuadXor2>(v));
+  v = fmaxf(v, dpp32<kDppHalfMirror>(v));
+  v = fmaxf(v, dpp32<kDppMirror>(v));
+  v = fmaxf(v, swz_xor16(v));
+  return fmaxf(v, __shfl_xor(v, 32));
+}
+
+template <int CTX>
+static __global__ __launch_bounds__(kTileThreads) void k_attn_tile(ExactArgs a, int seq) {
+  __shared__ __attribute__((aligned(16))) float sc[kTileQ][CTX + 4];
+  static_assert(CTX % kTileThreads == 0, "the softmax reads whole threads' positions");
+  __shared__ __attribute__((aligned(16))) uint16_t ks[kTileWaves][16][kHeadDim + 8];  // padded over the banks
+  const int tid = threadIdx.x, lane = tid & (kWave - 1), w = tid / kWave, n = lane & 15, g = lane >> 4;
+  const int tiles = (seq + kTileQ - 1) / kTileQ;
+  const int h = blockIdx.x % a.heads, t0 = (tiles - 1 - blockIdx.x / a.heads) * kTileQ;
+  const int kvh = h / (a.heads / a.kv_heads);
+  const int kmax = a.past + min(t0 + kTileQ - 1, seq - 1);  // the tile's last key
+  if (kmax >= CTX || kmax >= a.capacity) return;            // the host keeps positions inside both
+  const uint16_t* kb = a.kc + (size_t)kvh * a.capacity * kHeadDim;
+  const uint16_t* vb = a.vt + (size_t)kvh * kHeadDim * a.vstride;
+
+  // Scores: key tiles w, w + 8, ..; accumulator register r holds query 4r + g, key n. A wave
+  // loads its tile's key rows once (a lane a quarter row, the next two tiles' in flight) and
+  // passes them through its own LDS to the lanes' elements 4s + g.
+  {
+    const float* q = a.q + ((size_t)min(t0 + n, seq - 1) * a.heads + h) * kHeadDim + g;
+    double qd[16];
+    v4u k[3][2];
+    auto load = [&](int kt, v4u (&d)[2]) {
+      const v4u* kr = reinterpret_cast<const v4u*>(kb + (size_t)min(16 * kt + n, kmax) * kHeadDim) + 2 * g;
+      d[0] = kr[0];
+      d[1] = kr[1];
+    };
+    load(w, k[0]);
+    load(w + kTileWaves, k[1]);
+#pragma unroll
+    for (int s = 0; s < 16; s++) qd[s] = (double)q[4 * s];
+    auto tile = [&](int kt, const v4u (&d)[2]) {
+      v4u* dst = reinterpret_cast<v4u*>(&ks[w][n][16 * g]);
+      dst[0] = d[0];
+      dst[1] = d[1];
+      __builtin_amdgcn_wave_barrier();  // the wave's LDS operations run in order
+      _Float16 e[16];
+#pragma unroll
+      for (int s = 0; s < 16; s++) e[s] = __builtin_bit_cast(_Float16, ks[w][n][4 * s + g]);
+      __builtin_amdgcn_wave_barrier();
+      f64x4 acc = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+      for (int s = 0; s < 16; s++)
+        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(qd[s], (double)(float)e[s], acc, 0, 0, 0);
+#pragma unroll
+      for (int r = 0; r < 4; r++) sc[4 * r + g][tile_at(16 * kt + n)] = (float)(acc[r] * 0.125);
+    };
+#pragma unroll 1
+    for (int kt = w; 16 * kt <= kmax; kt += 3 * kTileWaves) {
+      load(kt + 2 * kTileWaves, k[2]);
+      tile(kt, k[0]);
+      if (16 * (kt + kTileWaves) > kmax) break;
+      load(kt + 3 * kTileWaves, k[0]);
+      tile(kt + kTileWaves, k[1]);
+      if (16 * (kt + 2 * kTileWaves) > kmax) break;
+      load(kt + 4 * kTileWaves, k[1]);
+      tile(kt + 2 * kTileWaves, k[2]);
+    }
+  }
+  __syncthreads();
+  // PV's first values load while the softmax runs (waves 0-3, 16 dimensions each).
+  const uint16_t* vr = vb + (size_t)(16 * (w & 3) + n) * a.vstride;
+  const int full = (a.past + t0 + 1) >> 4;  // whole 16-position groups every query sees
+  const int lastg = (a.vstride >> 4) - 1;
+  constexpr int kAhead = 4;                 // groups whose values are loaded together
+  v4u vv[3][kAhead][2];                     // three such batches: two in flight under one's products
+  auto load = [&](int j0, v4u (&d)[kAhead][2]) {
+#pragma unroll
+    for (int j = 0; j < kAhead; j++) {
+      const v4u* src = reinterpret_cast<const v4u*>(vr + 16 * min(j0 + j, lastg));
+      d[j][0] = src[0];
+      d[j][1] = src[1];
+    }
+  };
+  // Softmax: wave w takes queries 2w and 2w + 1 together, lane l the positions of threads l,
+  // 64 + l, ..; two threads' worth of each query at a time, so exponentials and butterflies
+  // overlap. (A query past the end is a copy of the last.)
+  {
+    int ctx[2];
+    float* row[2];
+    double M[2], sum[2] = {0.0, 0.0}, inv[2];
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+      ctx[i] = a.past + min(t0 + 2 * w + i, seq - 1) + 1;
+      row[i] = sc[2 * w + i];
+    }
+    float m[2] = {-INFINITY, -INFINITY};
+#pragma unroll 1
+    for (int p0 = 0; p0 < ctx[1]; p0 += 4 * kWave) {
+      float v[2][4];
+#pragma unroll
+      for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int u = 0; u < 4; u++) v[i][u] = row[i][tile_at(p0 + u * kWave + lane)];
+#pragma unroll
+      for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+          if (p0 + u * kWave + lane < ctx[i]) m[i] = fmaxf(m[i], v[i][u]);
+    }
+#pragma unroll
+    for (int i = 0; i < 2; i++) M[i] = wave_max_dpp(m[i]);
+#pragma unroll 1
+    for (int v0 = 0; v0 < kTileWaves && v0 * kWave < ctx[1]; v0 += 2) {
+      double part[2][2] = {};
+#pragma unroll 1
+      for (int p0 = v0 * kWave; p0 < ctx[1]; p0 += kTileThreads) {
+        double e[2][2];
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+#pragma unroll
+          for (int u = 0; u < 2; u++) e[i][u] = exp((double)row[i][tile_at(p0 + u * kWave + lane)] - M[i]);
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+#pragma unroll
+          for (int u = 0; u < 2; u++) {
+            const int p = p0 + u * kWave + lane;
+            if (p < ctx[i]) {
+              row[i][tile_at(p)] = (float)e[i][u];
+              part[i][u] += e[i][u];
+            }
+          }
+      }
+#pragma unroll
+      for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int u = 0; u < 2; u++) part[i][u] = team_sum<64>(part[i][u]);
+#pragma unroll
+      for (int i = 0; i < 2; i++) sum[i] = (sum[i] + part[i][0]) + part[i][1];
+    }
+#pragma unroll
+    for (int i = 0; i < 2; i++) inv[i] = 1.0 / sum[i];
+#pragma unroll 1
+    for (int p0 = 0; p0 < ctx[1]; p0 += 4 * kWave) {
+      float v[2][4];
+#pragma unroll
+      for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int u = 0; u < 4; u++) v[i][u] = row[i][tile_at(p0 + u * kWave + lane)];
+#pragma unroll
+      for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+          if (p0 + u * kWave + lane < ctx[i])
+            row[i][tile_at(p0 + u * kWave + lane)] = (float)((double)v[i][u] * inv[i]);
+    }
+  }
+  v4u tv[2][2];  // the tile's last groups, which not every query sees whole
+  if (w < 4) {
+    load(0, vv[0]);
+    load(kAhead, vv[1]);
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+      const v4u* src = reinterpret_cast<const v4u*>(vr + 16 * min(full + j, lastg));
+      tv[j][0] = src[0];
+      tv[j][1] = src[1];
+    }
+  }
+  __syncthreads();
+  if (w >= 4) return;
+  // PV: wave w sums dimensions 16w .. +15 over the positions; register r holds query 4g + r.
+  f32x4t o = {0.f, 0.f, 0.f, 0.f};
+  auto group = [&](int j, const v4u (&d)[2], const v4f p) {
+#pragma unroll
+    for (int s = 0; s < 4; s++) o = __builtin_amdgcn_mfma_f32_16x16x4f32(p[s], tile_f16(d, s, g), o, 0, 0, 0);
+  };
+  auto batch = [&](int j0, const v4u (&d)[kAhead][2]) {
+    v4f p[kAhead];
+#pragma unroll
+    for (int j = 0; j < kAhead; j++) p[j] = *reinterpret_cast<const v4f*>(&sc[n][16 * min(j0 + j, CTX / 16 - 1) + 4 * g]);
+#pragma unroll
+    for (int j = 0; j < kAhead; j++)
+      if (j0 + j < full) group(j0 + j, d[j], p[j]);  // uniform
+  };
+#pragma unroll 1
+  for (int j0 = 0; j0 < full; j0 += 3 * kAhead) {
+    load(j0 + 2 * kAhead, vv[2]);
+    batch(j0, vv[0]);
+    load(j0 + 3 * kAhead, vv[0]);
+    batch(j0 + kAhead, vv[1]);
+    load(j0 + 4 * kAhead, vv[1]);
+    batch(j0 + 2 * kAhead, vv[2]);
+  }
+  // The last groups: positions two at a time (a dword of values), each under its query's bound.
+#pragma unroll
+  for (int j = 0; j < 2; j++) {
+    const int p0 = 16 * (full + j);
+    if (p0 <= kmax) {  // uniform
+#pragma unroll
+      for (int k = 0; k < 8; k++) {
+        const uint32_t d = tv[j][k >> 2][k & 3];
+        const int p = p0 + 2 * k;
+        if (p <= kmax) {  // uniform
+#pragma unroll
+          for (int r = 0; r < 4; r++) {
+            const int last = min(a.past + t0 + 4 * g + r, kmax);
+            const float x = fmaf(sc[4 * g + r][tile_at(p)], f16_lo(d), o[r]);
+            o[r] = p <= last ? x : o[r];
+            const float y = fmaf(sc[4 * g + r][tile_at(p + 1)], f16_hi(d), o[r]);
+            o[r] = p + 1 <= last ? y : o[r];
+          }
+        }
+      }
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < 4; r++)
+    if (t0 + 4 * g + r < seq) a.out[((size_t)(t0 + 4 * g + r) * a.heads + h) * kHeadDim + 16 * w + n] = o[r];
+}
+
+// Exact attention of `seq` queries over past + seq positions: query tiles for prompts that fit
+// and fill them (attn_tile_pays), else a (query, head) block up to kPLds positions -- of context for the operator, of
+// capacity for the model (`limit`), whose decode step picks by capacity -- else spans. All
+// evaluate a query alike.
+hipError_t launch_attn_exact(hipStream_t s, const ExactArgs& a, int seq, int limit, int spans) {
+  const int total = a.past + seq;
+  if (attn_tile_pays(seq, a.heads, total) && total <= kTileCtx && limit <= kPLds) {
+    const dim3 grid((seq + kTileQ - 1) / kTileQ * a.heads), block(kTileThreads);
+    if (total <= 512) hipLaunchKernelGGL(k_attn_tile<512>, grid, block, 0, s, a, seq);
+    else if (total <= 1024) hipLaunchKernelGGL(k_attn_tile<1024>, grid, block, 0, s, a, seq);
+    else hipLaunchKernelGGL(k_attn_tile<kTileCtx>, grid, block, 0, s, a, seq);
+  } else if (limit <= kPLds) {
+    hipLaunchKernelGGL(k_attn_block, dim3(a.heads, seq), dim3(kAttnThreads), 0, s, a);
+  } else {
+    hipLaunchKernelGGL(k_attn_exact, dim3(spans, a.heads, seq), dim3(kBlock), 0, s, a);
+  }
+  return hipGetLastError();
+}
+
 // --------------------------------------------------------------- attention --
 static int score_stride(int total) { return (total + 3) & ~3; }
 

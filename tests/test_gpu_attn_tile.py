@@ -1,4 +1,4 @@
-"""Exact attention of a prompt by tiles of 16 queries (csrc/attention.h k_attn_tile): every query
+"""Exact attention of a prompt by tiles of 16 queries (csrc/ops.hip k_attn_tile): every query
 equals its own one-query call bit for bit, at the edges of the tiles and of the score rows."""
 import numpy as np
 import pytest
