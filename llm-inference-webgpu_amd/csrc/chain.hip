@@ -555,7 +555,7 @@ __global__ __launch_bounds__(kBlock, 2) void k_chain_f64(ChainArgs a) {
 #pragma unroll
       for (int i = 0; i < S; i++) rc[i].set(wr[i], sr[i], zr[i]);
       if (more) load(cn);
-      __builtin_amdgcn_wave_barrier();  // the wave's own stores of this slab precede its reads
+      wave_lds_handoff();  // the wave's own stores of this slab precede its reads
       const float* xb = xs[wave];
 #pragma unroll
       for (int i = 0; i < S; i++) {
@@ -581,7 +581,7 @@ __global__ __launch_bounds__(kBlock, 2) void k_chain_f64(ChainArgs a) {
           chain64_steps<FMT, kSteps, T>(rc[i], xv, g4, two, acc[i]);
         }
       }
-      __builtin_amdgcn_wave_barrier();
+      wave_lds_handoff();
       if (more) store(xs[wave]);
     }
 #pragma unroll

@@ -802,6 +802,15 @@ __device__ __forceinline__ v4f chain_value4(const ChainOut& o, int t, int i4) {
   return v;
 }
 
+// Between a wave's LDS stores and other lanes' reads of them, and those reads and the next stores:
+// a wave's LDS operations run in order, so the hardware needs no wait, but the compiler has to be
+// told that another lane's data is read.
+__device__ __forceinline__ void wave_lds_handoff() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+}
+
 // Team width of a matrix: 32 lanes when a row has at most 32 chunks, else 64.
 // It fixes which chunks a lane sums and the butterfly, so it is a function of
 // the shape alone and every path over a given matrix sums in one order.

@@ -543,11 +543,11 @@ static __global__ __launch_bounds__(kTileThreads) void k_attn_tile(ExactArgs a, 
       v4u* dst = reinterpret_cast<v4u*>(&ks[w][n][16 * g]);
       dst[0] = d[0];
       dst[1] = d[1];
-      __builtin_amdgcn_wave_barrier();  // the wave's LDS operations run in order
+      wave_lds_handoff();
       _Float16 e[16];
 #pragma unroll
       for (int s = 0; s < 16; s++) e[s] = __builtin_bit_cast(_Float16, ks[w][n][4 * s + g]);
-      __builtin_amdgcn_wave_barrier();
+      wave_lds_handoff();
       f64x4 acc = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
       for (int s = 0; s < 16; s++)
