@@ -109,6 +109,19 @@ __global__ void k_rope_kv(const float* __restrict__ qkv, int splits, const float
   }
 }
 
+// The decode step's slot merge for every query: out [seq][heads*64]. grid (seq).
+__global__ __launch_bounds__(kBlock) void k_attn_merge_rows(const float* __restrict__ part, int heads,
+                                                            float* __restrict__ out) {
+  __shared__ float wl[kBlock];
+  const int t = blockIdx.x;
+  CombineIn in;
+  in.load(part + (size_t)t * heads * kDecodeSlots * kPartStride, heads);
+  const v4f acc = attn_combine_quad(in, wl);
+  const int i = threadIdx.x;
+  if (i < heads * kCombineLanes)
+    *reinterpret_cast<v4f*>(out + (size_t)t * heads * kHeadDim + 4 * i) = acc;
+}
+
 // h[t][j] = silu(g) * u over interleaved gate|up rows (g = gu[t][2j], u = gu[t][2j+1]), as
 // the decode step's SWIGLU epilogue evaluates it: in f64 (src/core/ops.js:81-91), or in
 // f32 for fast numerics (F32).
@@ -175,6 +188,21 @@ __global__ void k_embed_rows(const uint16_t* __restrict__ embed, const int* __re
     rows[(size_t)t * hidden + i] = __builtin_bit_cast(float, (uint32_t)src[i] << 16);
 }
 
+// Whether the attention of `seq` prompt queries, the last over `total` positions, runs as the decode
+// step's launch and a merge over its partials -- 16 blocks a query and kv head -- instead of in
+// launch_attn_prompt's one block, which goes through a long context in twice two slots a wave, a
+// round per 256 blocks, while few queries leave the chip to the 16. The difference, fitted to 2 to
+// 64 queries over 0 to 8000 positions of 1 to 16 kv heads; us a layer, one block | 16 and merge, of 2
+// kv heads: 2 queries after 8000 positions +50, after 2000 +11, after 200 -0.6; 32 after 8000 +39,
+// after 1000 +1.4, after 500 -3; 64 after 3000 +3.7, after 2000 -1.3.
+static bool attn_steps_pay(int seq, int kv_heads, int total) {
+  const int rows = seq * kv_heads;
+  const float k = 0.001f * total;
+  return 6.6f * k * ((rows + 255) / 256) > 1.5f + rows * (0.07f + 0.0165f * k);
+}
+// The most queries that do; their partials are in the workspace.
+static int step_queries(int kv_heads) { return std::max(64, 256 / kv_heads); }
+
 // Whether batched contractions of `seq` positions run on the f32 matrix cores (launch_chain_f32, the
 // same bits) or in launch_matvec_f32's tiles of 8 / 4 / 2 / 1 positions. A chain launch costs the
 // same up to 64 positions, the tiles by pass: about 4 units a tile of 8, 5 a smaller one; int4
@@ -228,7 +256,8 @@ PrefillBytes prefill_bytes(const ModelDev& m, const CacheDev& c, int matmul) {
   const size_t d = m.hidden, kv = (size_t)m.kv_heads * m.head_dim, f = m.intermediate;
   PrefillBytes b{};
   b.floats = P * (5 * d + (d + 2 * kv) + 3 * f);
-  if (m.numerics == QH_NUMERICS_FAST && decode_attn_long(c.capacity)) b.floats += P * m.heads * kDecodeSlots * kPartStride;
+  if (m.numerics == QH_NUMERICS_FAST)
+    b.floats += (decode_attn_long(c.capacity) ? P : std::min<size_t>(P, step_queries(m.kv_heads))) * m.heads * kDecodeSlots * kPartStride;
   else if (m.numerics == QH_NUMERICS_EXACT && c.capacity > kPLds) b.floats += P * m.heads * (c.score_stride + attn_spans(c.capacity));
   b.counters = m.numerics == QH_NUMERICS_EXACT ? P * m.heads : 0;
   const bool chain = m.numerics == QH_NUMERICS_FAST && !(matmul == QH_MATMUL_MFMA && all_mfma(m));
@@ -463,6 +492,12 @@ static hipError_t batched_attention(hipStream_t s, const ModelDev& m, const Cach
   a.heads = m.heads;
   a.kv_heads = m.kv_heads;
   if (!decode_attn_long(c.capacity)) {
+    if (seq <= step_queries(m.kv_heads) && attn_steps_pay(seq, m.kv_heads, past + seq)) {
+      const hipError_t e = launch_attn_decode(s, a, seq, 1);
+      if (e != hipSuccess) return e;
+      hipLaunchKernelGGL(k_attn_merge_rows, dim3(seq), dim3(kBlock), 0, s, a.part, m.heads, p.ATT);
+      return hipGetLastError();
+    }
     a.out = p.ATT;
     return launch_attn_prompt(s, a, seq);
   }

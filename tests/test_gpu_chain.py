@@ -156,6 +156,55 @@ def test_prompt_attention_past_1024_positions_equals_steps_bitwise(ctx, hip):
     model.destroy()
 
 
+def test_short_prompts_after_a_past_equal_steps_bitwise(ctx, hip):
+    """Few queries over a long context take the decode step's blocks and a merge, others a block per
+    query and kv head: the steps' logits and K/V rows in both, on both sides of the line."""
+    cfg = hip.ModelConfig(hidden=256, intermediate=256, layers=2, heads=4, kv_heads=2, vocab=1000)
+    model = hip.GpuModel.load(ctx, hip.device_tensors(hip.synthesize_checkpoint(cfg, seed=25), cfg, "int8", 128, "int8"),
+                              cfg, maxPositions=2300)
+    ids = hip.synth_tokens(25, "chain.after", cfg.vocab, 2300)
+    steps, cache = model.newCache(2300), model.newCache(2300)
+    done = 0
+    for n in (100, 2, 190, 2, 9, 800, 40, 64, 128, 700, 40, 64, 129, 2, 9):
+        model.set_matmul("matvec")
+        want = model.forward_tokens(ids[done:done + n], steps)["logits"]
+        model.set_matmul("batched")
+        got = model.forward_tokens(ids[done:done + n], cache)["logits"]
+        np.testing.assert_array_equal(got.view(np.uint32), want.view(np.uint32), err_msg=f"{n} after {done}")
+        done += n
+    for L in range(cfg.layers):
+        p, s = cache.present(L), steps.present(L)
+        np.testing.assert_array_equal(p["key"], s["key"])
+        np.testing.assert_array_equal(p["value"], s["value"])
+    cache.destroy()
+    steps.destroy()
+    model.destroy()
+
+
+def test_short_prompts_after_a_long_past_cost_what_they_cost_at_first(ctx, hip):
+    """Two queries over 8000 positions: 16 blocks each share the context, where one block each would
+    more than double the forward."""
+    cfg = hip.ModelConfig(hidden=256, intermediate=256, layers=8, heads=4, kv_heads=1, vocab=1000)
+    model = hip.GpuModel.load(ctx, hip.device_tensors(hip.synthesize_checkpoint(cfg, seed=26), cfg, "int8", 128, "int8"),
+                              cfg, maxPositions=8192)
+    ids = hip.synth_tokens(26, "chain.long.past", cfg.vocab, 8000)
+    cache = model.newCache(8192)
+    model.forward_tokens(ids, cache, wantLogits=False)
+
+    def best(past):
+        least = 1e9
+        for _ in range(30):
+            cache.length = past
+            start = time.perf_counter()
+            model.forward_tokens(ids[:2], cache)
+            least = min(least, time.perf_counter() - start)
+        return least
+    late = best(8000)
+    assert late < 1.6 * best(0)
+    cache.destroy()
+    model.destroy()
+
+
 @pytest.mark.parametrize("fmt", ["f16", "int8", "int4"])
 @pytest.mark.parametrize("cols", [896, 4864])     # positions in LDS; an f64 copy of all of them
 def test_matvec_of_unaligned_positions_equals_single_positions_bitwise(ctx, hip, fmt, cols):
