@@ -352,7 +352,7 @@ size_t chain_partials_bound(const DMat& m, int P) {
 }
 
 // A launch's latency and its blocks' slabs one after another, more of them where a CU holds
-// several blocks. Fitted with matvec_f32_us to prompts of 9 to 512 positions through models of 128
+// several blocks, slower ones where few share the loads. Fitted with matvec_f32_us to prompts of 9 to 512 positions through models of 128
 // to 1024 columns and 256 to 8192 ffn rows in every format, and to a head of 151936 rows.
 float chain_f32_us(const DMat& m, int seq) {
   const int kS = m.format == QH_FMT_INT4 ? 2 : 4, tl = team_width(m.nchunks), splits = chain_splits(m, seq);
@@ -360,7 +360,7 @@ float chain_f32_us(const DMat& m, int seq) {
   const int slabs = groups * ((m.nchunks + tl - 1) / tl);
   const long blocks = (long)((m.rows + kChainN - 1) / kChainN) * ((seq + kChainM - 1) / kChainM) * splits;
   const float slab = m.format == QH_FMT_F16 ? 0.5f : m.format == QH_FMT_INT8 ? 0.9f : 1.3f;
-  return 3.5f + slab * slabs * std::max(1.f, 1.2f * blocks / 256);
+  return 3.5f + slab * slabs * std::max(blocks < 16 ? 1.2f : 1.f, 1.2f * blocks / 256);
 }
 
 template <int FMT, int LV>
