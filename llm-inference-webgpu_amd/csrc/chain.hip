@@ -37,7 +37,11 @@ struct ChainFmt {
   static constexpr int kWRow = kWBytes + 16;               // staged, padded against bank conflicts
   static constexpr int kPieces = kChainN * kS;             // 16-byte pieces of a weight slab
   static constexpr int kPer = (kPieces + kBlock - 1) / kBlock;
-  static constexpr int kLevels = FMT == QH_FMT_INT4 ? 5 : 4;  // log2(64 / kS)
+  // log2 of the slot groups of one block: 16 at most (chain_splits cuts an int4 team of 64 lanes in
+  // two at least), and fewer where lanes sum several chunks: in int8 and int4 those are rows of more
+  // than 1024 or 2048 columns, a down projection's at most 1024 of them, cut in four at least.
+  static constexpr int kLevels = 4;
+  static constexpr int kMultiLevels = FMT == QH_FMT_F16 ? 4 : FMT == QH_FMT_INT8 ? 2 : 3;
 };
 
 struct ChainArgs {
@@ -329,7 +333,8 @@ __global__ __launch_bounds__(kBlock) void k_chain_finish(ChainOut o, float* __re
   if (i < (size_t)o.seq * o.rows) y[i] = chain_value(o, i, (int)(i % o.rows));
 }
 
-// Splits of the team's slots over blocks: enough that the chip holds about three blocks per CU.
+// Splits of the team's slots over blocks: until there are two blocks per CU, which is what the
+// registers of nearly every form allow.
 // A split is a whole subtree of the butterfly, so the splits' roots meet in the same tree.
 static int chain_splits(const DMat& m, int seq) {
   const int kS = m.format == QH_FMT_INT4 ? 2 : 4, tl = team_width(m.nchunks);
@@ -363,14 +368,22 @@ float chain_f32_us(const DMat& m, int seq) {
   return 3.5f + slab * slabs * std::max(blocks < 16 ? 1.2f : 1.f, 1.2f * blocks / 256);
 }
 
-template <int FMT, int LV>
-static void chain_lv(hipStream_t s, const ChainArgs& a, dim3 grid, int lv) {
-  if (lv == LV) {
-    if (a.m.nchunks > a.tl) hipLaunchKernelGGL((k_chain_f32<FMT, LV, true>), grid, dim3(kBlock), 0, s, a);
-    else hipLaunchKernelGGL((k_chain_f32<FMT, LV, false>), grid, dim3(kBlock), 0, s, a);
-  } else if constexpr (LV > 0) {
-    chain_lv<FMT, LV - 1>(s, a, grid, lv);
+// False where no form sums that many levels.
+template <int FMT, int LV = ChainFmt<FMT>::kLevels>
+static bool chain_lv(hipStream_t s, const ChainArgs& a, dim3 grid, int lv) {
+  if (lv < LV) {
+    if constexpr (LV > 0) return chain_lv<FMT, LV - 1>(s, a, grid, lv);
   }
+  if (lv > LV) return false;
+  if (a.m.nchunks <= a.tl) {
+    hipLaunchKernelGGL((k_chain_f32<FMT, LV, false>), grid, dim3(kBlock), 0, s, a);
+    return true;
+  }
+  if constexpr (LV <= ChainFmt<FMT>::kMultiLevels) {
+    hipLaunchKernelGGL((k_chain_f32<FMT, LV, true>), grid, dim3(kBlock), 0, s, a);
+    return true;
+  }
+  return false;
 }
 
 hipError_t launch_chain_roots(hipStream_t s, const DMat& m, const float* x, const float* bias, float* y, int seq,
@@ -387,11 +400,10 @@ hipError_t launch_chain_roots(hipStream_t s, const DMat& m, const float* x, cons
   const dim3 grid((m.rows + kChainN - 1) / kChainN, (seq + kChainM - 1) / kChainM, splits);
   int lv = 0;
   while (((m.format == QH_FMT_INT4 ? 2 : 4) << lv) < a.tl / splits) lv++;
-  switch (m.format) {
-    case QH_FMT_F16: chain_lv<QH_FMT_F16, ChainFmt<QH_FMT_F16>::kLevels>(s, a, grid, lv); break;
-    case QH_FMT_INT8: chain_lv<QH_FMT_INT8, ChainFmt<QH_FMT_INT8>::kLevels>(s, a, grid, lv); break;
-    default: chain_lv<QH_FMT_INT4, ChainFmt<QH_FMT_INT4>::kLevels>(s, a, grid, lv); break;
-  }
+  const bool ok = m.format == QH_FMT_F16    ? chain_lv<QH_FMT_F16>(s, a, grid, lv)
+                  : m.format == QH_FMT_INT8 ? chain_lv<QH_FMT_INT8>(s, a, grid, lv)
+                                            : chain_lv<QH_FMT_INT4>(s, a, grid, lv);
+  if (!ok) return hipErrorInvalidValue;
   *out = ChainOut{a.y, splits, m.rows, seq, splits > 1 && m.format == QH_FMT_INT8 ? m.scales : nullptr,
                   splits > 1 ? bias : nullptr};
   return hipGetLastError();

@@ -52,6 +52,33 @@ def test_batched_prefill_on_matrix_cores_equals_steps_bitwise(ctx, hip, scheme, 
     model.destroy()
 
 
+@pytest.mark.parametrize("scheme", ["f16", "int8", "int4"])
+@pytest.mark.parametrize("hidden,ffn,heads", [
+    (1024, 8192, 16),       # the widest fast model: the deepest tree with several chunks a lane
+    (512, 1536, 8),         # int4 down: a team of 64 lanes cut once; gate|up: one of 32, whole
+])
+def test_batched_prefill_deepest_trees_equal_steps_bitwise(ctx, hip, scheme, hidden, ffn, heads):
+    cfg = hip.ModelConfig(hidden=hidden, intermediate=ffn, layers=2, heads=heads, kv_heads=2, vocab=1000)
+    model = hip.GpuModel.load(ctx, hip.device_tensors(hip.synthesize_checkpoint(cfg, seed=27), cfg, scheme, 128, "int8"),
+                              cfg, maxPositions=512)
+    ids = hip.synth_tokens(27, "chain.deep", cfg.vocab, 512)
+    steps = model.newCache(512)
+    model.set_matmul("matvec")
+    want = {n: model.forward_tokens(ids[a:n], steps)["logits"] for a, n in ((0, 65), (65, 319), (319, 512))}
+    model.set_matmul("batched")
+    for n, logits in want.items():
+        cache = model.newCache(512)
+        got = model.forward_tokens(ids[:n], cache)["logits"]
+        np.testing.assert_array_equal(got.view(np.uint32), logits.view(np.uint32), err_msg=f"{n} positions")
+        for L in range(cfg.layers):
+            p, s = cache.present(L), steps.present(L)
+            for name in ("key", "value"):
+                np.testing.assert_array_equal(p[name], s[name][:, :n], err_msg=f"{n} positions, layer {L} {name}")
+        cache.destroy()
+    steps.destroy()
+    model.destroy()
+
+
 @pytest.mark.parametrize("fmt", ["f16", "int8", "int4"])
 @pytest.mark.parametrize("rows,cols,group", [
     (1, 128, 128),          # one row: a tile of clamped rows
