@@ -37,8 +37,8 @@ Also reported on the same JSON line:
                  paths checked to compute the same model, then prompt time-to-logits at 1 ..
                  512 tokens and single-token steps, median/min/max per path
   perplexity     the reference's perplexity protocol on a seeded 48-token passage (no tokenizer
-                 or checkpoint here): f16 / int8 / int4-g128 / int4-g32 scored one token at a time
-                 on the decode kernels, paired NLL change vs f16 +- SE, and |dNLL| vs the oracle
+                 or checkpoint here): f16 / int8 / int4-g128 / int4-g32 scored in one batched pass
+                 with the decode kernels' bits, paired NLL change vs f16 +- SE, and |dNLL| vs the oracle
   greedy_match   every timed token against the CPU oracle continuing from the GPU's cache
                  (teacher-forced), the smallest top-2 margin, and per layer the max-abs
                  relative error and cosine of the K/V rows the decoded positions stored
@@ -333,8 +333,8 @@ def prefill_bench(ctx, cfg, ckpt, seed, prompt_len=512, modes=("matvec", "batche
 def perplexity_bench(ctx, cfg, ckpt, seed, n=48, oracle_check=True):
     """The reference's perplexity protocol (web/perplexity.html:125-215, validate/perplexity.js)
     on a seeded n-token passage of this synthetic model -- no tokenizer or checkpoint is here:
-    every scheme scores the same n - 1 positions one token at a time through the cache
-    (qh_score: the decode kernels reading the int8/int4 codes), perplexity = exp(mean NLL), and
+    every scheme scores the same n - 1 positions in one batched pass through the cache
+    (qh_score: the int8/int4 codes, with the bits of one decode step after another), perplexity = exp(mean NLL), and
     the paired per-position NLL change against f16 with its standard error (the reference's
     "not distinguishable" test at 2 SE). Layers and head use the scheme, as the reference's
     round trip covers the tied embedding; input rows are the bf16 rows. With the oracle check,
@@ -375,7 +375,7 @@ def perplexity_bench(ctx, cfg, ckpt, seed, n=48, oracle_check=True):
         rows[label] = row
         log(f"perplexity {label}: {row['perplexity']} over {row['scored']} positions"
             + (f", |dNLL| vs oracle <= {row['max_abs_nll_vs_oracle']}" if oracle_check else ""))
-    return {"protocol": f"seeded {n}-token passage, full left context, one token at a time, nothing scored twice, "
+    return {"protocol": f"seeded {n}-token passage, full left context, one batched pass with the bits of single steps, nothing scored twice, "
                         f"{n - 1} positions", "schemes": rows}
 
 

@@ -516,8 +516,8 @@ static hipError_t batched_attention(hipStream_t s, const ModelDev& m, const Cach
 }
 
 // The batched fast-numerics layers with every contraction on the f32 matrix cores, its splits'
-// tree, scale, residual add, rmsnorm or swiglu in its consumer: eight launches a layer against
-// twelve (scoring 127 positions of int4 layers 4.1 -> 3.7 ms). The same operations in the same order, so the
+// tree, scale, residual add, rmsnorm or swiglu in its consumer: nine launches a layer against eleven
+// and a finish per split contraction (scoring 127 positions of int4 layers 4.1 -> 3.7 ms). The same operations in the same order, so the
 // same bits, as the launches of enqueue_prefill_layers.
 static hipError_t prefill_layers_chain(hipStream_t s, const ModelDev& m, const CacheDev& c, const PrefillDev& p,
                                        int past, int seq) {

@@ -83,10 +83,11 @@ struct PrefillDev {
   float* Y;            // [P][hidden] o / down outputs
   float* GU;           // [P][2*intermediate] interleaved gate|up
   float* H;            // [P][intermediate]
-  float* part;         // fast: [P][heads][kDecodeSlots][kPartStride] attention slot partials
+  float* part;         // fast: attention slot partials [heads][kDecodeSlots][kPartStride] of P queries (long caches)
+                       // or of those that take the decode step's launch
   float* scores;       // exact past kPLds: [P][heads][score_stride] + [P][heads][spans]
   int* counters;       // exact: [P][heads], zero between launches
-  void* scratch;       // matmul scratch (f64 activations, MFMA splits)
+  void* scratch;       // matmul scratch (split roots, f64 activations of a few positions, MFMA splits)
   size_t scratch_bytes;
 };
 struct PrefillBytes {

@@ -96,8 +96,8 @@ static hipError_t matvec_nb(hipStream_t s, const DMat& m, const float* x, const 
 template <int FMT>
 static hipError_t matvec_fmt(hipStream_t s, const DMat& m, const float* x, const double* x64,
                              const float* bias, float* y, int seq) {
-  // Tiles of 8 positions (src/gpu/model.js:133-138 batchTileFor), then 4, 2 and 1 for the
-  // remainder. The tile decides only how many positions share a weight read, never how an
+  // Tiles of 8 positions (src/gpu/model.js:133-138 batchTileFor; from 6 only where x is off its
+  // 16 bytes), then 4, 2 and 1 for the remainder. The tile decides only how many positions share a weight read, never how an
   // output is summed.
   hipError_t e = hipSuccess;
   int done = 0;

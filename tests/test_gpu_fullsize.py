@@ -83,7 +83,7 @@ def same_f16_layers(cfg, gpu_cache, pinned_cache, upto, label):
 @pytest.mark.timeout(600)
 def test_config4_1024_prompt_and_256_graph_replayed_greedy_tokens(ctx, hip, full_ckpt):
     """BASELINE config 4 as the bench runs it: int4-g128 layers, int8 head, f16 cache, a seeded
-    1024-token prompt prefilled (8-position batched tiles), then 256 greedy tokens by hipGraph
+    1024-token prompt prefilled (batched), then 256 greedy tokens by hipGraph
     replay (runs of 8 steps per graph launch). Checks:
       - prompt logits vs the oracle's own 1024-token prefill within 1e-4, same argmax; per-layer
         present K/V max-abs and cosine reported;
@@ -159,7 +159,7 @@ def test_config4_1024_prompt_and_256_graph_replayed_greedy_tokens(ctx, hip, full
 @pytest.mark.timeout(600)
 def test_config5_512_prefill_batched_and_mfma_match_oracle(ctx, hip, full_ckpt):
     """a seeded 512-token prompt, int8 layers and head, f16 cache, through
-    the 8-position batched tiles and through the MFMA contraction + flash attention.
+    the batched contractions and through the MFMA contraction + flash attention.
       - batched: logits within 1e-4 of the oracle's own prefill (bitwise equal to one decode
         step per position, tested elsewhere);
       - MFMA: within 1e-4 of the same-f16 oracle (the oracle attending to the MFMA run's own

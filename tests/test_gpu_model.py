@@ -310,7 +310,7 @@ def test_fast_numerics_long_context_matches_exact(ctx, hip, prompt_len):
 @pytest.mark.parametrize("numerics", ["fast", "exact"])
 @pytest.mark.parametrize("scheme", ["f16", "int8", "int4"])
 def test_batched_prefill_equals_one_position_steps_bitwise(ctx, hip, numerics, scheme):
-    """QH_MATMUL_BATCHED runs all positions per layer through 8-position weight tiles; every
+    """QH_MATMUL_BATCHED runs all positions per layer (tiles or matrix cores); every
     output is summed as the decode step sums it, so its logits and cache equal a prefill made
     of single decode steps (QH_MATMUL_MATVEC) bit for bit -- over two 512-position chunks."""
     cfg = tiny(hip)
@@ -364,7 +364,7 @@ def test_long_cache_batched_prefill_equals_one_position_steps_bitwise(ctx, hip):
 def test_config5_prefill_batched_and_mfma_match_oracle(ctx, hip, full_ckpt, numerics):
     """Config 5's model (int8 layers and head, f16 cache) prefilling a seeded 96-token prompt.
 
-    The batched tiles sum as the CPU does: logits within LOGIT_REL of the oracle's own prefill
+    The batched contractions sum as the CPU does: logits within LOGIT_REL of the oracle's own prefill
     (exact numerics: equal). The MFMA contraction agrees with the CPU's f64 sums to ~4e-7 per
     output but not to the bit, so an entry of its f16 cache can round to the neighbouring f16
     value where the CPU's does not; it is held to LOGIT_REL against the same-f16 oracle (the

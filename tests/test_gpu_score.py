@@ -1,7 +1,8 @@
 """Perplexity scoring on the device kernels (qh_score): the reference's perplexity page scores a
 passage one token at a time through the cache and takes -log softmax at the true next token
-(web/perplexity.html:146-170). Here every step is the decode step itself (int8/int4 codes read by
-the kernels, not an f16 round trip), and the log-softmax runs on the device in f64.
+(web/perplexity.html:146-170). Here the positions run in one batched pass with the bits of one
+decode step after another (int8/int4 codes read by the kernels, not an f16 round trip; up to three
+as steps), and the log-softmax runs on the device in f64.
 
 Checks, per weight format and numerics mode:
   - each NLL equals the oracle's expression (oracle/oracle.c `or_nll`) applied to the logits the
@@ -69,7 +70,7 @@ def test_score_continues_from_a_prompt(ctx, hip):
     a = model.newCache(64)
     whole = model.score(ids, a)
     b = model.newCache(64)
-    model.forward_tokens(ids[:15], b, wantLogits=False)   # positions 0..14 through the 8-position tiles
+    model.forward_tokens(ids[:15], b, wantLogits=False)   # positions 0..14 in one batched pass
     tail = model.score(ids[15:], b)                        # feeds ids[15..38], scores ids[16..39]
     assert tail.shape == (24,) and b.length == 15 + 24
     # the batched prefill equals one-position steps bit for bit, so the scores agree exactly
