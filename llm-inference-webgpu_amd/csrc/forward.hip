@@ -189,12 +189,12 @@ __global__ void k_embed_rows(const uint16_t* __restrict__ embed, const int* __re
 }
 
 // Whether the attention of `seq` prompt queries, the last over `total` positions, runs as the decode
-// step's launch and a merge over its partials -- 16 blocks a query and kv head -- instead of in
-// launch_attn_prompt's one block, which goes through a long context in twice two slots a wave, a
-// round per 256 blocks, while few queries leave the chip to the 16. The difference, fitted to 2 to
-// 64 queries over 0 to 8000 positions of 1 to 16 kv heads; us a layer, one block | 16 and merge, of 2
-// kv heads: 2 queries after 8000 positions +50, after 2000 +11, after 200 -0.6; 32 after 8000 +39,
-// after 1000 +1.4, after 500 -3; 64 after 3000 +3.7, after 2000 -1.3.
+// step's launch and a merge over its partials, 16 blocks a query and kv head, instead of in
+// launch_attn_prompt's one block: its eight waves take the context's 16 slots two each, for every 256
+// blocks once more, where the 16 blocks of few queries have the chip to themselves. What one block
+// costs more than 16 and the merge was fitted to 2 to 64 queries over 0 to 8000 positions of 1 to 16
+// kv heads; us a layer, 2 kv heads: 2 queries after 8000 positions +50, after 2000 +11, after 200
+// -0.6; 32 after 8000 +39, after 1000 +1.4, after 500 -3; 64 after 3000 +3.7, after 2000 -1.3.
 static bool attn_steps_pay(int seq, int kv_heads, int total) {
   const int rows = seq * kv_heads;
   const float k = 0.001f * total;
